@@ -32,25 +32,11 @@ sys.path.insert(0, HERE)
 
 PEAK_FP64_TFLOPS = 78.6     # MI355X dense FP64 (vector and matrix)
 PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense FP32 on the matrix cores
-FLOP_PER_NODE = {0: 292.0, 1: 376.0, 2: 498.0}   # the library's algorithmic model (hbem_profile_query)
 
-# HBM bytes per launch of the general-pair assembly kernel (rocprofv3
-# FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000, KiB per dispatch, scaled by the
-# counters' reading of a plain 1 GiB copy): profiles/k_assemble_x2_general_*.txt
-TRAFFIC_BYTES = {"star400": 1.7076e10, "polygon2000": 8.2862e10}
-# ... on a context with the lower-order rules on separated pairs: the
-# launches of a sweep (one per separation class and run of k blocks sharing an
-# order) averaged (profiles/k_cgemm32_sub_polygon2000_far_traffic.txt)
-TRAFFIC_BYTES_FAR = {"polygon2000": 1.2371e10}     # 7.423e10 B per sweep over 6 launches
 # HBM bytes per launch of the LU's matrix-core updates, averaged over the 217
 # launches of one polygon2000 sweep (the same counters and factors; 4.268e11 B
 # per sweep against 3.900e11 B of algorithmic C, A and B traffic)
 GEMM_TRAFFIC_BYTES = {("polygon2000", "f32"): 1.9666e9}
-# FP64 FLOP the general-pair kernel executes per quadrature node (rocprofv3
-# SQ_INSTS_VALU_{FMA,MUL,ADD,TRANS}_F64 x 64 lanes, FMA twice, over the nodes of
-# the launch), next to the 292 / 376 / 498 of the algorithmic model at d = 0/1/2:
-# profiles/k_assemble_x2_general_polygon2000_counters.txt, k_assemble_x2_star400_executed_flops.txt
-EXECUTED_FLOP_PER_NODE = {"polygon2000": 243.3, "star400": 337.6}
 
 WORKLOADS = {
     "polygon2000": dict(panels=2000, order=11, c_i=20.0, c_o=1.0, nk=128, k_min=5.0, k_max=40.0, der=0, seed=3,
@@ -111,7 +97,7 @@ def cpu_baseline(name, w, mesh, R, threads):
 
 def run_workload(H, name, steps, warmup, mixed=False, bd=None, ref_sigma=None, far=False):
     """Times `steps` sweeps of the workload (FP64, or with the mixed-precision
-    dense stage; far: on a context with the lower-order rules on separated
+    dense stage; far: on a context with the 5e-14 tolerance on separated
     pairs); with ref_sigma, also the largest relative sigma difference."""
     w = WORKLOADS[name]
     mesh = make_mesh(H, w)
@@ -154,8 +140,6 @@ def run_workload(H, name, steps, warmup, mixed=False, bd=None, ref_sigma=None, f
     ms_gen, n_gen, fl_gen = prof[0]
     avg_launch_s = ms_gen * 1e-3 / max(n_gen, 1)
     achieved = (fl_gen / max(n_gen, 1)) / avg_launch_s / 1e12 if n_gen else 0.0
-    ex_node = EXECUTED_FLOP_PER_NODE[name]
-    executed = achieved * ex_node / FLOP_PER_NODE[der] if ex_node else None
     ms_lu, n_lu, fl_lu = prof[3]
     lu_tflops = fl_lu / (ms_lu * 1e-3) / 1e12 if ms_lu > 0 else None
     out = {
@@ -168,15 +152,13 @@ def run_workload(H, name, steps, warmup, mixed=False, bd=None, ref_sigma=None, f
         "panel_pair_evals_per_s": pairs_per_k * evals / asm_s if asm_s > 0 else None,
         "phase_seconds_per_step": {ph: p[0] * 1e-3 / steps for ph, p in zip(PHASES, prof)},
         "lu_model_tflops": lu_tflops,
-        "roofline_assembly": {"kernel": "k_assemble_x2<general, d=%d> (general panel pairs, %d k x 2 c per launch%s)"
-                               % (der, w["nk"], "; one launch per separation class and run of k blocks of one order, Gauss orders 11 to 5" if far else ""),
-                     "bound": "fp64_valu", "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / PEAK_FP64_TFLOPS,
-                     "traffic": (TRAFFIC_BYTES_FAR if far else TRAFFIC_BYTES).get(name),
-                     "avg_launch_ms": avg_launch_s * 1e3, "launches": n_gen,
-                     "flops_per_launch": fl_gen / max(n_gen, 1),
-                     "executed_tflops": executed, "executed_frac": executed / PEAK_FP64_TFLOPS if executed else None,
-                     "seconds_per_step": ms_gen * 1e-3 / steps},
+        "roofline_assembly": {"kernel": "k_band_eval<d=%d> (band functionals x Hankel basis, all pairs of hat functions, "
+                                        "%d k)" % (der, w["nk"]),
+                              "bound": "fp64_mfma", "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
+                              "frac": achieved / PEAK_FP64_TFLOPS, "traffic": None,
+                              "avg_launch_ms": avg_launch_s * 1e3, "launches": n_gen,
+                              "flops_per_launch": fl_gen / max(n_gen, 1),
+                              "seconds_per_step": ms_gen * 1e-3 / steps},
     }
     if n_mm:
         f32 = mixed
@@ -193,9 +175,8 @@ def run_workload(H, name, steps, warmup, mixed=False, bd=None, ref_sigma=None, f
     cands = [v for v in (out["roofline_assembly"], out.get("roofline_lu_gemm")) if v]
     out["roofline"] = max(cands, key=lambda v: v["seconds_per_step"])
     if far:
-        out["far_field"] = "general pairs closer than one panel diameter at Gauss order 11, one to two diameters " \
-                           "apart at 9, two to eight at 8, eight to sixteen at 6, farther at 5 for the k blocks " \
-                           "with kappa d <= 0.4 and 6 for the others"
+        out["far_field"] = "separated pairs interpolated to 5e-14 of the largest kernel value on their distance band " \
+                           "instead of 1e-16 (kappa d <= 5)"
     if mixed:
         out["refine_steps"] = {"last_solve": MIXED_REFINE, "other_solves": MIXED_REFINE_INNER}
         out["fp64_fallbacks"] = fallback[0]
@@ -248,7 +229,7 @@ def run_resonance(H, steps, warmup):
     """The batched resonance search: the unit square in 1000 line panels and a
     random 10-vertex polygon (seed 4) in 1000 panels, order 11, c_i = 20, c_o =
     1.  Per instance: a 4096-point grid on [5, 50] swept in mixed precision on a
-    context with the lower-order rules on separated pairs and in FP64 on the
+    context with the 5e-14 tolerance on separated pairs and in FP64 on the
     plain one (sigma within 1e-8, same brackets), then Newton on every bracket
     with the batched sigma'' (FP64, plain context, q_refine = 20), so the roots
     are the plain path's.  One step = both instances' grids."""
@@ -292,7 +273,7 @@ def run_resonance(H, steps, warmup):
     evals = 2 * ks.size
     return {"metric": "sigma_min(k) evals/s", "value": evals / t_grid, "unit": "evals/s", "n_gpus": 1,
             "steps": steps, "warmup": warmup, "ms_per_step": (t_grid + t_newton) * 1e3, "higher_is_better": True,
-            "scaling": "weak", "vs_baseline": None, "dtype": "f32 LU + f64 refinement, lower-order rules on separated pairs (grid), f64 (Newton)",
+            "scaling": "weak", "vs_baseline": None, "dtype": "f32 LU + f64 refinement, 5e-14 tolerance on separated pairs (grid), f64 (Newton)",
             "data": "synthetic",
             "config": {"workload": "unit square and random 10-vertex polygon (seed 4), 1000 line panels each, order "
                                    "11, c_i=20, c_o=1, 4096 k in linspace(5,50) per instance, then Newton with "
@@ -312,7 +293,7 @@ def main():
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--legs", default="fp64,mixed,mixed_far",
                     help="sweeps to time: fp64 (the plain path), mixed (FP32 LU + FP64 refinement), mixed_far "
-                         "(the same on a context with the lower-order rules on separated pairs); the headline is "
+                         "(the same on a context with the 5e-14 tolerance on separated pairs); the headline is "
                          "the fastest within the 1e-8 bar of the fp64 leg")
     ap.add_argument("--cpu-threads", type=int, default=16)
     ap.add_argument("--copy-calibration", type=int, default=0, metavar="MIB",
@@ -379,7 +360,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f64" if head is fp64 else ("f32 LU + f64 refinement (assembly f64%s)"
-                                              % (", lower-order rules on separated pairs" if head is mixed_far else "")),
+                                              % (", 5e-14 tolerance on separated pairs" if head is mixed_far else "")),
         "data": "synthetic",
         "config": dict(head["config"], name=args.workload),
         "panel_pair_evals_per_s": head["panel_pair_evals_per_s"],

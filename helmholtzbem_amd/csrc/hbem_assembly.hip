@@ -1,4 +1,7 @@
-// hbem_assembly.hip -- Galerkin assembly of V, K, W (and d/dk, d2/dk2) on gfx950.
+// hbem_assembly.hip -- node-loop assembly of V, K, W (and d/dk, d2/dk2) on gfx950,
+// for the wavenumbers the distance bands of hbem_radial.hip do not serve (kappa
+// times the largest panel diameter above 20, strongly complex kappa, kappa = 0,
+// fewer than eight panels, and the coinciding single layer's k-derivative quirk).
 //
 // Restates GalerkinBuilder (galerkin_builder.cpp:17-1018) for continuous P1
 // test = trial spaces:
@@ -8,12 +11,10 @@
 //   * per pair and wavenumber the kernel produces the reference's local
 //     interaction matrices (double layer direct + transposed block,
 //     hypersingular, single layer; derivative orders 0..D) into a pair-indexed
-//     buffer;
-//   * a gather kernel sums, for each global entry, the (at most four) pair
-//     blocks that touch it, in a fixed order -- deterministic, no atomics --
-//     and applies the factor i/4 (galerkin_builder.cpp:1014-1017).
+//     buffer, from which k_records_from_locals sums the records of the pairs of
+//     hats in a fixed order -- deterministic, no atomics.
 //
-// Geometry is precomputed once per mesh into per-pair node tables
+// Geometry is precomputed once per mesh, on first use, into per-pair node tables
 // {r, r^2, v.N_j |tau_i|, -v.N_i |tau_j|, tau_i.tau_j, |tau_i||tau_j|, 1/r,
 // (2/pi) ln r, 1/sqrt(r)}, so the per-wavenumber kernels only evaluate the
 // Hankel functions and accumulate.
@@ -611,56 +612,6 @@ struct AccX {
     cdbl kd[D + 1][2], kt[D + 1][2], wb[D + 1][2], v[D + 1][2], wa[D + 1];
 };
 
-// J0, Y0, J1, Y1 of x = kappa r from the node's kappa-free factors.
-//   y = x^2 / 64, L2 = (2/pi) ln(x/2) = lk + lr, 1/x = kinv / r,
-//   1/sqrt(pi x) = ksq / sqrt(r)
-// TINY >= 1 (touching panel pairs, whose arguments are small): x < HBEM_TINY_X
-// takes the entire parts from the degree-HBEM_TINY_DEG table fitted on that
-// range instead of the degree-HBEM_SMALL_DEG table of (0, 8); TINY = 2 takes
-// x < HBEM_TINY1_X from the degree-HBEM_TINY1_DEG table of that range first.
-// sin / cos beyond x = 1e6 (never reached by the benchmark's arguments): kept
-// out of line so the library routine's constants do not occupy registers of
-// the callers' loops
-__device__ __noinline__ void sincos_far(double x, double& s, double& c) { sincos(x, &s, &c); }
-
-template <int TINY>
-__device__ __forceinline__ void bessel_jy01_f(double x, double y, double L2, double xinv, double b, double& j0,
-                                              double& y0, double& j1, double& y1) {
-    if (x < 8.0) {
-        double A, B, C, Dd;
-        if (TINY >= 2 && x < (double)HBEM_TINY1_X)
-            horner4<HBEM_TINY1_DEG>(bessel_table() + HBEM_TAB_TINY1, y, A, B, C, Dd);
-        else if (TINY >= 1 && x < (double)HBEM_TINY_X)
-            horner4<HBEM_TINY_DEG>(bessel_table() + HBEM_TAB_TINY, y, A, B, C, Dd);
-        else
-            horner4<HBEM_SMALL_DEG>(bessel_table() + HBEM_TAB_SMALL, y, A, B, C, Dd);
-        const bool pos = x > 0.0;
-        const double J1 = x * B;
-        j0 = pos ? A : 1.0;
-        j1 = pos ? J1 : 0.0;
-        y0 = pos ? fma(L2, A, C) : 0.0;
-        y1 = pos ? fma(L2, J1, fma(x, Dd, -kTwoOverPi * xinv)) : 0.0;
-    } else if (x <= 1e6) {
-        double s, c;
-        sincos_med(x, s, c);
-        const double cs = c + s, sc = s - c;
-        const double z = 64.0 * xinv * xinv;
-        double P0, Q0, P1, Q1;
-        horner4<HBEM_PQ_DEG>(bessel_table() + HBEM_TAB_PQ, z, P0, Q0, P1, Q1);
-        Q0 *= xinv;
-        Q1 *= xinv;
-        j0 = b * fma(P0, cs, -Q0 * sc);
-        y0 = b * fma(P0, sc, Q0 * cs);
-        j1 = b * fma(P1, sc, Q1 * cs);
-        y1 = b * fma(Q1, sc, -P1 * cs);
-    } else {
-        double s, c;
-        sincos_far(x, s, c);
-        const double cs = c + s, sc = s - c;
-        j0 = b * cs; y0 = b * sc; j1 = b * sc; y1 = -b * cs;
-    }
-}
-
 // one node's contribution to this lane's sums (entries q = m + 2h).  General
 // and adjacent pairs: K direct, W and V go to the running row-free sums U in
 // slot m = 1 (see row_fold); K transposed to both entries as for coinciding
@@ -783,8 +734,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     int q = qb * 32 + j;
     const bool active = qb < nqb && q < P.nk;
     if (q >= P.nk) q = P.nk - 1;
-    const int qi = (P.einst ? P.einst[e] * P.nk : 0) + q;   // the slot's entry in the kappa tables
-    const double kap = P.kap[qi];
+    const double kap = P.kap[q];
     const double lk = kTwoOverPi * log(0.5 * kap);
     const double kinv = 1.0 / kap;
     const double ksq = 1.0 / sqrt(kPi * kap);
@@ -800,8 +750,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         lo = hn * nh + (chunk - hn * cph) * P.chunk;
         hi = min(hn * nh + nh, lo + P.chunk);
     }
-    const double* __restrict__ geo =
-        P.einst ? P.igeo[P.einst[e]] + (size_t)(e - P.ibase[P.einst[e]]) * nn * kNodeStride : P.ngeo + (size_t)e * nn * kNodeStride;
+    const double* __restrict__ geo = P.ngeo + (size_t)e * nn * kNodeStride;
 
     AccX<D> A;
 #pragma unroll
@@ -891,7 +840,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 
     // Sums -> this lane's entries q = m + 2h of the reference's local matrices
     // (same scalings as acc_store)
-    const double kr = P.kr[qi], c = P.cv[qi];
+    const double kr = P.kr[q], c = P.cv[q];
     const double sqc = sqrt(c), k2h = 0.5 * kap * kap;
     cdbl Ko[D + 1][2], Kto[D + 1][2], Wo[D + 1][2], Vo[D + 1][2];
 #pragma unroll
@@ -947,7 +896,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         // it in scratch memory).  Every thread reaches the barriers.
         static_assert((STG + 1) * REC >= 256 * 4 * 2, "exchange needs 16 KB of staging LDS");
         const int mine = wv & 1;
-        const int kt = P.kt0 + ((qb >> 1) << 5) + j;
+        const int kt = ((qb >> 1) << 5) + j;
         const bool kact = qb < nqb && kt < P.nkt;
         const size_t nkt = (size_t)P.nkt;
         cdbl* out = P.out + rec * (16 * (D + 1)) * nkt + kt;
@@ -1008,167 +957,6 @@ __global__ void k_chunk_sum(const cdbl* __restrict__ part, int nent, int nchunk,
     cdbl acc = mk(0, 0);
     for (int c = 0; c < nchunk; ++c) acc = acc + p[(size_t)c * nslot * nk];
     L[((size_t)pidx[e] * nslot + s) * nk + q] = acc;
-}
-
-// ---------------------------------------------------------------------------
-// Gather: global entry (m, n) of an operator = sum of the local blocks of the
-// panel pairs (P, Q), P in {m-1, m}, Q in {n-1, n} (P1 dofs: dof(0,P) = P+1,
-// dof(1,P) = P; continuous_space.hpp:36-45), scatter rule of
-// galerkin_builder.cpp:992-1009.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ long long tri(int i, int j) { return (long long)i * (i + 1) / 2 + j; }
-
-// layer: 0 K, 1 W, 2 V
-__device__ __forceinline__ cdbl op_entry(const cdbl* __restrict__ L, int nk, int nslot, int q, int layer, int t,
-                                         int m, int n, int N) {
-    cdbl e[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-        const int P = a == 0 ? (m == 0 ? N - 1 : m - 1) : m;
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int Q = b == 0 ? (n == 0 ? N - 1 : n - 1) : n;
-            long long p;
-            int slot;
-            if (P >= Q) {
-                p = tri(P, Q);
-                slot = (layer == 0 ? 0 : layer == 1 ? 8 : 12) + a + 2 * b;
-            } else {
-                p = tri(Q, P);
-                slot = layer == 0 ? 4 + a + 2 * b : (layer == 1 ? 8 : 12) + b + 2 * a;
-            }
-            e[a][b] = L[((size_t)p * nslot + 16 * t + slot) * nk + q];
-        }
-    }
-    // (e00 + e11) + (e01 + e10): under (m, n) -> (n, m) the symmetric layers
-    // exchange e01 and e10 only, so V and W come out exactly symmetric
-    const cdbl acc = (e[0][0] + e[1][1]) + (e[0][1] + e[1][0]);
-    return mk(-0.25 * acc.y, 0.25 * acc.x);   // * i/4
-}
-
-// Builder matrices for wavenumber slot q: out[layer][t] (N x N column-major)
-__global__ void k_gather_layers(const cdbl* __restrict__ L, int nk, int nslot, int q, int N, int D, int layers,
-                                cdbl* __restrict__ Kout, cdbl* __restrict__ Wout, cdbl* __restrict__ Vout) {
-    const long long NN = (long long)N * N;
-    long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= NN * (D + 1)) return;
-    const int t = (int)(id / NN);
-    const long long e = id - t * NN;
-    const int m = (int)(e % N), n = (int)(e / N);
-    if ((layers & 1) && Kout) Kout[id] = op_entry(L, nk, nslot, q, 0, t, m, n, N);
-    if ((layers & 4) && Wout) Wout[id] = op_entry(L, nk, nslot, q, 1, t, m, n, N);
-    if ((layers & 2) && Vout) Vout[id] = op_entry(L, nk, nslot, q, 2, t, m, n, N);
-}
-
-// Transmission matrix (assemble_operator, gen_sol_op.cpp:59-74, unprojected):
-// T = [[K_i - K_o + M, V_o - V_i], [W_o - W_i, K_o - K_i + M^T]], M only for t = 0.
-// Output b uses wavenumber slots qi[b] (inner c_i), qo[b] (outer c_o); with qo
-// null, L holds the differences per wavenumber (K_i - K_o, W_o - W_i, V_o - V_i
-// at slot qi[b]; the paired-lane kernel's tdiff layout).  T_t of output b is
-// written at Tt + b ld^2.
-// Workgroup = one pair of 8 x 8 tiles (I, J), I >= J, of the N x N blocks for
-// 32 outputs b; thread (i, jb) = (threadIdx & 7, threadIdx >> 3) forms the
-// four block entries (m, n), (m + N, n + N), (m, n + N), (m + N, n) of row
-// m = 8 I + i over the 8 columns of tile (I, J), then (for I > J) of row
-// 8 J + i over the columns of tile (J, I).  op_entry sums the symmetric layers
-// W and V bitwise symmetric, so tile (J, I) takes them from tile (I, J)
-// through LDS: every local-matrix record is read once.  Reads run over 32
-// wavenumbers per record slot, writes over 8 rows per column; the output
-// chunks of one tile pair are neighbouring workgroups, so the chunks of a
-// record slot are read at about the same time (long runs in each DRAM page).
-__global__ __launch_bounds__(256) void k_form_T(const cdbl* __restrict__ L, int nk, int nslot,
-                                                const int* __restrict__ qi, const int* __restrict__ qo, int nb, int N,
-                                                int D, const double* __restrict__ M, cdbl* __restrict__ T0,
-                                                cdbl* __restrict__ T1, cdbl* __restrict__ T2, int ld,
-                                                cflt* __restrict__ T32) {
-    __shared__ cdbl sW[8][8][32];   // [column in tile (I, J)][row in tile (I, J)][output]
-    __shared__ cdbl sV[8][8][32];
-    const int mt = (N + 7) >> 3, nbc = (nb + 31) >> 5;
-    const int bc = blockIdx.x % nbc, tile = blockIdx.x / nbc;
-    const int I = tile % mt, J = tile / mt;
-    if (J > I) return;                       // whole workgroup: no barrier is skipped
-    const int i = threadIdx.x & 7, jb = threadIdx.x >> 3;
-    const int b = bc * 32 + jb;
-    const bool act = b < nb;                 // idle threads still reach every barrier
-    const int n2 = ld;                       // leading dimension (2N, or more for a zero-padded T)
-    const size_t NN = (size_t)n2 * n2;
-    const bool diff = qo == nullptr;
-    const int a = act ? qi[b] : 0, o = act && !diff ? qo[b] : 0;
-    const bool mirror = I != J;
-    for (int t = 0; t <= D; ++t) {
-        cdbl* Tt = (t == 0 ? T0 : (t == 1 ? T1 : T2)) + (size_t)(act ? b : 0) * NN;
-        // T and, when asked, its FP32 copy for the mixed-precision LU (each
-        // entry rounded to nearest) in the same pass
-        cflt* Ts = t == 0 && T32 ? T32 + (size_t)(act ? b : 0) * NN : nullptr;
-        auto put = [&](size_t idx, cdbl v) {
-            Tt[idx] = v;
-            if (Ts) Ts[idx] = cflt{(float)v.x, (float)v.y};
-        };
-        const int m = 8 * I + i;
-        for (int c = 0; c < 8; ++c) {
-            const int n = 8 * J + c;
-            if (!act || m >= N || n >= N) continue;
-            cdbl k00, k11, w, v;
-            if (diff) {
-                k00 = op_entry(L, nk, nslot, a, 0, t, m, n, N);
-                k11 = mk(-k00.x, -k00.y);
-                w = op_entry(L, nk, nslot, a, 1, t, m, n, N);
-                v = op_entry(L, nk, nslot, a, 2, t, m, n, N);
-            } else {
-                const cdbl Ki = op_entry(L, nk, nslot, a, 0, t, m, n, N), Ko = op_entry(L, nk, nslot, o, 0, t, m, n, N);
-                const cdbl Wi = op_entry(L, nk, nslot, a, 1, t, m, n, N), Wo = op_entry(L, nk, nslot, o, 1, t, m, n, N);
-                const cdbl Vi = op_entry(L, nk, nslot, a, 2, t, m, n, N), Vo = op_entry(L, nk, nslot, o, 2, t, m, n, N);
-                k00 = Ki - Ko; k11 = Ko - Ki;
-                w = Wo - Wi; v = Vo - Vi;
-            }
-            if (t == 0) { k00.x += M[m + (size_t)n * N]; k11.x += M[n + (size_t)m * N]; }
-            put(m + (size_t)n * n2, k00);
-            put((m + N) + (size_t)(n + N) * n2, k11);
-            put(m + (size_t)(n + N) * n2, v);
-            put((m + N) + (size_t)n * n2, w);
-            if (mirror) { sW[c][i][jb] = w; sV[c][i][jb] = v; }
-        }
-        if (!mirror) continue;
-        __syncthreads();
-        const int r = 8 * J + i;
-        for (int c = 0; c < 8; ++c) {
-            const int col = 8 * I + c;
-            if (!act || r >= N || col >= N) continue;
-            cdbl k00, k11;
-            if (diff) {
-                k00 = op_entry(L, nk, nslot, a, 0, t, r, col, N);
-                k11 = mk(-k00.x, -k00.y);
-            } else {
-                const cdbl Ki = op_entry(L, nk, nslot, a, 0, t, r, col, N), Ko = op_entry(L, nk, nslot, o, 0, t, r, col, N);
-                k00 = Ki - Ko; k11 = Ko - Ki;
-            }
-            if (t == 0) { k00.x += M[r + (size_t)col * N]; k11.x += M[col + (size_t)r * N]; }
-            put(r + (size_t)col * n2, k00);
-            put((r + N) + (size_t)(col + N) * n2, k11);
-            put(r + (size_t)(col + N) * n2, sV[i][c][jb]);   // V(r, col) = V(col, r)
-            put((r + N) + (size_t)col * n2, sW[i][c][jb]);
-        }
-        __syncthreads();                     // the next order overwrites sW / sV
-    }
-}
-
-// Right-hand-side operator of the transmission solve (tp::direct_second_kind::
-// A_rhs, solvers.cpp:116-122) from the outer operators of wavenumber slot o:
-// A_o = [[-K_o + M/2, V_o], [W_o, K_o^T + M/2]] (2N x 2N, column-major).
-// One thread per (m, n) writes the four block entries; K_o^T(m, n) = K_o(n, m)
-// is gathered from the local matrices directly.
-__global__ __launch_bounds__(256) void k_form_Ao(const cdbl* __restrict__ L, int nk, int nslot, int o, int N,
-                                                 const double* __restrict__ M, cdbl* __restrict__ A) {
-    const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= (long long)N * N) return;
-    const int m = (int)(id % N), n = (int)(id / N);
-    const size_t n2 = 2 * (size_t)N;
-    const double hm = 0.5 * M[m + (size_t)n * N];
-    const cdbl Ko = op_entry(L, nk, nslot, o, 0, 0, m, n, N), KoT = op_entry(L, nk, nslot, o, 0, 0, n, m, N);
-    A[m + (size_t)n * n2] = mk(-Ko.x + hm, -Ko.y);
-    A[m + (size_t)(n + N) * n2] = op_entry(L, nk, nslot, o, 2, 0, m, n, N);
-    A[(m + N) + (size_t)n * n2] = op_entry(L, nk, nslot, o, 1, 0, m, n, N);
-    A[(m + N) + (size_t)(n + N) * n2] = mk(KoT.x + hm, KoT.y);
 }
 
 // ---------------------------------------------------------------------------
@@ -1240,20 +1028,6 @@ void launch_chunk_sum(const cdbl* part, int nent, int nchunk, int nk, int nslot,
                        nslot, pidx, npairs, L);
 }
 
-void launch_gather_layers(const cdbl* L, int nk, int nslot, int q, int N, int D, int layers, cdbl* K, cdbl* W,
-                          cdbl* V, hipStream_t st) {
-    long long n = (long long)N * N * (D + 1);
-    hipLaunchKernelGGL(k_gather_layers, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, L, nk, nslot, q, N, D,
-                       layers, K, W, V);
-}
-
-void launch_form_T(const cdbl* L, int nk, int nslot, const int* qi, const int* qo, int nb, int N, int D,
-                   const double* M, cdbl* T0, cdbl* T1, cdbl* T2, hipStream_t st, int ld, cflt* T32) {
-    const unsigned mt = (unsigned)((N + 7) / 8);
-    hipLaunchKernelGGL(k_form_T, dim3(mt * mt * (unsigned)((nb + 31) / 32)), dim3(256), 0, st, L, nk, nslot, qi, qo,
-                       nb, N, D, M, T0, T1, T2, ld > 0 ? ld : 2 * N, T32);
-}
-
 // The rows and columns n..ld-1 of nb matrices of order ld (stride ld^2): the
 // identity there, so that a matrix of order n padded to ld has the same LU
 // factors on its leading n x n block and the identity below.
@@ -1274,12 +1048,6 @@ void launch_pad_identity(cdbl* T, int n, int ld, int nb, hipStream_t st) {
     const long long total = (long long)(ld - n) * ld + (long long)(ld - n) * n;
     if (total <= 0 || nb <= 0) return;
     hipLaunchKernelGGL(k_pad_identity, dim3((unsigned)((total + 255) / 256), nb), dim3(256), 0, st, T, n, ld);
-}
-
-void launch_form_Ao(const cdbl* L, int nk, int nslot, int o, int N, const double* M, cdbl* A, hipStream_t st) {
-    const long long n = (long long)N * N;
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_form_Ao, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, L, nk, nslot, o, N, M, A);
 }
 
 }  // namespace hbem

@@ -59,6 +59,19 @@ T* upload(DBuf& b, const std::vector<T>& v, hipStream_t st) {
     return d;
 }
 
+constexpr size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Several host arrays laid out for one upload, each 256-byte aligned.
+struct Packed {
+    std::vector<char> bytes;
+    template <class T> size_t add(const std::vector<T>& v) {
+        const size_t at = al256(bytes.size());
+        bytes.resize(at + v.size() * sizeof(T) + 8);
+        if (!v.empty()) std::memcpy(bytes.data() + at, v.data(), v.size() * sizeof(T));
+        return at;
+    }
+};
+
 // Real sparse n x n matrix in compressed-row form on the device.
 struct DCsr {
     DBuf rp, ci, v;
@@ -155,17 +168,19 @@ constexpr int kChunkNodes = 2048;
 long long adj_chunks(int nc) { return 2 * (((long long)nc * nc + kChunkNodes - 1) / kChunkNodes); }
 long long coi_chunks(int nc) { return ((long long)nc * nc + kChunkNodes - 1) / kChunkNodes; }
 
-// Device bytes a sigma sweep needs per wavenumber of a batch: local matrices
-// and chunk partials (lcols columns per k: 1 in the T-difference layout, 2
-// for the two refraction indices otherwise), T (factorised in place), T',
-// T'', pivots and the thin blocks of the randomized SVD.
-size_t sweep_bytes_per_k(long long npairs, long long nadj, long long ncoi, int nc_rule, int n, int D, int ncols,
-                         int lcols) {
+// Device bytes a sigma sweep needs per wavenumber of a batch: on the node loops
+// the local matrices and chunk partials (lcols columns per k: 1 in the
+// T-difference layout, 2 for the two refraction indices otherwise); T
+// (factorised in place), T', T'', pivots and the thin blocks of the randomized SVD.
+size_t locals_bytes_per_k(long long npairs, long long nadj, long long ncoi, int nc_rule, int D, int lcols) {
     const size_t nslot = 16 * (size_t)(D + 1);
     const size_t part = (size_t)std::max(nadj * adj_chunks(nc_rule), ncoi * coi_chunks(nc_rule));
+    return (size_t)lcols * ((size_t)npairs + part) * nslot * sizeof(cdbl);
+}
+size_t dense_bytes_per_k(int n, int D, int ncols) {
     const size_t nn = (size_t)n * n;
-    return (size_t)lcols * ((size_t)npairs + part) * nslot * sizeof(cdbl) + (size_t)(D + 1) * nn * sizeof(cdbl) +
-           2 * (size_t)n * sizeof(int) + (4 * (size_t)ncols + 4) * n * sizeof(cdbl) + 64;
+    return (size_t)(D + 1) * nn * sizeof(cdbl) + 2 * (size_t)n * sizeof(int) + (4 * (size_t)ncols + 4) * n * sizeof(cdbl) +
+           64;
 }
 
 // Sweeps of >= 32 real positive wavenumbers run every batch on the paired-lane
@@ -219,7 +234,6 @@ int sweep_batch(size_t per_k, size_t avail, int nk) {
 // thin-solve work (2 n nc complex).
 constexpr int kNaMaxN = 2048;
 constexpr int kNaMaxCols = 8;
-constexpr size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 constexpr size_t kNaBytes = al256(sizeof(cdbl) * (size_t)kNaMaxN * kNaMaxN) + 2 * al256(sizeof(int) * (size_t)kNaMaxN) +
                             4 * al256(sizeof(cdbl) * (size_t)kNaMaxN * kNaMaxCols);
 static __device__ __align__(256) unsigned char scratch[kNaBytes];
@@ -254,6 +268,16 @@ size_t usable_device_bytes(size_t held) {
 
 }  // namespace
 
+// Work space of an assembly call: the slots' tables and column lists ...
+struct RecBufs {
+    DBuf tab;                                    // slots and columns, one upload
+    std::vector<std::unique_ptr<DBuf>> lslots;   // slot tables of the groups on the node loops
+};
+// ... and what the groups use in turn
+struct RecScratch {
+    DBuf E, L, part;                             // E: the records, then a group's basis
+};
+
 struct hbem_geometry {
     int dev = 0;
     hipStream_t st = nullptr;
@@ -265,39 +289,57 @@ struct hbem_geometry {
     std::vector<int> tr;
     // device geometry
     DBuf d_panels, d_coefs, d_xg, d_wg, d_xc, d_wc, d_gtab;
-    DBuf d_gent, d_gpidx, d_gflags, d_gngeo;
-    DBuf d_aent, d_apidx, d_aflags, d_angeo;
-    DBuf d_cent, d_cpidx, d_cflags, d_cngeo;
-    int ngen = 0, nadj = 0, ncoi = 0;
-    // General pairs in order of separation (the distance of the panels'
-    // bounding discs in panel diameters): sep[0] pairs closer than one
-    // diameter (or on a trigonometric or spline panel), sep[1] at one to two, sep[2] at two to
-    // eight, sep[3] at eight to sixteen, sep[4] farther apart (see far_order);
-    // dmax is the largest panel diameter.
-    static constexpr int kSep = 5;
-    int sep[kSep] = {0, 0, 0, 0, 0};
-    double dmax = 0.0;
-    // node tables of the separated classes at lower Gauss orders, built on
-    // first use: key 64 cls + order
-    struct FarSet {
-        DBuf xg, wg, gtab, flags, ngeo;
+    std::vector<int> aent;                 // adjacent panel pairs (i, j, swap), i > j
+    std::vector<double> disc;              // bounding disc of every panel: centre, radius
+    double dmax = 0.0;                     // largest disc diameter
+    // Panel pairs by class (coinciding, adjacent, general) with their node tables,
+    // for the node-loop kernels; built on first use.
+    struct Loops {
+        bool built = false;
+        int cnt[3] = {0, 0, 0};
+        DBuf ent[3], pidx[3], flags[3], ngeo[3];
+    } loops;
+    // Radial functionals (hbem_radial.hip): the pairs of hats by distance band,
+    // and per tier of kappa dmax the bands' points and coefficient tables.
+    struct Tier {
+        bool built = false;
+        int pmax = 0, pnear = 0, basis = 0;   // most points of a band; the near band's; basis records per slot
+        double points = 0.0;               // points summed over the far pairs
+        DBuf mem;                          // bands, tiles, transforms; coefficients; extra sums
+        const hbem::Band* bands = nullptr;
+        const hbem::BandTile* tiles = nullptr;
+        const double *costab = nullptr, *tab = nullptr, *ext = nullptr;
     };
-    std::map<int, std::unique_ptr<FarSet>> far;
+    static constexpr int kTiers = 6;
+    struct Radial {
+        bool built = false, usable = false;
+        int nbands = 0, ntile = 0, ntile_near = 0;
+        long long nfar = 0;
+        double R = 0.0, first = 0.0, step = 0.0, width = 0.0;
+        std::vector<hbem::RadialNear> near;
+        std::vector<int> tile_band;
+        DBuf plan, flagmem;                // near pairs, tiles' pairs; bands, skip flags
+        const unsigned char* flags = nullptr;
+        const hbem::RadialNear* d_near = nullptr;
+        const int* recs = nullptr;
+        Tier tier[kTiers];
+    } rad;
     DBuf d_M, d_Finvc;
     DCsr s_F, s_FT, s_FinvT, s_Finv;   // F, F^T, Finv^T and Finv of the projection
     // work space
     DBuf w_Ao, w_U, w_rhs, w_flag;
     DBuf w_Tp, w_B, w_mv, w_bpiv, w_bperm, w_bvec, w_d2;   // bordered system of sv_der2 (sweeps)
     DBuf w_T32, w_rb, w_rr, w_rpart, w_flag2, w_rprev;       // mixed-precision dense stage
-    DBuf w_kapi, w_kri, w_L, w_T0, w_T1, w_T2, w_piv, w_perm, w_X, w_Y, w_work, w_R, w_u, w_v, w_a, w_b, w_sig, w_dsig, w_kap,
-        w_kr, w_cv, w_qi, w_qo, w_tmp, w_out, w_part;
+    DBuf w_T0, w_T1, w_T2, w_piv, w_perm, w_X, w_Y, w_work, w_R, w_u, w_v, w_a, w_b, w_sig, w_dsig, w_tmp, w_out;
+    RecBufs w_rec;
+    RecScratch w_scr;
     // profiling (hbem_profile_enable / query)
     bool prof = false;
     EventLog plog;
     std::mutex mu;
     // bytes held by the per-batch work buffers of the sweep
     size_t work_held() const {
-        const DBuf* bs[] = {&w_L, &w_part, &w_T0, &w_T1, &w_T2, &w_piv, &w_perm, &w_X, &w_Y, &w_work, &w_u, &w_v, &w_a, &w_b,
+        const DBuf* bs[] = {&w_scr.E, &w_scr.L, &w_scr.part, &w_T0, &w_T1, &w_T2, &w_piv, &w_perm, &w_X, &w_Y, &w_work, &w_u, &w_v, &w_a, &w_b,
                             &w_Tp, &w_B, &w_bpiv, &w_bperm, &w_bvec, &w_T32, &w_rb, &w_rr, &w_rpart, &w_rprev};
         size_t s = 0;
         for (auto* b : bs) s += b->n;
@@ -333,220 +375,540 @@ void check_k(double k_re, double k_im, double c) {
 // k_rp of initialize_constants: the real Hankel path
 bool real_positive(double k_re, double k_im) { return k_im == 0.0 && k_re > 0.0; }
 
-// Slot tables of the tdiff layout (AsmParams::tdiff) for nb wavenumbers ks
-// with refraction indices c_i (inner) and c_o: blocks of 32 slots, block 2w
-// inner and block 2w + 1 outer for wavenumbers 32w .. 32w + 31; slots past
-// the last wavenumber repeat it (computed, never written).
-void tdiff_slots(const double* ks, int nb, double c_i, double c_o, std::vector<double>& kap, std::vector<double>& kr,
-                 std::vector<double>& cv) {
-    const int nblk = (nb + 31) / 32;
-    kap.resize(64 * (size_t)nblk);
-    kr.resize(kap.size());
-    cv.resize(kap.size());
-    for (size_t q = 0; q < kap.size(); ++q) {
-        const int blk = (int)(q >> 5), kt = std::min(nb - 1, (blk >> 1) * 32 + (int)(q & 31));
-        const double c = (blk & 1) ? c_o : c_i;
-        kap[q] = ks[kt] * std::sqrt(c);
-        kr[q] = ks[kt];
-        cv[q] = c;
+// ---------------------------------------------------------------------------
+// Pairs of hats by distance band, and the bands' tables per tier of kappa dmax
+// ---------------------------------------------------------------------------
+// Upper edges of kappa dmax.  A tier serves every kappa up to its edge, so each
+// doubling of the mesh width in wavelengths adds points to the bands (0.625, ten
+// panels a wavelength: 20 points, 2.5: 32, 20: 108); beyond the last edge, where
+// no rule resolves the panels, the node loops take over.
+constexpr double kTierEdge[hbem_geometry::kTiers] = {0.625, 1.25, 2.5, 5.0, 10.0, 20.0};
+// Interpolation error of the far bands relative to the radial function, and of
+// separated line and arc panels on contexts with HBEM_FLAG_FAR_FIELD (up to
+// kappa dmax = 5: half of the flag's 1e-13).
+constexpr double kBandTol = 1e-16, kBandTolFar = 5e-14, kNearTol = 1e-17;
+// Near radius, band step and largest interval width in units of dmax.  A hat's
+// support is at most 2 dmax wide, so a pair's distances spread over 4 dmax at
+// most; R = 10 puts the first far band at c / a = 3 (24 points at the first
+// tier, 20 from c / a = 5 on), and step 2 makes the bands half as wide again as
+// the widest interval.
+constexpr double kNearRadius = 10.0, kBandStep = 2.0, kBandWidth = 4.0;
+
+int tier_of(double kd) {
+    if (!(kd > 0.0)) return -1;
+    for (int t = 0; t < hbem_geometry::kTiers; ++t)
+        if (kd <= kTierEdge[t]) return t;
+    return -1;
+}
+
+int class_nodes(const hbem_geometry* g, int cls) {
+    return cls == 2 ? g->ns * g->ns : (cls == 1 ? 2 * g->nc * g->nc : g->nc * g->nc);
+}
+
+long long tri_index(int i, int j) { return i >= j ? (long long)i * (i + 1) / 2 + j : (long long)j * (j + 1) / 2 + i; }
+
+// Bands and tiles of the geometry (independent of kappa), built on first use.
+hbem_geometry::Radial& radial_base(hbem_geometry* g) {
+    auto& r = g->rad;
+    if (r.built) return r;
+    const int N = g->N;
+    if (N < 8 || g->npairs > 0x7fffffffLL || !(g->dmax > 0.0)) {
+        r.built = true;                       // too few panels for disjoint supports: the node loops
+        return r;
     }
-}
-
-// Gauss order of the tensor rule for the separated general pairs of class cls
-// (1: one to two panel diameters apart, 2: two to eight, 3: eight to sixteen,
-// 4: farther) when kappa times the largest panel diameter is at most kd: the
-// lowest order whose single- and double-layer local matrices stay within 1e-13
-// of their largest entry of the 11-point rule's -- with a margin of two, 5e-14
-// -- for straight panels at the class's least separation, end-on, side by side
-// and at 42 random angles, at both ends of the kd interval (the rule's error
-// falls as (separation)^(-2m) and with the oscillation kappa d as
-// (kappa d)^(2m) / (2m)!); ns when no lower order qualifies.
-int far_order(double kd, int cls, int ns) {
-    static const double edge[5] = {0.4, 0.65, 1.25, 2.5, 5.0};
-    static const int order[5][4] = {{9, 8, 6, 5}, {9, 8, 6, 6}, {9, 8, 7, 7}, {9, 8, 8, 8}, {10, 10, 10, 10}};
-    for (int t = 0; t < 5; ++t)
-        if (kd <= edge[t]) return std::min(order[t][cls - 1], ns);
-    return ns;
-}
-
-// The node tables of separation class cls (1 to 4) at Gauss order m < ns,
-// built on first use (one setup launch per table).
-hbem_geometry::FarSet& far_set(hbem_geometry* g, int cls, int m) {
-    auto& slot = g->far[64 * cls + m];
-    if (slot) return *slot;
-    auto f = std::make_unique<hbem_geometry::FarSet>();
-    std::vector<double> xg(m), wg(m);
-    hbem::gauss_rule(0.0, 1.0, m, xg.data(), wg.data());
-    const double* dxg = upload(f->xg, xg, g->st);
-    upload(f->wg, wg, g->st);
-    double* gtab = f->gtab.as<double>((size_t)g->N * m * 5);
-    hbem::launch_setup_gauss_table((const double*)g->d_panels.p, (const double*)g->d_coefs.p, g->N, dxg, m, gtab, g->st);
-    int off = 0;
-    for (int s = 0; s < cls; ++s) off += g->sep[s];
-    const int cnt = g->sep[cls];
-    f->flags.get(std::max(1, cnt));
-    double* ngeo = f->ngeo.as<double>(std::max<size_t>(1, (size_t)cnt * m * m * hbem::kNodeStride));
-    if (cnt > 0)
-        hbem::launch_setup_general((const int*)g->d_gent.p + 3 * (size_t)off, cnt, gtab, m, ngeo,
-                                   (unsigned char*)f->flags.p, g->st);
+    r.R = kNearRadius * g->dmax;
+    r.width = kBandWidth * g->dmax * (1.0 + 1e-12);
+    r.step = kBandStep * g->dmax;
+    r.first = r.R - r.width;
+    // pairs of hats over a coinciding or adjacent panel pair
+    std::vector<unsigned short> band((size_t)g->npairs, 0);
+    std::vector<std::vector<std::pair<int, int>>> adj(N);      // adjacent lower-numbered panels, their entries
+    auto touch = [&](int P, int Q) {
+        for (int a = 0; a < 2; ++a)
+            for (int b = 0; b < 2; ++b) band[tri_index((P + a) % N, (Q + b) % N)] = 1;
+    };
+    for (int P = 0; P < N; ++P) touch(P, P);
+    for (size_t e = 0; e < g->aent.size(); e += 3) {
+        touch(g->aent[e], g->aent[e + 1]);
+        adj[std::max(g->aent[e], g->aent[e + 1])].emplace_back(std::min(g->aent[e], g->aent[e + 1]), (int)(e / 3));
+    }
+    // bands and skip flags in one buffer
+    const size_t obf = al256(band.size() * sizeof(band[0]));
+    unsigned short* db = (unsigned short*)r.flagmem.get(obf + g->npairs);
+    HIPC(hipMemcpyAsync(db, band.data(), band.size() * sizeof(band[0]), hipMemcpyHostToDevice, g->st));
+    hbem::launch_radial_band((const double*)g->d_gtab.p, N, g->ns, (int)g->npairs, r.R, r.first, r.step, db, g->st);
+    unsigned char* fl = (unsigned char*)db + obf;
+    r.flags = fl;
+    HIPC(hipMemcpyAsync(band.data(), db, band.size() * sizeof(band[0]), hipMemcpyDeviceToHost, g->st));
+    HIPC(hipStreamSynchronize(g->st));
+    hbem::launch_radial_flags((const double*)g->d_gtab.p, g->ns, (int)g->npairs, fl, g->st);
     HIPC(hipGetLastError());
-    slot = std::move(f);
-    return *slot;
-}
-
-// Contexts with HBEM_FLAG_FAR_FIELD: the node tables every order far_order
-// gives for these kappa builds now (a batch's order is the order of one of its
-// kappa), so that batch sizing sees the memory they take.
-void prepare_far(hbem_geometry* g, const std::vector<double>& kap) {
-    if (!(g->flags & HBEM_FLAG_FAR_FIELD)) return;
-    for (int s = 1; s < hbem_geometry::kSep; ++s) {
-        if (g->sep[s] == 0) continue;
-        for (double v : kap) {
-            const int m = far_order(std::fabs(v) * g->dmax, s, g->ns);
-            if (m < g->ns) far_set(g, s, m);
-        }
+    int top = 0;
+    for (unsigned short b : band) top = std::max<int>(top, b);
+    r.nbands = top + 1;
+    // tiles of 16 pairs, band by band (the last of a band padded with -1)
+    std::vector<long long> count(r.nbands, 0), pos(r.nbands, 0);
+    for (unsigned short b : band) ++count[b];
+    long long slots = 0;
+    for (int b = 0; b < r.nbands; ++b) {
+        pos[b] = slots;
+        const long long nt = (count[b] + 15) / 16;
+        slots += nt * 16;
+        for (long long t = 0; t < nt; ++t) r.tile_band.push_back(b);
     }
+    r.ntile = (int)r.tile_band.size();
+    r.ntile_near = (int)((count[0] + 15) / 16);
+    r.nfar = g->npairs - count[0];
+    std::vector<int> recs((size_t)slots, -1);
+    long long rec = 0;
+    for (int m = 0; m < N; ++m)
+        for (int n = 0; n <= m; ++n, ++rec) {
+            const int b = band[rec];
+            recs[pos[b]++] = (int)rec;
+            if (b) continue;
+            hbem::RadialNear e = {m, n, {0, 0, 0, 0}};
+            for (int q = 0; q < 4; ++q) {
+                const int P = (m + N - 1 + (q & 1)) % N, Q = (n + N - 1 + (q >> 1)) % N;
+                e.type[q] = P == Q ? 4 * P : 3;
+                for (const auto& a : adj[std::max(P, Q)])
+                    if (a.first == std::min(P, Q)) e.type[q] = 1 + 4 * a.second;
+            }
+            r.near.push_back(e);
+        }
+    Packed pk;
+    const size_t on = pk.add(r.near), orec = pk.add(recs);
+    const char* plan = (const char*)r.plan.get(pk.bytes.size());
+    HIPC(hipMemcpyAsync(r.plan.p, pk.bytes.data(), pk.bytes.size(), hipMemcpyHostToDevice, g->st));
+    r.d_near = (const hbem::RadialNear*)(plan + on);
+    r.recs = (const int*)(plan + orec);
+    HIPC(hipStreamSynchronize(g->st));        // the upload reads a host vector
+    r.usable = true;
+    r.built = true;
+    return r;
 }
 
-// Assemble the local matrices of all pairs for wavenumber slots (kap, kr, cv)
-// with imaginary parts (kapi, kri) when any slot is not real positive; returns
-// the local buffer.  Wide real batches run on the paired-lane kernel, the rest
-// on node-parallel groups of lanes per item.  nkt > 0: the slots are in the
-// tdiff layout (tdiff_slots) for nkt wavenumbers, the paired-lane kernel runs
-// whatever the width, and the buffer holds the differences T is formed from,
-// nkt columns wide.  Contexts with HBEM_FLAG_FAR_FIELD and real slots: the
-// separated general pairs take the lower Gauss orders of far_order, chosen for
-// the largest kappa of each block of 32 wavenumbers in the tdiff layout (of
-// the batch otherwise); a launch per separation class and run of consecutive
-// blocks with the same order.
-cdbl* assemble_locals(hbem_geometry* g, const std::vector<double>& kap, const std::vector<double>& kr,
-                      const std::vector<double>& cv, int D, const std::vector<double>& kapi = {},
-                      const std::vector<double>& kri = {}, int nkt = 0) {
-    const int nk = (int)kap.size();
-    const int nslot = 16 * (D + 1);
-    const bool tdiff = nkt > 0;
-    if (tdiff && (!kapi.empty() || nk % 64 != 0 || 2 * nkt > nk || 2 * nkt <= nk - 64))
-        throw Error(HBEM_EINVAL, "tdiff layout needs real slots in blocks of 64 for its wavenumbers");
-    const int nko = tdiff ? nkt : nk;   // columns of the output layouts
-    cdbl* L = g->w_L.as<cdbl>((size_t)nko * g->npairs * nslot);
+// Points and coefficient tables of tier t, built on first use (null: a band
+// would need more than kBandMaxP points).
+hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
+    auto& r = radial_base(g);
+    if (!r.usable || t < 0) return nullptr;
+    auto& T = r.tier[t];
+    if (T.built) return T.pmax > 0 ? &T : nullptr;
+    bool straight = true;                     // line and arc panels only
+    for (int i = 0; i < g->N; ++i) straight = straight && g->panels[8 * (size_t)i] < 2.0;
+    const double tol = (g->flags & HBEM_FLAG_FAR_FIELD) && straight && kTierEdge[t] <= 5.0 ? kBandTolFar : kBandTol;
+    const double kmax = kTierEdge[t] / g->dmax;
+    std::vector<hbem::Band> bands(r.nbands);
+    std::vector<double> cosv;
+    std::map<int, int> cosoff;
+    std::map<int, std::vector<long double>> points;
+    int pmax = 0, basis = 0;
+    for (int b = 0; b < r.nbands; ++b) {
+        hbem::Band& B = bands[b];
+        if (b == 0) {
+            B.c = 0.0;
+            B.a = r.R;
+        } else {
+            const double lo = r.first + (b - 1) * r.step;
+            B.c = lo + 0.5 * (r.step + r.width);
+            B.a = 0.5 * (r.step + r.width);
+        }
+        B.p = hbem::band_order(B.c, B.a, kmax, b == 0 ? kNearTol : tol, b == 0);
+        if (B.p == 0) {
+            T.built = true;
+            return nullptr;
+        }
+        const int p = B.p;
+        auto it = cosoff.find(p);
+        if (it == cosoff.end()) {
+            it = cosoff.emplace(p, (int)cosv.size()).first;
+            for (int j = 0; j < p; ++j) points[p].push_back(cosl(acosl(-1.0L) * (2 * j + 1) / (2.0L * p)));
+            for (int j = 0; j < p; ++j)
+                for (int q = 0; q < p; ++q)
+                    cosv.push_back((q == 0 ? 1.0 : 2.0) / p * std::cos(M_PI * (double)((long long)q * (2 * j + 1) % (4 * p)) / (2.0 * p)));
+        }
+        B.cos = it->second;
+        B.rad = (int)cosv.size();
+        std::vector<double> res;              // the points' radii, then what rounding took from them
+        for (int j = 0; j < p; ++j) {
+            const long double s = points[p][j];
+            const long double x = b == 0 ? B.a * sqrtl(0.5L * (s + 1.0L)) : B.c + B.a * s;
+            cosv.push_back((double)x);
+            res.push_back((double)(x - (double)x));
+        }
+        cosv.insert(cosv.end(), res.begin(), res.end());
+        B.basis = basis;
+        basis += 2 * p;
+        pmax = std::max(pmax, p);
+    }
+    std::vector<hbem::BandTile> tiles(r.ntile);
+    long long off = 0;
+    for (int i = 0; i < r.ntile; ++i) {
+        const int b = r.tile_band[i];
+        tiles[i] = {off, b, 0};
+        off += (long long)bands[b].p * (b == 0 ? 10 : 5) * 16;
+        if (b) T.points += 16.0 * bands[b].p;
+    }
+    std::vector<int> cent;
+    for (int i = 0; i < g->N; ++i) cent.insert(cent.end(), {i, i, 0});
+    const std::vector<int>* ents[2] = {&cent, &g->aent};
+    // one upload: bands, tiles, transforms, and the singular pairs' lists
+    Packed pk;
+    const size_t ob = pk.add(bands), ot = pk.add(tiles), oc = pk.add(cosv), oe[2] = {pk.add(*ents[0]), pk.add(*ents[1])};
+    // ... and one buffer for these, the coefficients, the extra sums and the
+    // singular pairs' moments (which the tier does not need later)
+    const int pn = bands[0].p;
+    size_t need = al256(pk.bytes.size());
+    auto place = [&](size_t bytes) {
+        const size_t at = need;
+        need += al256(bytes);
+        return at;
+    };
+    size_t omom[2], oext[2];
+    const size_t otab = place((size_t)off * sizeof(double));
+    const size_t osum = place(std::max<size_t>(1, (size_t)r.ntile_near * 7 * 16) * sizeof(double));
+    for (int cls = 0; cls < 2; ++cls) {
+        const size_t cnt = ents[cls]->size() / 3 * (1 + cls);
+        omom[cls] = place(cnt * pn * hbem::kRadialMoments * sizeof(double));
+        oext[cls] = place(cnt * 8 * sizeof(double));
+    }
+    char* plan = (char*)T.mem.get(need);
+    HIPC(hipMemcpyAsync(plan, pk.bytes.data(), pk.bytes.size(), hipMemcpyHostToDevice, g->st));
+    const hbem::Band* db = T.bands = (const hbem::Band*)(plan + ob);
+    const hbem::BandTile* dt = T.tiles = (const hbem::BandTile*)(plan + ot);
+    const double* dc = T.costab = (const double*)(plan + oc);
+    double *tab = (double*)(plan + otab), *ext = (double*)(plan + osum);
+    T.tab = tab;
+    T.ext = ext;
+    const double* gtab = (const double*)g->d_gtab.p;
+    const double *xg = (const double*)g->d_xg.p, *wg = (const double*)g->d_wg.p;
+    for (int cls = 0; cls < 2; ++cls)
+        hbem::launch_radial_moments(cls, (const int*)(plan + oe[cls]), (int)ents[cls]->size() / 3,
+                                    (const double*)g->d_panels.p, (const double*)g->d_coefs.p, (const double*)g->d_xc.p,
+                                    (const double*)g->d_wc.p, g->nc, r.R, pn, (double*)(plan + omom[cls]),
+                                    (double*)(plan + oext[cls]), g->st);
+    hbem::launch_radial_near(r.d_near, (int)r.near.size(), dt, db, pn, gtab, xg, wg, g->N, g->ns,
+                             r.flags, (const double*)(plan + omom[0]), (const double*)(plan + oext[0]),
+                             (const double*)(plan + omom[1]), (const double*)(plan + oext[1]), dc, tab, ext, g->st);
+    hbem::launch_radial_far(r.recs, dt, r.ntile_near, r.ntile - r.ntile_near, db, pmax, gtab, xg, wg, g->N,
+                            g->ns, r.flags, dc, tab, g->st);
+    HIPC(hipGetLastError());
+    HIPC(hipStreamSynchronize(g->st));        // the uploads above read host vectors; other streams may use the tables
+    T.pmax = pmax;
+    T.pnear = pn;
+    T.basis = basis;
+    T.built = true;
+    return &T;
+}
+
+// Classes and node tables of all panel pairs.
+hbem_geometry::Loops& node_loops(hbem_geometry* g) {
+    auto& s = g->loops;
+    if (s.built) return s;
+    const int N = g->N;
+    std::vector<int> ent[3];
+    std::vector<long long> pidx[3];
+    auto add = [&](int cls, int i, int j, int swap) {
+        ent[cls].insert(ent[cls].end(), {i, j, swap});
+        pidx[cls].push_back(tri_index(i, j));
+    };
+    std::vector<std::vector<int>> nb(N);      // adjacent lower-numbered panels
+    for (int i = 0; i < N; ++i) add(0, i, i, 0);
+    for (size_t e = 0; e < g->aent.size(); e += 3) {
+        add(1, g->aent[e], g->aent[e + 1], g->aent[e + 2]);
+        nb[g->aent[e]].push_back(g->aent[e + 1]);
+    }
+    for (int i = 0; i < N; ++i)
+        for (int j = 0; j < i; ++j)
+            if (std::find(nb[i].begin(), nb[i].end(), j) == nb[i].end()) add(2, i, j, 0);
+    for (int c = 0; c < 3; ++c) {
+        s.cnt[c] = (int)pidx[c].size();
+        const int* de = upload(s.ent[c], ent[c], g->st);
+        upload(s.pidx[c], pidx[c], g->st);
+        unsigned char* fl = (unsigned char*)s.flags[c].get(std::max(1, s.cnt[c]));
+        double* ng = s.ngeo[c].as<double>(std::max<size_t>(1, (size_t)s.cnt[c] * class_nodes(g, c) * hbem::kNodeStride));
+        if (c == 2)
+            hbem::launch_setup_general(de, s.cnt[c], (const double*)g->d_gtab.p, g->ns, ng, fl, g->st);
+        else
+            hbem::launch_setup_singular(c, de, s.cnt[c], (const double*)g->d_panels.p, (const double*)g->d_coefs.p,
+                                        (const double*)g->d_xc.p, g->nc, ng, fl, g->st);
+    }
+    HIPC(hipGetLastError());
+    HIPC(hipStreamSynchronize(g->st));
+    s.built = true;
+    return s;
+}
+
+// The tier of a column with |kappa| between lo and hi and Im kappa at most im, or -1
+// for the node loops: kappa = 0, beyond the last tier, or so far from the real
+// axis that J and iY of the near band, each of size e^{Im kappa r}, would leave
+// H with fewer digits (kNearImag: e^{2 Im kappa R} below 3).
+constexpr double kNearImag = 0.5;
+int record_tier(hbem_geometry* g, double lo, double hi, double im) {
+    const int t = lo > 0.0 ? tier_of(hi * g->dmax) : -1;
+    if (t < 0 || !radial_tier(g, t)) return -1;
+    if (im > 0.0 && (im * g->rad.R > kNearImag || hi * g->rad.R > hbem::kEntireMax)) return -1;
+    return t;
+}
+
+// ---------------------------------------------------------------------------
+// Assembly of the records of a call's columns.  prepare_records does what needs
+// the host (tables, uploads, buffers), launch_records only launches, so that it
+// can stand in a captured graph.
+// ---------------------------------------------------------------------------
+// A group of columns that take the same way: tier >= 0: the bands' tables of that
+// tier; tier < 0: the node loops.
+struct RecGroup {
+    int tier, start, count;
+    double *kap = nullptr, *kr = nullptr, *cv = nullptr, *kapi = nullptr, *kri = nullptr;   // node loops: the group's slots
+    int nslots = 0;
+};
+// Values per order of the records of a call (see hbem_radial.hip).
+int record_values(const hbem_geometry* g, int D) { return (g->flags & HBEM_FLAG_QUIRK_SLP_COINC_DER) && D >= 1 ? hbem::kRecValues + 1 : hbem::kRecValues; }
+
+struct RecJob {
+    hbem_geometry* g = nullptr;
+    RecScratch* w = nullptr;
+    int D = 0, ncol = 0, nslot2 = 0, nv = 4;
+    bool diff = false, cplx = false, tdiff = false, prof = false;   // prof: time into the context's log
+    hipStream_t st = nullptr;
+    const double *kap = nullptr, *kapi = nullptr, *kr = nullptr, *kri = nullptr, *cv = nullptr;
+    const int* cols = nullptr;
+    size_t obasis = 0;                           // the basis' place behind the records
+    std::vector<RecGroup> groups;
+};
+
+// lanes per item of the node loops for ns slots: 0 = the paired-lane kernel
+// (32 wavenumbers x 2 nodes per wavefront), else groups of lanes per item
+void loop_lanes(int ns, bool cplx, bool tdiff, int& general, int& singular) {
+    general = cplx ? 16 : (ns >= 64 || tdiff ? 0 : (ns >= 16 ? 4 : 16));
+    singular = (ns >= 64 || tdiff) && !cplx ? 0 : 64;
+}
+
+// chunks of a class's nodes: singular pairs chunks of 2048 nodes (paired-lane
+// kernel, 16 staging rounds; for adjacent pairs each of the two node halves is
+// chunked on its own) or 64 x 48 nodes (one wavefront per item)
+void loop_chunks(int cls, int G, int nodes, int& chunk, int& nchunk) {
+    chunk = cls == 2 ? nodes : (G == 0 ? kChunkNodes : 64 * 48);
+    nchunk = (nodes + chunk - 1) / chunk;
+    if (cls == 1 && G == 0) nchunk = 2 * ((nodes / 2 + chunk - 1) / chunk);
+}
+
+// Node loops of one group: local matrices of all panel pairs, then the records.
+void launch_loops(const RecJob& J, const RecGroup& r) {
+    hbem_geometry* g = J.g;
+    const auto& set = g->loops;
+    const int nslot = 16 * (J.D + 1), nko = J.tdiff ? r.count : r.nslots;
+    cdbl* L = (cdbl*)J.w->L.p;
     hbem::AsmParams P;
     std::memset(&P, 0, sizeof(P));
     P.xg = (const double*)g->d_xg.p;
     P.wg = (const double*)g->d_wg.p;
     P.xc = (const double*)g->d_xc.p;
     P.wc = (const double*)g->d_wc.p;
-    const double* dkap = upload(g->w_kap, kap, g->st);
-    const double* dkr = upload(g->w_kr, kr, g->st);
-    const double* dcv = upload(g->w_cv, cv, g->st);
-    const bool cplx = !kapi.empty();
-    const double* dkapi = cplx ? upload(g->w_kapi, kapi, g->st) : nullptr;
-    const double* dkri = cplx ? upload(g->w_kri, kri, g->st) : nullptr;
     P.npairs_total = g->npairs;
     P.ns = g->ns;
     P.nc = g->nc;
     P.qflags = g->flags;
-    P.tdiff = tdiff ? 1 : 0;
-    P.nkt = nkt;
-    // lanes per item: G = 0 selects the paired-lane kernel for wide batches
-    // (32 wavenumbers x 2 nodes per wavefront); node groups of G lanes otherwise
-    const int Gg = cplx ? 16 : (nk >= 64 || tdiff ? 0 : (nk >= 16 ? 4 : 16));
-    const int Gs = ((nk >= 64 || tdiff) && !cplx) ? 0 : 64;
-    struct Launch {
-        int cls, which, G, nent, nodes;
-        const int* ent;
-        const double* ngeo;
-        const unsigned char* flags;
-        const long long* pidx;
-        int ns;                       // general pairs: order of the tensor rule
-        const double *xg, *wg;
-        int q0, nq, kt0;              // slots [q0, q0 + nq) of the batch; first wavenumber column (tdiff)
-    };
-    const double* dxg = (const double*)g->d_xg.p;
-    const double* dwg = (const double*)g->d_wg.p;
-    std::vector<Launch> ls;
-    const int* gent = (const int*)g->d_gent.p;
-    const long long* gpidx = (const long long*)g->d_gpidx.p;
-    const unsigned char* gflags = (const unsigned char*)g->d_gflags.p;
-    const double* gngeo = (const double*)g->d_gngeo.p;
-    if ((g->flags & HBEM_FLAG_FAR_FIELD) && !cplx) {
-        // units of slots that share an order: blocks of 32 wavenumbers (64
-        // slots) in the tdiff layout, the whole batch otherwise
-        const int uslots = tdiff ? 64 : nk, nunit = nk / uslots;
-        std::vector<double> ukd(nunit, 0.0);
-        for (int u = 0; u < nunit; ++u)
-            for (int q = u * uslots; q < (u + 1) * uslots; ++q) ukd[u] = std::max(ukd[u], std::fabs(kap[q]) * g->dmax);
-        int off = 0;
-        for (int s = 0; s < hbem_geometry::kSep; ++s) {
-            const int cnt = g->sep[s];
-            auto order_of = [&](int u) { return s == 0 ? g->ns : far_order(ukd[u], s, g->ns); };
-            for (int u = 0; u < nunit && cnt > 0;) {
-                const int m = order_of(u);
-                int v = u + 1;
-                while (v < nunit && order_of(v) == m) ++v;
-                Launch l{2, 0, Gg, cnt, g->ns * g->ns, gent + 3 * (size_t)off,
-                         gngeo + (size_t)off * g->ns * g->ns * hbem::kNodeStride, gflags + off, gpidx + off, g->ns,
-                         dxg, dwg, u * uslots, (v - u) * uslots, tdiff ? 32 * u : 0};
-                if (m < g->ns) {
-                    auto& f = far_set(g, s, m);
-                    l.nodes = m * m;
-                    l.ngeo = (const double*)f.ngeo.p;
-                    l.flags = (const unsigned char*)f.flags.p;
-                    l.ns = m;
-                    l.xg = (const double*)f.xg.p;
-                    l.wg = (const double*)f.wg.p;
-                }
-                ls.push_back(l);
-                u = v;
-            }
-            off += cnt;
-        }
-    } else {
-        ls.push_back({2, 0, Gg, g->ngen, g->ns * g->ns, gent, gngeo, gflags, gpidx, g->ns, dxg, dwg, 0, nk, 0});
-    }
-    ls.push_back({1, 1, Gs, g->nadj, 2 * g->nc * g->nc, (const int*)g->d_aent.p, (const double*)g->d_angeo.p,
-                  (const unsigned char*)g->d_aflags.p, (const long long*)g->d_apidx.p, g->ns, dxg, dwg, 0, nk, 0});
-    ls.push_back({0, 2, Gs, g->ncoi, g->nc * g->nc, (const int*)g->d_cent.p, (const double*)g->d_cngeo.p,
-                  (const unsigned char*)g->d_cflags.p, (const long long*)g->d_cpidx.p, g->ns, dxg, dwg, 0, nk, 0});
-    for (auto& l : ls) {
-        if (l.nent == 0) continue;
-        P.nent = l.nent;
-        P.ent = l.ent;
-        P.ngeo = l.ngeo;
-        P.flags = l.flags;
-        P.pidx = l.pidx;
-        P.ns = l.ns;
-        P.xg = l.xg;
-        P.wg = l.wg;
-        P.nk = l.nq;
-        P.kap = dkap + l.q0;
-        P.kr = dkr + l.q0;
-        P.cv = dcv + l.q0;
-        if (cplx) {
-            P.kapi = dkapi + l.q0;
-            P.kri = dkri + l.q0;
-        }
-        P.kt0 = l.kt0;
-        // general pairs: one chunk; singular pairs: chunks of 2048 nodes (paired-lane
-        // kernel, 16 staging rounds; for adjacent pairs each of the two node halves
-        // is chunked on its own) or 64 x 48 nodes (one wavefront per item)
-        const int chunk_nodes = l.cls == 2 ? l.nodes : (l.G == 0 ? kChunkNodes : (l.G == 1 ? 512 : 64 * 48));
-        P.chunk = chunk_nodes;
-        P.nchunk = (l.nodes + chunk_nodes - 1) / chunk_nodes;
-        if (l.cls == 1 && l.G == 0) P.nchunk = 2 * ((l.nodes / 2 + chunk_nodes - 1) / chunk_nodes);
-        cdbl* part = nullptr;
-        if (P.nchunk > 1) part = g->w_part.as<cdbl>((size_t)nko * l.nent * P.nchunk * nslot);
+    P.tdiff = J.tdiff ? 1 : 0;
+    P.nkt = J.tdiff ? r.count : 0;
+    P.nk = r.nslots;
+    P.kap = r.kap;
+    P.kr = r.kr;
+    P.cv = r.cv;
+    P.kapi = r.kapi;
+    P.kri = r.kri;
+    int Gg, Gs;
+    loop_lanes(r.nslots, J.cplx, J.tdiff, Gg, Gs);
+    const int which[3] = {kProfCoinciding, kProfAdjacent, kProfGeneral};
+    for (int cls = 2; cls >= 0; --cls) {
+        if (set.cnt[cls] == 0) continue;
+        const int G = cls == 2 ? Gg : Gs, nodes = class_nodes(g, cls);
+        P.nent = set.cnt[cls];
+        P.ent = (const int*)set.ent[cls].p;
+        P.ngeo = (const double*)set.ngeo[cls].p;
+        P.flags = (const unsigned char*)set.flags[cls].p;
+        P.pidx = (const long long*)set.pidx[cls].p;
+        loop_chunks(cls, G, nodes, P.chunk, P.nchunk);
+        cdbl* part = (cdbl*)J.w->part.p;
         P.out = P.nchunk > 1 ? part : L;
         // the class's kernel alone is timed: the chunk sums are a separate launch
-        hipEvent_t e0 = g->prof ? g->plog.begin(g->st) : nullptr;
-        hbem::launch_assemble(l.cls, D, P, l.G, g->st);
-        HIPC(hipGetLastError());
-        if (g->prof) g->plog.end(g->st, l.which, e0, (double)l.nent * l.nq * l.nodes * flops_per_node(D));
-        if (P.nchunk > 1) {
-            hbem::launch_chunk_sum(part, l.nent, P.nchunk, nko, nslot, l.pidx, g->npairs, L, g->st);
-            HIPC(hipGetLastError());
+        hipEvent_t e0 = J.prof ? g->plog.begin(J.st) : nullptr;
+        hbem::launch_assemble(cls, J.D, P, G, J.st);
+        if (J.prof) g->plog.end(J.st, which[cls], e0, (double)P.nent * P.nk * nodes * flops_per_node(J.D));
+        if (P.nchunk > 1) hbem::launch_chunk_sum(part, P.nent, P.nchunk, nko, nslot, P.pidx, g->npairs, L, J.st);
+    }
+    const int lout = J.diff && !J.tdiff ? r.count : 0;
+    hbem::launch_records_from_locals(L, nko, J.D, lout, (int)g->npairs, J.cols + r.start, r.count, g->N, (cdbl*)J.w->E.p,
+                                     J.ncol, J.nv, J.st);
+}
+
+// Slot tables kap = k sqrt(c), k, c (imaginary parts kapi, kri: any slot is not
+// real positive) of a call with ncol columns: ncol slots, or (diff) 2 ncol, the
+// inner slots then the outer, whose differences T is formed from.  tdiff: the
+// node loops take the paired-lane kernel in the difference layout whatever the
+// width (sweeps of >= 32 wavenumbers, so that a wavenumber's bits do not depend
+// on its batch).
+RecJob prepare_records(hbem_geometry* g, RecBufs& b, RecScratch& w, hipStream_t st, const std::vector<double>& kap,
+                       const std::vector<double>& kr, const std::vector<double>& cv, int D, bool diff,
+                       const std::vector<double>& kapi = {}, const std::vector<double>& kri = {}, bool tdiff = false) {
+    RecJob J;
+    J.g = g;
+    J.w = &w;
+    J.st = st;
+    J.D = D;
+    J.diff = diff;
+    J.cplx = !kapi.empty();
+    J.tdiff = tdiff && diff && !J.cplx;
+    J.ncol = (int)kap.size() / (diff ? 2 : 1);
+    J.nslot2 = diff ? J.ncol : 0;
+    const int n = J.ncol;
+    // a column's way depends on its own kappa
+    J.nv = record_values(g, D);
+    const bool quirk = J.nv != hbem::kRecValues;
+    std::map<int, std::vector<int>> by;
+    for (int c = 0; c < n; ++c) {
+        double lo = 1e300, hi = 0.0, im = 0.0;
+        for (int h = 0; h < (diff ? 2 : 1); ++h) {
+            const int q = c + h * n;
+            const double m = J.cplx ? std::hypot(kap[q], kapi[q]) : std::fabs(kap[q]);
+            lo = std::min(lo, m);
+            hi = std::max(hi, m);
+            if (J.cplx) im = std::max(im, kapi[q]);
+        }
+        by[quirk ? -1 : record_tier(g, lo, hi, im)].push_back(c);
+    }
+    std::vector<int> cols;
+    size_t nL = 0, npart = 0, nbasis = 0;
+    size_t nl = 0;
+    for (auto& kv : by) {
+        RecGroup r;
+        r.tier = kv.first;
+        r.start = (int)cols.size();
+        r.count = (int)kv.second.size();
+        cols.insert(cols.end(), kv.second.begin(), kv.second.end());
+        if (r.tier >= 0)
+            nbasis = std::max(nbasis, (size_t)(g->rad.tier[r.tier].basis + (J.cplx ? 2 * g->rad.tier[r.tier].pnear : 0)) *
+                                          r.count * (diff ? 2 : 1));
+        if (r.tier < 0) {
+            // the group's slots: blocks of 32 wavenumbers, inner and outer in turn
+            // (tdiff), or in the order of its columns, inner then outer
+            std::vector<int> slot;
+            if (J.tdiff) {
+                const int nblk = (r.count + 31) / 32;
+                for (int q = 0; q < 64 * nblk; ++q) {
+                    const int blk = q >> 5, c = kv.second[std::min(r.count - 1, (blk >> 1) * 32 + (q & 31))];
+                    slot.push_back((blk & 1) ? c + n : c);
+                }
+            } else {
+                for (int h = 0; h < (diff ? 2 : 1); ++h)
+                    for (int c : kv.second) slot.push_back(c + h * n);
+            }
+            r.nslots = (int)slot.size();
+            auto table = [&](const std::vector<double>& v) -> double* {
+                if (v.empty()) return nullptr;
+                std::vector<double> x;
+                for (int q : slot) x.push_back(v[q]);
+                if (b.lslots.size() <= nl) b.lslots.push_back(std::make_unique<DBuf>());
+                return upload(*b.lslots[nl++], x, st);
+            };
+            r.kap = table(kap);
+            r.kr = table(kr);
+            r.cv = table(cv);
+            r.kapi = table(kapi);
+            r.kri = table(kri);
+            auto& set = node_loops(g);
+            const size_t rows = (size_t)16 * (D + 1) * (J.tdiff ? r.count : r.nslots);
+            nL = std::max(nL, rows * (size_t)g->npairs);
+            int G[2];
+            loop_lanes(r.nslots, J.cplx, J.tdiff, G[0], G[1]);
+            for (int cls = 0; cls < 3; ++cls) {
+                int chunk, nchunk;
+                loop_chunks(cls, cls == 2 ? G[0] : G[1], class_nodes(g, cls), chunk, nchunk);
+                if (nchunk > 1) npart = std::max(npart, rows * set.cnt[cls] * nchunk);
+            }
+        }
+        J.groups.push_back(r);
+    }
+    Packed pk;
+    const std::vector<double>* tabs[5] = {&kap, &kr, &cv, &kapi, &kri};
+    const double** dst[5] = {&J.kap, &J.kr, &J.cv, &J.kapi, &J.kri};
+    size_t at[5];
+    for (int i = 0; i < 5; ++i) at[i] = pk.add(*tabs[i]);
+    const size_t ocols = pk.add(cols);
+    const char* d = (const char*)b.tab.get(pk.bytes.size());
+    HIPC(hipMemcpyAsync(b.tab.p, pk.bytes.data(), pk.bytes.size(), hipMemcpyHostToDevice, st));
+    for (int i = 0; i < 5; ++i) *dst[i] = tabs[i]->empty() ? nullptr : (const double*)(d + at[i]);
+    J.cols = (const int*)(d + ocols);
+    J.obasis = al256((size_t)g->npairs * J.nv * (D + 1) * n * sizeof(cdbl));
+    w.E.get(J.obasis + nbasis * sizeof(cdbl));
+    if (nL) w.L.get(nL * sizeof(cdbl));
+    if (npart) w.part.get(npart * sizeof(cdbl));
+    HIPC(hipGetLastError());
+    return J;
+}
+
+cdbl* launch_records(const RecJob& J) {
+    hbem_geometry* g = J.g;
+    cdbl* E = (cdbl*)J.w->E.p;
+    for (const RecGroup& r : J.groups) {
+        if (r.tier >= 0) {
+            const auto& R = g->rad;
+            const auto& T = R.tier[r.tier];
+            hbem::RadialParams P;
+            P.kap = J.kap;
+            P.kapi = J.kapi;
+            P.kr = J.kr;
+            P.kri = J.kri;
+            P.cv = J.cv;
+            P.cols = J.cols + r.start;
+            P.ncolg = r.count;
+            P.nslot2 = J.nslot2;
+            P.ncol = J.ncol;
+            P.nv = J.nv;
+            P.nbasis = T.basis;
+            P.basis = (cdbl*)((char*)E + J.obasis);
+            P.out = E;
+            const auto* bands = T.bands;
+            const auto* tiles = T.tiles;
+            const auto* recs = R.recs;
+            const double *cs = T.costab, *tab = T.tab, *ext = T.ext;
+            hipEvent_t e0 = J.prof ? g->plog.begin(J.st) : nullptr;
+            hbem::launch_band_basis(P, J.diff, bands, R.nbands, T.pmax, cs, J.st);
+            hbem::launch_band_eval(J.D, J.diff, false, P, recs, tiles, R.ntile_near, R.ntile - R.ntile_near, bands, cs, tab,
+                                   ext, J.st);
+            if (J.prof)
+                g->plog.end(J.st, kProfGeneral, e0, 20.0 * (J.D + 1) * T.points * r.count * (J.diff ? 2.0 : 1.0));
+            hbem::launch_band_eval(J.D, J.diff, true, P, recs, tiles, 0, R.ntile_near, bands, cs, tab, ext, J.st);
+        } else {
+            launch_loops(J, r);
         }
     }
-    return L;
+    return E;
+}
+
+// Records of a call on the context's own buffers and stream.
+cdbl* assemble_records(hbem_geometry* g, const std::vector<double>& kap, const std::vector<double>& kr,
+                       const std::vector<double>& cv, int D, bool diff, const std::vector<double>& kapi = {},
+                       const std::vector<double>& kri = {}, bool tdiff = false) {
+    RecJob J = prepare_records(g, g->w_rec, g->w_scr, g->st, kap, kr, cv, D, diff, kapi, kri, tdiff);
+    J.prof = g->prof;
+    cdbl* E = launch_records(J);
+    HIPC(hipGetLastError());
+    return E;
+}
+
+// Device bytes per column of a call with these kappa (the larger one of each
+// column): its records, and where one of them takes the node loops for every
+// pair their local matrices and partials too.  Builds the tiers the call needs,
+// so that the free memory seen afterwards is what its batches can use.
+size_t records_bytes_per_k(hbem_geometry* g, const std::vector<double>& kap, int D, int lcols) {
+    bool loops = false;
+    for (double v : kap) {
+        loops = loops || record_tier(g, std::fabs(v), std::fabs(v), 0.0) < 0;
+    }
+    return (size_t)g->npairs * record_values(g, D) * (D + 1) * sizeof(cdbl) +
+           (loops ? locals_bytes_per_k(g->npairs, (long long)g->aent.size() / 3, g->N, g->nc, D, lcols) : 0);
 }
 
 // Dense stage shared by sv, sv_der and the sweep: given LU factors of the
@@ -672,21 +1034,19 @@ void project_inplace(hbem_geometry* g, cdbl* T, int count, cdbl* tmp = nullptr) 
 void tp_system(hbem_geometry* g, double k_re, double k_im, double c_o, double c_i, const void* U, int nrhs,
                cdbl*& T, cdbl*& rhs) {
     const double si = std::sqrt(c_i), so = std::sqrt(c_o);
-    cdbl* L = real_positive(k_re, k_im)
-                  ? assemble_locals(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, 0)
-                  : assemble_locals(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, 0, {k_im * si, k_im * so},
-                                    {k_im, k_im});
+    // the outer operators are wanted by themselves: one column per refraction index
+    cdbl* E = real_positive(k_re, k_im)
+                  ? assemble_records(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, 0, false)
+                  : assemble_records(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, 0, false,
+                                     {k_im * si, k_im * so}, {k_im, k_im});
     const int N = g->N, n = 2 * N;
     const size_t nn = (size_t)n * n;
     const double* dM = (const double*)g->d_M.p;
     T = g->w_T0.as<cdbl>(nn);
-    std::vector<int> qi = {0}, qo = {1};
-    const int* dqi = upload(g->w_qi, qi, g->st);
-    const int* dqo = upload(g->w_qo, qo, g->st);
-    hbem::launch_form_T(L, 2, 16, dqi, dqo, 1, N, 0, dM, T, nullptr, nullptr, g->st);
+    hbem::launch_form_T(E, 2, hbem::kRecValues, 0, 1, 1, N, 0, dM, T, nullptr, nullptr, g->st);
     HIPC(hipGetLastError());
     cdbl* Ao = g->w_Ao.as<cdbl>(nn);
-    hbem::launch_form_Ao(L, 2, 16, 1, N, dM, Ao, g->st);
+    hbem::launch_form_Ao(E, 2, 1, N, dM, Ao, g->st);
     HIPC(hipGetLastError());
     cdbl* dU = g->w_U.as<cdbl>((size_t)n * nrhs);
     HIPC(hipMemcpyAsync(dU, U, sizeof(cdbl) * (size_t)n * nrhs, hipMemcpyHostToDevice, g->st));
@@ -764,83 +1124,34 @@ int hbem_geometry_create(const double* panels, int npanels, const double* coefs,
     hbem::composite_rule(order, g->xc.data(), g->wc.data());
     const int N = npanels;
     g->npairs = (long long)N * (N + 1) / 2;
-    // classify pairs (galerkin_builder.cpp:872-897; adjacency test 189-201)
-    std::vector<long long> gpi, api, cpi;
-    std::vector<int> gent, aent, cent;
-    gent.reserve(3 * (size_t)g->npairs);
-    gpi.reserve((size_t)g->npairs);
+    // adjacent pairs (galerkin_builder.cpp:872-897; adjacency test 189-201)
     const double* cptr = g->coefs.empty() ? nullptr : g->coefs.data();
-    std::vector<double> ends(4 * (size_t)N), disc(3 * (size_t)N);
+    std::vector<double> ends(4 * (size_t)N);
+    g->disc.resize(3 * (size_t)N);
     hbem::panel_endpoints(g->panels.data(), cptr, N, ends.data());
-    hbem::panel_bounds(g->panels.data(), cptr, N, disc.data());
-    for (int i = 0; i < N; ++i) g->dmax = std::max(g->dmax, 2.0 * disc[3 * (size_t)i + 2]);
-    // general pairs by separation eta = (distance of the discs) / (larger
-    // diameter), a lower bound of the panels' distance in diameters
-    std::vector<int> sent[hbem_geometry::kSep];
-    std::vector<long long> spi[hbem_geometry::kSep];
-    // (line and arc panels only: a trigonometric or spline panel's |gamma'| has
-    // complex branch points a few panel lengths away, which bound every rule
-    // on the panel whatever the separation)
-    auto separation = [&](int i, int j) {
-        if ((int)g->panels[8 * (size_t)i] >= 2 || (int)g->panels[8 * (size_t)j] >= 2) return 0;
-        const double* a = &disc[3 * (size_t)i];
-        const double* b = &disc[3 * (size_t)j];
-        const double eta = (std::hypot(a[0] - b[0], a[1] - b[1]) - a[2] - b[2]) / (2.0 * std::max(a[2], b[2]));
-        return eta >= 16.0 ? 4 : (eta >= 8.0 ? 3 : (eta >= 2.0 ? 2 : (eta >= 1.0 ? 1 : 0)));
-    };
+    hbem::panel_bounds(g->panels.data(), cptr, N, g->disc.data());
+    for (int i = 0; i < N; ++i) g->dmax = std::max(g->dmax, 2.0 * g->disc[3 * (size_t)i + 2]);
     const double tol = 100.0 * hbem::kDblEps;
+    auto meet = [&](const double* a, const double* b) {
+        return std::fabs(a[0] - b[0]) < tol && std::fabs(a[1] - b[1]) < tol && std::hypot(a[0] - b[0], a[1] - b[1]) < tol;
+    };
     for (int i = 0; i < N; ++i)
-        for (int j = 0; j <= i; ++j) {
-            long long p = (long long)i * (i + 1) / 2 + j;
+        for (int j = 0; j < i; ++j) {
             const double* ei = &ends[4 * (size_t)i];
             const double* ej = &ends[4 * (size_t)j];
-            if (i == j) { cent.push_back(i); cent.push_back(i); cent.push_back(0); cpi.push_back(p); }
-            else if (std::hypot(ei[2] - ej[0], ei[3] - ej[1]) < tol) {            // end(i) == start(j)
-                aent.push_back(i); aent.push_back(j); aent.push_back(0); api.push_back(p);
-            } else if (std::hypot(ei[0] - ej[2], ei[1] - ej[3]) < tol) {          // start(i) == end(j)
-                aent.push_back(i); aent.push_back(j); aent.push_back(1); api.push_back(p);
-            } else {
-                const int s = separation(i, j);
-                sent[s].push_back(i); sent[s].push_back(j); sent[s].push_back(0); spi[s].push_back(p);
-            }
+            if (meet(ei + 2, ej)) g->aent.insert(g->aent.end(), {i, j, 0});           // end(i) == start(j)
+            else if (meet(ei, ej + 2)) g->aent.insert(g->aent.end(), {i, j, 1});      // start(i) == end(j)
         }
-    for (int s = 0; s < hbem_geometry::kSep; ++s) {
-        g->sep[s] = (int)spi[s].size();
-        gent.insert(gent.end(), sent[s].begin(), sent[s].end());
-        gpi.insert(gpi.end(), spi[s].begin(), spi[s].end());
-        std::vector<int>().swap(sent[s]);
-        std::vector<long long>().swap(spi[s]);
-    }
-    g->ngen = (int)gpi.size();
-    g->nadj = (int)api.size();
-    g->ncoi = (int)cpi.size();
     hipStream_t st = g->st;
     const double* dpan = upload(g->d_panels, g->panels, st);
     std::vector<double> cf = g->coefs.empty() ? std::vector<double>(3, 0.0) : g->coefs;
     const double* dcoef = upload(g->d_coefs, cf, st);
     const double* dxg = upload(g->d_xg, g->xg, st);
     upload(g->d_wg, g->wg, st);
-    const double* dxc = upload(g->d_xc, g->xc, st);
+    upload(g->d_xc, g->xc, st);
     upload(g->d_wc, g->wc, st);
     double* gtab = g->d_gtab.as<double>((size_t)N * g->ns * 5);
     hbem::launch_setup_gauss_table(dpan, dcoef, N, dxg, g->ns, gtab, st);
-    upload(g->d_gent, gent, st);
-    upload(g->d_gpidx, gpi, st);
-    g->d_gflags.get(std::max(1, g->ngen));
-    double* gngeo = g->d_gngeo.as<double>(std::max<size_t>(1, (size_t)g->ngen * g->ns * g->ns * hbem::kNodeStride));
-    hbem::launch_setup_general((const int*)g->d_gent.p, g->ngen, gtab, g->ns, gngeo, (unsigned char*)g->d_gflags.p, st);
-    upload(g->d_aent, aent, st);
-    upload(g->d_apidx, api, st);
-    g->d_aflags.get(std::max(1, g->nadj));
-    double* angeo = g->d_angeo.as<double>(std::max<size_t>(1, (size_t)g->nadj * 2 * g->nc * g->nc * hbem::kNodeStride));
-    hbem::launch_setup_singular(1, (const int*)g->d_aent.p, g->nadj, dpan, dcoef, dxc, g->nc, angeo,
-                                (unsigned char*)g->d_aflags.p, st);
-    upload(g->d_cent, cent, st);
-    upload(g->d_cpidx, cpi, st);
-    g->d_cflags.get(std::max(1, g->ncoi));
-    double* cngeo = g->d_cngeo.as<double>(std::max<size_t>(1, (size_t)g->ncoi * g->nc * g->nc * hbem::kNodeStride));
-    hbem::launch_setup_singular(0, (const int*)g->d_cent.p, g->ncoi, dpan, dcoef, dxc, g->nc, cngeo,
-                                (unsigned char*)g->d_cflags.p, st);
     HIPC(hipGetLastError());
     // mass matrix and projection factor (gen_sol_op.cpp:23-43)
     g->M.resize((size_t)N * N);
@@ -896,11 +1207,13 @@ int hbem_geometry_release_work(hbem_geometry_t g) {
     std::lock_guard<std::mutex> lk(g->mu);
     HIPC(hipSetDevice(g->dev));
     HIPC(hipStreamSynchronize(g->st));
-    DBuf* bs[] = {&g->w_Ao, &g->w_U, &g->w_rhs, &g->w_flag, &g->w_Tp, &g->w_B, &g->w_mv, &g->w_bpiv, &g->w_bperm,
-                  &g->w_bvec, &g->w_d2, &g->w_T32, &g->w_rb, &g->w_rr, &g->w_rpart, &g->w_flag2, &g->w_rprev, &g->w_kapi, &g->w_kri,
-                  &g->w_L, &g->w_T0, &g->w_T1, &g->w_T2, &g->w_piv, &g->w_perm, &g->w_X, &g->w_Y, &g->w_work,
-                  &g->w_R, &g->w_u, &g->w_v, &g->w_a, &g->w_b, &g->w_sig, &g->w_dsig, &g->w_kap, &g->w_kr, &g->w_cv,
-                  &g->w_qi, &g->w_qo, &g->w_tmp, &g->w_out, &g->w_part};
+    std::vector<DBuf*> bs = {&g->w_Ao, &g->w_U, &g->w_rhs, &g->w_flag, &g->w_Tp, &g->w_B, &g->w_mv, &g->w_bpiv, &g->w_bperm,
+                             &g->w_bvec, &g->w_d2, &g->w_T32, &g->w_rb, &g->w_rr, &g->w_rpart, &g->w_flag2, &g->w_rprev,
+                             &g->w_T0, &g->w_T1, &g->w_T2, &g->w_piv, &g->w_perm, &g->w_X, &g->w_Y, &g->w_work,
+                             &g->w_R, &g->w_u, &g->w_v, &g->w_a, &g->w_b, &g->w_sig, &g->w_dsig, &g->w_tmp, &g->w_out,
+                             &g->w_rec.tab,
+                             &g->w_scr.E, &g->w_scr.L, &g->w_scr.part};
+    for (auto& b : g->w_rec.lslots) bs.push_back(b.get());
     for (DBuf* b : bs) {
         if (b->p) (void)hipFree(b->p);
         b->p = nullptr;
@@ -928,12 +1241,12 @@ int hbem_assemble_dense(hbem_geometry_t g, double k_re, double k_im, double c, i
     std::lock_guard<std::mutex> lk(g->mu);
     HIPC(hipSetDevice(g->dev));
     const double sc = std::sqrt(c);
-    cdbl* L = real_positive(k_re, k_im) ? assemble_locals(g, {k_re * sc}, {k_re}, {c}, d)
-                                        : assemble_locals(g, {k_re * sc}, {k_re}, {c}, d, {k_im * sc}, {k_im});
+    cdbl* E = real_positive(k_re, k_im) ? assemble_records(g, {k_re * sc}, {k_re}, {c}, d, false)
+                                        : assemble_records(g, {k_re * sc}, {k_re}, {c}, d, false, {k_im * sc}, {k_im});
     const int N = g->N;
     const size_t NN = (size_t)N * N * (d + 1);
     cdbl* out = g->w_out.as<cdbl>(3 * NN);
-    hbem::launch_gather_layers(L, 1, 16 * (d + 1), 0, N, d, layers, out, out + NN, out + 2 * NN, g->st);
+    hbem::launch_gather_layers(E, 1, record_values(g, d), 0, N, d, layers, out, out + NN, out + 2 * NN, g->st);
     HIPC(hipGetLastError());
     if (layers & HBEM_LAYER_DOUBLE) copy_out_square(out, K, NN, g->st);
     if (layers & HBEM_LAYER_HYPERSINGULAR) copy_out_square(out + NN, W, NN, g->st);
@@ -955,16 +1268,11 @@ int hbem_assemble_dense_batch(hbem_geometry_t g, const double* ks, int nk, doubl
     const int N = g->N;
     const size_t NN = (size_t)N * N * (d + 1);
     cdbl* out = g->w_out.as<cdbl>(3 * NN);
-    // one wavenumber slot per k: its local matrices and chunk partials
-    const size_t nslot = 16 * (size_t)(d + 1);
-    const size_t part = (size_t)std::max(g->nadj * adj_chunks(g->nc), g->ncoi * coi_chunks(g->nc));
-    const size_t per = ((size_t)g->npairs + part) * nslot * sizeof(cdbl);
-    {
-        std::vector<double> all(nk);
-        for (int i = 0; i < nk; ++i) all[i] = ks[i] * sc;
-        prepare_far(g, all);
-    }
-    const int B = sweep_batch(per, usable_device_bytes(g->w_L.n + g->w_part.n), nk);
+    // one wavenumber slot per k: its records, and its local matrices where it takes the node loops
+    std::vector<double> all(nk);
+    for (int i = 0; i < nk; ++i) all[i] = ks[i] * sc;
+    const size_t per = records_bytes_per_k(g, all, d, 1);
+    const int B = sweep_batch(per, usable_device_bytes(g->w_scr.E.n + g->w_scr.L.n + g->w_scr.part.n), nk);
     for (int k0 = 0; k0 < nk; k0 += B) {
         const int nb = std::min(B, nk - k0);
         std::vector<double> kap(nb), kr(nb), cv(nb, c);
@@ -975,9 +1283,9 @@ int hbem_assemble_dense_batch(hbem_geometry_t g, const double* ks, int nk, doubl
             allpos = allpos && ks[k0 + b] > 0.0;
         }
         const std::vector<double> zero(allpos ? 0 : nb, 0.0);
-        cdbl* L = assemble_locals(g, kap, kr, cv, d, zero, zero);
+        cdbl* E = assemble_records(g, kap, kr, cv, d, false, zero, zero);
         for (int b = 0; b < nb; ++b) {
-            hbem::launch_gather_layers(L, nb, 16 * (d + 1), b, N, d, layers, out, out + NN, out + 2 * NN, g->st);
+            hbem::launch_gather_layers(E, nb, record_values(g, d), b, N, d, layers, out, out + NN, out + 2 * NN, g->st);
             HIPC(hipGetLastError());
             const size_t off = (size_t)(k0 + b) * NN * sizeof(cdbl);
             if ((layers & HBEM_LAYER_DOUBLE) && K) copy_out_square(out, (char*)K + off, NN, g->st);
@@ -1015,19 +1323,16 @@ int hbem_gen_sol_op(hbem_geometry_t g, double k_re, double k_im, double c_o, dou
     std::lock_guard<std::mutex> lk(g->mu);
     HIPC(hipSetDevice(g->dev));
     const double si = std::sqrt(c_i), so = std::sqrt(c_o);
-    cdbl* L = real_positive(k_re, k_im)
-                  ? assemble_locals(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, d)
-                  : assemble_locals(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, d, {k_im * si, k_im * so},
-                                    {k_im, k_im});
+    cdbl* E = real_positive(k_re, k_im)
+                  ? assemble_records(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, d, true)
+                  : assemble_records(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, d, true,
+                                     {k_im * si, k_im * so}, {k_im, k_im});
     const int n = 2 * g->N;
     const size_t nn = (size_t)n * n;
     cdbl* T0 = g->w_T0.as<cdbl>(nn);
     cdbl* T1 = d >= 1 ? g->w_T1.as<cdbl>(nn) : nullptr;
     cdbl* T2 = d >= 2 ? g->w_T2.as<cdbl>(nn) : nullptr;
-    std::vector<int> qi = {0}, qo = {1};
-    const int* dqi = upload(g->w_qi, qi, g->st);
-    const int* dqo = upload(g->w_qo, qo, g->st);
-    hbem::launch_form_T(L, 2, 16 * (d + 1), dqi, dqo, 1, g->N, d, (const double*)g->d_M.p, T0, T1, T2, g->st);
+    hbem::launch_form_T(E, 1, record_values(g, d), 0, -1, 1, g->N, d, (const double*)g->d_M.p, T0, T1, T2, g->st);
     HIPC(hipGetLastError());
     cdbl* Ts[3] = {T0, T1, T2};
     void* hs[3] = {T, Td, Tdd};
@@ -1468,24 +1773,17 @@ void sweep_run(hbem_geometry* g, const double* ks, int nk, double c_o, double c_
     const int n = 2 * g->N;
     const size_t nn = (size_t)n * n;
     const bool mx = mixed >= 0 && D == 0 && !d2sigma;
-    // Batch of B wavenumbers -> slots in blocks of 32 consecutive k of one
-    // refraction index: each wavefront of the assembly sees a single index
-    // and neighbouring k, so the arguments kappa r of its lanes stay close
-    // (fewer divergent Bessel branches).  B <= 256 gives the dense stage (one
-    // workgroup per matrix in the panel factorisation and the thin solves)
-    // up to one matrix per CU.  B is bounded by the free device memory: local
-    // matrices, chunk partials and T, T', T'' per wavenumber (and the
-    // bordered systems of the sigma'' stage).
+    // Batches of B <= 256 wavenumbers give the dense stage (one workgroup per
+    // matrix in the panel factorisation and the thin solves) up to one matrix
+    // per CU.  B is bounded by the free device memory: records (and local
+    // matrices and chunk partials where a wavenumber takes the node loops) and
+    // T, T', T'' per wavenumber (and the bordered systems of the sigma'' stage).
     const bool tdiff = sweep_tdiff(ks, nk);
-    const size_t per = sweep_bytes_per_k(g->npairs, g->nadj, g->ncoi, g->nc, n, D, nc, tdiff ? 1 : 2) +
-                       (d2sigma ? der2_bytes_per_k(n) : 0) +
-                       (mx ? mixed_bytes_per_k(n, nc) : 0);
-    {
-        std::vector<double> all;
-        for (int i = 0; i < nk; ++i)
-            if (ks[i] > 0.0) { all.push_back(ks[i] * std::sqrt(c_i)); all.push_back(ks[i] * std::sqrt(c_o)); }
-        prepare_far(g, all);
-    }
+    const double si = std::sqrt(c_i), so = std::sqrt(c_o);
+    std::vector<double> all;
+    for (int i = 0; i < nk; ++i) all.push_back(ks[i] * std::max(si, so));
+    const size_t per = records_bytes_per_k(g, all, D, tdiff ? 1 : 2) + dense_bytes_per_k(n, D, nc) +
+                       (d2sigma ? der2_bytes_per_k(n) : 0) + (mx ? mixed_bytes_per_k(n, nc) : 0);
     const int B = sweep_batch(per, usable_device_bytes(g->work_held()), nk);
     cdbl* dR = g->w_R.as<cdbl>((size_t)n * nc);
     HIPC(hipMemcpyAsync(dR, R, (size_t)n * nc * sizeof(cdbl), hipMemcpyHostToDevice, g->st));
@@ -1493,36 +1791,23 @@ void sweep_run(hbem_geometry* g, const double* ks, int nk, double c_o, double c_
         const int nb = std::min(B, nk - k0);
         bool allpos = true;
         for (int b = 0; b < nb; ++b) allpos = allpos && ks[k0 + b] > 0.0;
-        std::vector<double> kap, kr, cv;
-        std::vector<int> qi(nb), qo(nb);
-        if (tdiff) {
-            tdiff_slots(ks + k0, nb, c_i, c_o, kap, kr, cv);
-            for (int b = 0; b < nb; ++b) qi[b] = b;
-        } else {
-            // inner slots 0..nb-1, outer nb..2nb-1
-            kap.resize(2 * nb); kr.resize(2 * nb); cv.resize(2 * nb);
-            for (int b = 0; b < nb; ++b) {
-                const double k = ks[k0 + b];
-                kap[b] = k * std::sqrt(c_i); kr[b] = k; cv[b] = c_i;
-                kap[nb + b] = k * std::sqrt(c_o); kr[nb + b] = k; cv[nb + b] = c_o;
-                qi[b] = b;
-                qo[b] = nb + b;
-            }
+        // inner slots 0..nb-1, outer nb..2nb-1
+        std::vector<double> kap(2 * nb), kr(2 * nb), cv(2 * nb);
+        for (int b = 0; b < nb; ++b) {
+            const double k = ks[k0 + b];
+            kap[b] = k * si; kr[b] = k; cv[b] = c_i;
+            kap[nb + b] = k * so; kr[nb + b] = k; cv[nb + b] = c_o;
         }
         const std::vector<double> zero(allpos ? 0 : kap.size(), 0.0);
-        cdbl* L = assemble_locals(g, kap, kr, cv, D, zero, zero, tdiff ? nb : 0);
-        const int lcols = tdiff ? nb : 2 * nb;   // columns of the local buffer
+        cdbl* E = assemble_records(g, kap, kr, cv, D, true, zero, zero, tdiff);
         cdbl* T0 = g->w_T0.as<cdbl>(nn * nb);
         cdbl* T1 = D >= 1 ? g->w_T1.as<cdbl>(nn * nb) : nullptr;
         cdbl* T2 = D >= 2 ? g->w_T2.as<cdbl>(nn * nb) : nullptr;
-        const int* dqi = upload(g->w_qi, qi, g->st);
-        const int* dqo = tdiff ? nullptr : upload(g->w_qo, qo, g->st);
         // mixed precision: T formed in FP64 (kept for the residuals) and in FP32
         // (factorised on the FP32 matrix cores) in one pass
         cflt* T32 = mx ? g->w_T32.as<cflt>(nn * nb) : nullptr;
         hipEvent_t e0 = g->prof ? g->plog.begin(g->st) : nullptr;
-        hbem::launch_form_T(L, lcols, 16 * (D + 1), dqi, dqo, nb, g->N, D, (const double*)g->d_M.p, T0, T1, T2, g->st, 0,
-                            T32);
+        hbem::launch_form_T(E, nb, record_values(g, D), 0, -1, nb, g->N, D, (const double*)g->d_M.p, T0, T1, T2, g->st, 0, T32);
         if (g->prof) g->plog.end(g->st, kProfFormT, e0);
         int* piv = g->w_piv.as<int>((size_t)n * nb);
         int* perm = g->w_perm.as<int>((size_t)n * nb);
@@ -1600,8 +1885,8 @@ void sweep_run(hbem_geometry* g, const double* ks, int nk, double c_o, double c_
             const int m2 = 2 * n;
             cdbl* Tp = g->w_Tp.as<cdbl>(nn * nb);
             cdbl* Bw = g->w_B.as<cdbl>(4 * nn * nb);
-            hbem::launch_form_T(L, lcols, 16 * (D + 1), dqi, dqo, nb, g->N, 0, (const double*)g->d_M.p, Tp, nullptr,
-                                nullptr, g->st);
+            hbem::launch_form_T(E, nb, record_values(g, D), 0, -1, nb, g->N, D, (const double*)g->d_M.p, Tp, nullptr, nullptr, g->st, 0, nullptr,
+                                true);
             if (g->proj) project_inplace(g, Tp, nb, Bw);
             int* mv = g->w_mv.as<int>(nb);
             cdbl* vec = g->w_bvec.as<cdbl>(16 * (size_t)n * nb);
@@ -1692,8 +1977,9 @@ struct GraphEntry {
 };
 struct MultiWork {
     std::mutex mu;
-    DBuf ent[3], flags[3], pidx[3], einst[3], igeo[3], ibase[3], kap, kr, cv, L, part[3], T, piv, perm, X, Y, work, sig,
-        qi, desc, descT, roff, nrow, Rall;
+    DBuf T, piv, perm, X, Y, work, sig, desc, descT, roff, nrow, Rall;
+    std::vector<std::unique_ptr<RecBufs>> rec;   // per instance of a subset
+    RecScratch scr;
     std::vector<GraphEntry> graphs;
     void drop_graphs() {
         for (auto& e : graphs) (void)hipGraphExecDestroy(e.exec);
@@ -1737,53 +2023,22 @@ void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& 
     hbem_geometry* g0 = G[ids[0]];
     const hipStream_t st = g0->st;
     const int m = (int)ids.size();
-    const int nslot = 16, nks = 64 * ((nk + 31) / 32);   // tdiff slots per instance
     const size_t nn = (size_t)n_pad * n_pad;
     const int batch = m * nk;
     // ---- host side: every table the device phase reads, uploaded first ----
-    // slots of instance i: its nk wavenumbers in the tdiff layout (blocks of
-    // 32 with c_i(i), then c_o); the local buffer holds the T differences, nk
-    // columns
-    std::vector<double> kap, kr, cv;
-    std::vector<long long> pair_off(m + 1, 0);
+    const bool tdiff = true;                  // the difference layout of hbem_sigma_sweep (nk >= 32)
+    std::vector<RecJob> jobs;
+    while ((int)w.rec.size() < m) w.rec.push_back(std::make_unique<RecBufs>());
     for (int a = 0; a < m; ++a) {
         const int i = ids[a];
-        std::vector<double> ka, kb, kc;
-        tdiff_slots(ks + (size_t)i * nk, nk, c_i[i], c_o, ka, kb, kc);
-        kap.insert(kap.end(), ka.begin(), ka.end());
-        kr.insert(kr.end(), kb.begin(), kb.end());
-        cv.insert(cv.end(), kc.begin(), kc.end());
-        pair_off[a + 1] = pair_off[a] + G[i]->npairs;
-    }
-    const double* dkap = upload(w.kap, kap, st);
-    const double* dkr = upload(w.kr, kr, st);
-    const double* dcv = upload(w.cv, cv, st);
-    struct ClassPlan {
-        long long ne = 0;
-        std::vector<long long> base;
-        int nodes = 0, nchunk = 1;
-    } cp[3];
-    const double* const* digeo[3] = {nullptr, nullptr, nullptr};
-    const long long* dibase[3] = {nullptr, nullptr, nullptr};
-    for (int cls = 0; cls < 3; ++cls) {
-        ClassPlan& c = cp[cls];
-        c.base.assign(m + 1, 0);
-        std::vector<const double*> geo(m);
-        for (int a = 0; a < m; ++a) {
-            hbem_geometry* g = G[ids[a]];
-            const int ne = cls == 2 ? g->ngen : cls == 1 ? g->nadj : g->ncoi;
-            c.base[a + 1] = c.base[a] + ne;
-            geo[a] = (const double*)(cls == 2 ? g->d_gngeo.p : cls == 1 ? g->d_angeo.p : g->d_cngeo.p);
+        std::vector<double> kap(2 * nk), kr(2 * nk), cv(2 * nk);
+        for (int j = 0; j < nk; ++j) {
+            const double k = ks[(size_t)i * nk + j];
+            kap[j] = k * std::sqrt(c_i[i]); kr[j] = k; cv[j] = c_i[i];
+            kap[nk + j] = k * std::sqrt(c_o); kr[nk + j] = k; cv[nk + j] = c_o;
         }
-        c.ne = c.base[m];
-        c.nodes = cls == 2 ? g0->ns * g0->ns : cls == 1 ? 2 * g0->nc * g0->nc : g0->nc * g0->nc;
-        c.nchunk = cls == 2 ? 1 : cls == 1 ? (int)adj_chunks(g0->nc) : (int)coi_chunks(g0->nc);
-        digeo[cls] = upload(w.igeo[cls], geo, st);
-        dibase[cls] = upload(w.ibase[cls], c.base, st);
+        jobs.push_back(prepare_records(G[i], *w.rec[a], w.scr, st, kap, kr, cv, 0, true, {}, {}, tdiff));
     }
-    std::vector<int> qi(nk);
-    for (int j = 0; j < nk; ++j) qi[j] = j;
-    const int* dqi = upload(w.qi, qi, st);
     std::vector<hbem::CsrDesc> desc(batch), descT(batch);
     std::vector<long long> roff(batch);
     std::vector<int> nrow(batch);
@@ -1810,20 +2065,6 @@ void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& 
     const long long* droff = upload(w.roff, roff, st);
     const int* dnrow = upload(w.nrow, nrow, st);
     // ---- every device buffer at its final size before the device phase ----
-    cdbl* L = w.L.as<cdbl>((size_t)pair_off[m] * nslot * nk);
-    int* ent[3];
-    unsigned char* fl[3];
-    long long* pidx[3];
-    int* einst[3];
-    cdbl* part[3];
-    for (int cls = 0; cls < 3; ++cls) {
-        const size_t ne = (size_t)std::max<long long>(cp[cls].ne, 1);
-        ent[cls] = w.ent[cls].as<int>(3 * ne);
-        fl[cls] = w.flags[cls].as<unsigned char>(ne);
-        pidx[cls] = w.pidx[cls].as<long long>(ne);
-        einst[cls] = w.einst[cls].as<int>(ne);
-        part[cls] = cp[cls].nchunk > 1 ? w.part[cls].as<cdbl>((size_t)nk * ne * cp[cls].nchunk * nslot) : nullptr;
-    }
     cdbl* T = w.T.as<cdbl>(nn * batch);
     int* piv = w.piv.as<int>((size_t)n_pad * batch);
     int* perm = w.perm.as<int>((size_t)n_pad * batch);
@@ -1834,58 +2075,12 @@ void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& 
     HIPC(hipStreamSynchronize(st));   // uploads done; nothing below reads host memory
     // ---- device phase ----
     auto device_phase = [&]() {
-        hbem::AsmParams P;
-        std::memset(&P, 0, sizeof(P));
-        P.xg = (const double*)g0->d_xg.p;
-        P.wg = (const double*)g0->d_wg.p;
-        P.xc = (const double*)g0->d_xc.p;
-        P.wc = (const double*)g0->d_wc.p;
-        P.nk = nks;
-        P.kap = dkap;
-        P.kr = dkr;
-        P.cv = dcv;
-        P.npairs_total = pair_off[m];
-        P.ns = g0->ns;
-        P.nc = g0->nc;
-        P.qflags = g0->flags;
-        P.tdiff = 1;
-        P.nkt = nk;
-        for (int cls = 2; cls >= 0; --cls) {
-            const ClassPlan& c = cp[cls];
-            if (c.ne == 0) continue;
-            for (int a = 0; a < m; ++a) {
-                hbem_geometry* g = G[ids[a]];
-                const long long cnt = c.base[a + 1] - c.base[a];
-                if (cnt == 0) continue;
-                const DBuf& de = cls == 2 ? g->d_gent : cls == 1 ? g->d_aent : g->d_cent;
-                const DBuf& df = cls == 2 ? g->d_gflags : cls == 1 ? g->d_aflags : g->d_cflags;
-                const DBuf& dp = cls == 2 ? g->d_gpidx : cls == 1 ? g->d_apidx : g->d_cpidx;
-                hbem::copy_bytes(ent[cls] + 3 * c.base[a], de.p, 3 * cnt * sizeof(int), st);
-                hbem::copy_bytes(fl[cls] + c.base[a], df.p, (size_t)cnt, st);
-                hbem::copy_bytes(pidx[cls] + c.base[a], dp.p, cnt * sizeof(long long), st);
-                hbem::add_offset_ll(pidx[cls] + c.base[a], cnt, pair_off[a], st);
-                hbem::fill_int(einst[cls] + c.base[a], (int)cnt, a, st);
-            }
-            P.igeo = digeo[cls];
-            P.ibase = dibase[cls];
-            P.einst = einst[cls];
-            P.ent = ent[cls];
-            P.flags = fl[cls];
-            P.pidx = pidx[cls];
-            P.nent = (int)c.ne;
-            P.ngeo = nullptr;
-            P.chunk = cls == 2 ? c.nodes : kChunkNodes;
-            P.nchunk = c.nchunk;
-            P.out = c.nchunk > 1 ? part[cls] : L;
-            hbem::launch_assemble(cls, 0, P, 0, st);
-            if (c.nchunk > 1)
-                hbem::launch_chunk_sum(part[cls], (int)c.ne, c.nchunk, nk, nslot, pidx[cls], pair_off[m], L, st);
-        }
         for (int a = 0; a < m; ++a) {
             hbem_geometry* g = G[ids[a]];
             const int n = 2 * g->N;
-            hbem::launch_form_T(L + (size_t)pair_off[a] * nslot * nk, nk, nslot, dqi, nullptr, nk, g->N, 0,
-                                (const double*)g->d_M.p, T + (size_t)a * nk * nn, nullptr, nullptr, st, n_pad);
+            const cdbl* E = launch_records(jobs[a]);
+            hbem::launch_form_T(E, nk, hbem::kRecValues, 0, -1, nk, g->N, 0, (const double*)g->d_M.p, T + (size_t)a * nk * nn, nullptr,
+                                nullptr, st, n_pad);
             if (n < n_pad) hbem::launch_pad_identity(T + (size_t)a * nk * nn, n, n_pad, nk, st);
         }
         hbem::lu_factor_batched(T, n_pad, batch, piv, perm, st);
@@ -1908,10 +2103,16 @@ void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& 
         key.push_back((const void*)(size_t)nc);
         key.push_back((const void*)(size_t)q);
         key.push_back((const void*)(size_t)n_pad);
-        const void* bufs[] = {dkap, dkr, dcv, digeo[0], digeo[1], digeo[2], dibase[0], dibase[1], dibase[2], dqi,
-                              dF, dFT, dRall, droff, dnrow, L, T, piv, perm, X, Y, work, dsig,
-                              ent[0], ent[1], ent[2], fl[0], fl[1], fl[2], pidx[0], pidx[1], pidx[2], einst[0],
-                              einst[1], einst[2], part[0], part[1], part[2]};
+        const void* bufs[] = {dF, dFT, dRall, droff, dnrow, T, piv, perm, X, Y, work, dsig, w.scr.E.p, w.scr.L.p,
+                              w.scr.part.p};
+        // the ways its columns take, and the tables each reads
+        for (const RecJob& J : jobs) {
+            for (const void* p : {(const void*)J.kap, (const void*)J.kr, (const void*)J.cv, (const void*)J.cols}) key.push_back(p);
+            for (const RecGroup& r : J.groups)
+                for (const void* p : {(const void*)(size_t)(r.tier + 1), (const void*)(size_t)r.start, (const void*)(size_t)r.count,
+                                      (const void*)r.kap, (const void*)r.kr, (const void*)r.cv})
+                    key.push_back(p);
+        }
         key.insert(key.end(), std::begin(bufs), std::end(bufs));
         GraphEntry* ge = nullptr;
         for (auto& e : w.graphs)
@@ -1979,7 +2180,7 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
     size_t held = 0;
     {
         MultiWork& w = g_multi;
-        const DBuf* bs[] = {&w.L, &w.part[0], &w.part[1], &w.part[2], &w.T, &w.piv, &w.perm, &w.X, &w.Y, &w.work};
+        const DBuf* bs[] = {&w.scr.E, &w.scr.L, &w.scr.part, &w.T, &w.piv, &w.perm, &w.X, &w.Y, &w.work};
         for (auto* b : bs) held += b->n;
     }
     const size_t avail = usable_device_bytes(held);
@@ -1990,8 +2191,11 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
         size_t used = 0;
         while (a < key.size() && key[a].first == n_pad) {
             hbem_geometry* g = G[key[a].second];
-            const size_t part = (size_t)std::max(g->nadj * adj_chunks(g->nc), g->ncoi * coi_chunks(g->nc));
-            const size_t need = (size_t)nk * ((size_t)g->npairs + part) * 16 * sizeof(cdbl) +
+            const double* kg = ks + (size_t)key[a].second * nk;
+            const double cm = std::sqrt(std::max(c_i[key[a].second], c_o));
+            std::vector<double> kap;
+            for (int j = 0; j < nk; ++j) kap.push_back(kg[j] * cm);
+            const size_t need = (size_t)nk * records_bytes_per_k(g, kap, 0, 1) +
                                 (size_t)nk * ((size_t)n_pad * n_pad * sizeof(cdbl) + (size_t)n_pad * (8 + (4 * nc + 4) * sizeof(cdbl)));
             if (!ids.empty() && used + need > avail) break;
             ids.push_back(key[a].second);
@@ -2031,7 +2235,8 @@ int hbem_sweep_batch_size(int npanels, int order, int d, int nc, unsigned long l
     // a closed curve of N panels: N coinciding, N adjacent pairs
     const long long N = npanels;
     const int ncr = order * (order + 1) / 2 - 1;
-    *B = sweep_batch(sweep_bytes_per_k(N * (N + 1) / 2, N, N, ncr, 2 * npanels, d, nc, nk >= 32 ? 1 : 2),
+    *B = sweep_batch(locals_bytes_per_k(N * (N + 1) / 2, N, N, ncr, d, nk >= 32 ? 1 : 2) +
+                         dense_bytes_per_k(2 * npanels, d, nc),
                      (size_t)avail_bytes, nk);
     API_END
 }

@@ -181,6 +181,56 @@ __device__ __forceinline__ void bessel_jy01(double x, double& j0, double& y0, do
     }
 }
 
+// J0, Y0, J1, Y1 of x = kappa r from the node's kappa-free factors.
+//   y = x^2 / 64, L2 = (2/pi) ln(x/2) = lk + lr, 1/x = kinv / r,
+//   1/sqrt(pi x) = ksq / sqrt(r)
+// TINY >= 1 (touching panel pairs, whose arguments are small): x < HBEM_TINY_X
+// takes the entire parts from the degree-HBEM_TINY_DEG table fitted on that
+// range instead of the degree-HBEM_SMALL_DEG table of (0, 8); TINY = 2 takes
+// x < HBEM_TINY1_X from the degree-HBEM_TINY1_DEG table of that range first.
+// sin / cos beyond x = 1e6 (never reached by the benchmark's arguments): kept
+// out of line so the library routine's constants do not occupy registers of
+// the callers' loops
+static __device__ __noinline__ void sincos_far(double x, double& s, double& c) { sincos(x, &s, &c); }
+
+template <int TINY>
+__device__ __forceinline__ void bessel_jy01_f(double x, double y, double L2, double xinv, double b, double& j0,
+                                              double& y0, double& j1, double& y1) {
+    if (x < 8.0) {
+        double A, B, C, Dd;
+        if (TINY >= 2 && x < (double)HBEM_TINY1_X)
+            horner4<HBEM_TINY1_DEG>(bessel_table() + HBEM_TAB_TINY1, y, A, B, C, Dd);
+        else if (TINY >= 1 && x < (double)HBEM_TINY_X)
+            horner4<HBEM_TINY_DEG>(bessel_table() + HBEM_TAB_TINY, y, A, B, C, Dd);
+        else
+            horner4<HBEM_SMALL_DEG>(bessel_table() + HBEM_TAB_SMALL, y, A, B, C, Dd);
+        const bool pos = x > 0.0;
+        const double J1 = x * B;
+        j0 = pos ? A : 1.0;
+        j1 = pos ? J1 : 0.0;
+        y0 = pos ? fma(L2, A, C) : 0.0;
+        y1 = pos ? fma(L2, J1, fma(x, Dd, -kTwoOverPi * xinv)) : 0.0;
+    } else if (x <= 1e6) {
+        double s, c;
+        sincos_med(x, s, c);
+        const double cs = c + s, sc = s - c;
+        const double z = 64.0 * xinv * xinv;
+        double P0, Q0, P1, Q1;
+        horner4<HBEM_PQ_DEG>(bessel_table() + HBEM_TAB_PQ, z, P0, Q0, P1, Q1);
+        Q0 *= xinv;
+        Q1 *= xinv;
+        j0 = b * fma(P0, cs, -Q0 * sc);
+        y0 = b * fma(P0, sc, Q0 * cs);
+        j1 = b * fma(P1, sc, Q1 * cs);
+        y1 = b * fma(Q1, sc, -P1 * cs);
+    } else {
+        double s, c;
+        sincos_far(x, s, c);
+        const double cs = c + s, sc = s - c;
+        j0 = b * cs; y0 = b * sc; j1 = b * sc; y1 = -b * cs;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Complex helpers and H0, H1 of complex argument (wavenumbers that are not
 // real positive: GalerkinBuilder::H1_01_cplx, galerkin_builder.cpp:224-235)
@@ -268,6 +318,58 @@ __device__ inline void hankel01_cplx(cdbl z, cdbl& h0, cdbl& h1) {
     h1 = (-kTwoOverPi) * k1;
     if (!(isfinite(h0.x) && isfinite(h0.y))) h0 = mk(0.0, 0.0);
     if (!(isfinite(h1.x) && isfinite(h1.y))) h1 = mk(0.0, 0.0);
+}
+
+// J0(z), J1(z) / z and the entire parts C, D of Y0 = (2/pi) ln(z/2) J0 + C and
+// Y1 = (2/pi) ln(z/2) J1 - 2 / (pi z) + z D for complex z, Im z >= 0, |z| <=
+// kEntireMax: the ascending series (A&S 9.1.10-9.1.13) for |z| <= 2; above it J
+// by Miller's backward recurrence J_{n-1} = (2n / z) J_n - J_{n+1} normalised by
+// e^{-iz} = J0 + 2 sum (-i)^n J_n (A&S 9.1.27, 9.1.41-45), whose left side is not
+// small for Im z >= 0, and the parts from H0, H1.
+constexpr double kEntireMax = 200.0;
+__device__ inline void bessel_entire_cplx(cdbl z, cdbl& j0, cdbl& c0, cdbl& j1, cdbl& c1) {
+    if (cabsd(z) <= 2.0) {
+        const cdbl t = -0.25 * (z * z);
+        cdbl term = mk(1.0, 0.0), u = mk(1.0, 0.0), a = term, b = u, s0 = mk(0.0, 0.0);
+        cdbl s1 = mk(1.0 - 2.0 * kEuler, 0.0);
+        double h = 0.0;
+        for (int k = 1; k < 24; ++k) {
+            term = term * t * (1.0 / double(k * k));
+            u = u * t * (1.0 / double(k * (k + 1)));
+            h += 1.0 / k;
+            a = a + term;
+            b = b + u;
+            s0 = s0 + h * term;
+            s1 = s1 + (2.0 * h + 1.0 / (k + 1) - 2.0 * kEuler) * u;
+        }
+        j0 = a;
+        j1 = 0.5 * b;
+        c0 = kTwoOverPi * (kEuler * a - s0);
+        c1 = (-0.5 * kOneOverPi) * s1;
+        return;
+    }
+    const cdbl zi = recip(z);
+    int n = 2 * ((int)(0.5 * cabsd(z)) + 16 + (int)(2.0 * cbrt(cabsd(z))) * 2);
+    cdbl hi = mk(0.0, 0.0), lo = mk(1e-60, 0.0), sum = mk(0.0, 0.0);   // J_{n+1}, J_n
+    for (; n > 0; --n) {
+        // (-i)^n = 1, -i, -1, i for n mod 4 = 0 .. 3
+        const int m = n & 3;
+        sum = sum + (m == 0 ? lo : (m == 1 ? mk(lo.y, -lo.x) : (m == 2 ? mk(-lo.x, -lo.y) : mk(-lo.y, lo.x))));
+        const cdbl nx = (2.0 * n) * (zi * lo) - hi;
+        hi = lo;
+        lo = nx;
+    }
+    const cdbl w = mk(z.y, -z.x);                        // -iz
+    const cdbl sc = cdiv(cexpd(w), lo + 2.0 * sum);
+    j0 = sc * lo;
+    const cdbl J1 = sc * hi;
+    j1 = J1 * zi;
+    cdbl h0, h1;
+    hankel01_cplx(z, h0, h1);
+    const cdbl y0 = mk(h0.y - j0.y, j0.x - h0.x), y1 = mk(h1.y - J1.y, J1.x - h1.x);   // -i (H - J)
+    const cdbl L2 = kTwoOverPi * clogd(0.5 * z);
+    c0 = y0 - L2 * j0;
+    c1 = zi * (y1 - L2 * J1 + kTwoOverPi * zi);
 }
 
 // ---------------------------------------------------------------------------

@@ -36,14 +36,6 @@ struct AsmParams {
     long long npairs_total;      // N (N + 1) / 2
     cdbl* out;                   // nchunk == 1: local matrices [npairs_total][16 (D+1)][nk];
                                  // else partials [nent][nchunk][16 (D+1)][nk]
-    // several scatterers in one launch (paired-lane kernel only): entry e
-    // belongs to instance i = einst[e], whose nk slots are kap/kr/cv[i nk ..]
-    // and whose node table igeo[i] holds entry e at position e - ibase[i];
-    // pidx is then the pair's index in the concatenation of the instances'
-    // pair lists.  einst null: one instance.
-    const int* einst;
-    const double* const* igeo;
-    const long long* ibase;
     int ns, nc;                  // Gauss / composite rule sizes
     int qflags;                  // HBEM_FLAG_* quirk bits
     // paired-lane kernel only: the slots come in blocks of 32 (nk a multiple
@@ -51,9 +43,8 @@ struct AsmParams {
     // refraction index and block 2w + 1 the same ones with the outer; out
     // receives per wavenumber the differences T is formed from (K_i - K_o,
     // W_o - W_i, V_o - V_i) with nkt (the wavenumbers) in place of nk in the
-    // layouts above; kt0: the first wavenumber of the launch's slots in those
-    // layouts (a launch over a range of slot blocks)
-    int tdiff, nkt, kt0;
+    // layouts above
+    int tdiff, nkt;
 };
 
 // assembly (hbem_assembly.hip)
@@ -66,19 +57,80 @@ void launch_setup_singular(int cls, const int* ent, int nent, const double* pane
 void launch_assemble(int cls, int D, const AsmParams& P, int G, hipStream_t st);
 void launch_chunk_sum(const cdbl* part, int nent, int nchunk, int nk, int nslot, const long long* pidx, long long npairs,
                       cdbl* L, hipStream_t st);
-// L: local matrices [pair][slot][wavenumber] of nk wavenumber slots
-void launch_gather_layers(const cdbl* L, int nk, int nslot, int q, int N, int D, int layers, cdbl* K, cdbl* W,
-                          cdbl* V, hipStream_t st);
-// T_t for output b is written at T[t] + b * ld^2 (t = 0..D) with leading
-// dimension ld (0: 2N); qo null: L is in the tdiff layout (AsmParams) and
-// output b reads wavenumber qi[b] of it; T32 (may be null): T_0 again in
-// FP32, each entry rounded to nearest
-void launch_form_T(const cdbl* L, int nk, int nslot, const int* qi, const int* qo, int nb, int N, int D,
-                   const double* M, cdbl* T0, cdbl* T1, cdbl* T2, hipStream_t st, int ld = 0, cflt* T32 = nullptr);
 // identity in rows and columns n..ld-1 of nb matrices of order ld
 void launch_pad_identity(cdbl* T, int n, int ld, int nb, hipStream_t st);
-// A_o = [[-K_o + M/2, V_o], [W_o, K_o^T + M/2]] of wavenumber slot o (2N x 2N)
-void launch_form_Ao(const cdbl* L, int nk, int nslot, int o, int N, const double* M, cdbl* A, hipStream_t st);
+
+// radial functionals (hbem_radial.hip)
+constexpr int kBandMaxP = 200;   // most points of a band (320 bytes of LDS each while its tables are built)
+constexpr int kRecValues = 5;    // values of a record and order (6 with the quirk)
+// A distance band: its interval is [c - a, c + a] (near band, band 0: [0, a]);
+// p points, their basis at record offset `basis`, the weights (2 - delta_q0) / p
+// T_q(s_j) of their transform at costab + cos, [j][q], their radii at costab + rad.
+struct Band {
+    double c, a;
+    int p, basis, cos, rad;
+};
+// A tile of 16 pairs of hats of one band; its coefficients at table offset off.
+struct BandTile {
+    long long off;
+    int band, pad;
+};
+// A pair of hats of the near band and its panel pairs (P, Q), P = m - 1 + (i & 1),
+// Q = n - 1 + (i >> 1): class (0 coinciding, 1 adjacent, 3 general) + 4 x the
+// singular pair's index in its class.
+struct RadialNear {
+    int m, n, type[4];
+};
+// Wavenumber slots of a call: kap (kapi: imaginary parts, or null), kr (kri),
+// cv per slot; a group of ncolg columns cols[], column c using slot c (inner)
+// and, for differences, slot c + nslot2 (outer).  Records go to out, ncol
+// columns wide; basis: scratch for the group.
+struct RadialParams {
+    const double *kap, *kapi, *kr, *kri, *cv;
+    const int* cols;
+    int ncolg, nslot2, ncol, nv, nbasis;   // nbasis: basis records of all bands
+    cdbl* basis;
+    cdbl* out;
+};
+int band_order(double c, double a, double kmax, double tol, bool near);
+void launch_radial_band(const double* gtab, int N, int ns, int npairs, double R, double first, double step,
+                        unsigned short* band, hipStream_t st);
+void launch_radial_flags(const double* gtab, int ns, int npairs, unsigned char* flags, hipStream_t st);
+void launch_radial_far(const int* recs, const BandTile* tiles, int tile0, int ntile, const Band* bands, int pmax,
+                       const double* gtab, const double* xg, const double* wg, int N, int ns, const unsigned char* flags,
+                       const double* costab, double* tab, hipStream_t st);
+// moments of the cnt singular pairs of class cls: mom [pair][half][p][34], ext
+// [pair][half][8], two halves for adjacent pairs
+void launch_radial_moments(int cls, const int* ent, int cnt, const double* panels, const double* coefs, const double* xc,
+                           const double* wc, int nc, double R, int p, double* mom, double* ext, hipStream_t st);
+constexpr int kRadialMoments = 34;
+void launch_radial_near(const RadialNear* ent, int nent, const BandTile* tiles, const Band* bands, int p,
+                        const double* gtab, const double* xg, const double* wg, int N, int ns, const unsigned char* flags,
+                        const double* mom_c, const double* ext_c, const double* mom_a, const double* ext_a,
+                        const double* costab, double* tab, double* ext, hipStream_t st);
+// basis of all bands (at most pmax points each) for the group
+void launch_band_basis(const RadialParams& P, bool diff, const Band* bands, int nbands, int pmax, const double* costab,
+                       hipStream_t st);
+// records of the tiles tile0 .. tile0 + ntile - 1 (near: band 0's) for the group
+void launch_band_eval(int D, bool diff, bool near, const RadialParams& P, const int* recs, const BandTile* tiles, int tile0,
+                      int ntile, const Band* bands, const double* costab, const double* tab, const double* ext,
+                      hipStream_t st);
+// records of all pairs from local matrices L [panel pair][16 (D+1)][lcols];
+// lout > 0: differences of L's columns i and lout + i
+void launch_records_from_locals(const cdbl* L, int lcols, int D, int lout, int npairs, const int* cols, int ncolg, int N,
+                                cdbl* out, int ncol, int nv, hipStream_t st);
+// Consumers of records E, ncol columns wide, nv values per order.
+void launch_gather_layers(const cdbl* E, int ncol, int nv, int q, int N, int D, int layers, cdbl* K, cdbl* W, cdbl* V,
+                          hipStream_t st);
+// T_t for output b is written at T[t] + b * ld^2 (t = 0..D) with leading
+// dimension ld (0: 2N), from columns of differences (qo < 0: output b is
+// column b), or one output from the slot columns qi and qo; T32 (may be
+// null): T_0 again in FP32, each entry rounded to nearest; only0: records of
+// orders 0..D, only T_0 is formed
+void launch_form_T(const cdbl* E, int ncol, int nv, int qi, int qo, int nb, int N, int D, const double* M, cdbl* T0, cdbl* T1,
+                   cdbl* T2, hipStream_t st, int ld = 0, cflt* T32 = nullptr, bool only0 = false);
+// A_o = [[-K_o + M/2, V_o], [W_o, K_o^T + M/2]] of column o (2N x 2N)
+void launch_form_Ao(const cdbl* E, int ncol, int o, int N, const double* M, cdbl* A, hipStream_t st);
 
 // dense (hbem_dense.hip); all batched over `batch` matrices of order n with
 // stride n*n (column-major, lda = n) unless noted.

@@ -56,19 +56,16 @@ extern "C" {
  * entries).  Off by default: the default is the symmetric copy of the same
  * derivative order, which is what the k-derivative of V requires. */
 #define HBEM_FLAG_QUIRK_SLP_COINC_DER 1
-/* Lower-order quadrature on separated panel pairs.  Every assembly through the
- * context at real positive wavenumbers (matrices, T, sweeps) integrates the
- * general pairs of line and arc panels whose bounding discs lie at least one
- * panel diameter apart with a tensor Gauss rule of 5-10 points a side instead
- * of the quadrature order, the order chosen from the separation class (one to
- * two diameters, two to eight, eight to sixteen, more) and kappa times the
- * largest panel diameter -- per block of 32 wavenumbers in the sweeps, per
- * batch otherwise -- so that each pair's local matrices stay within 1e-13 of
- * their largest entry of the 11-point rule's.  Pairs on trigonometric-curve
- * or spline panels, complex wavenumbers, and kappa d > 5 keep the full rule.
- * Off by default: the reference integrates every general pair with the same
- * rule (galerkin_builder.cpp:308-327).  Not accepted by
- * hbem_sigma_sweep_multi. */
+/* Separated panel pairs to 5e-14 instead of rounding.  On meshes of line and
+ * arc panels only, every assembly through the context (matrices, T, sweeps)
+ * interpolates the kernels of separated pairs over their distance bands with
+ * as many points as keep them within 5e-14 of the largest value on the band
+ * (1e-16 without the flag), for the wavenumbers with kappa times the largest
+ * panel diameter up to 5.  Pairs closer than ten panel diameters, meshes with
+ * trigonometric-curve or spline panels, wavenumbers the bands do not serve and
+ * kappa d > 5 are those of the plain context.  Off by default: the reference
+ * integrates every general pair with the same rule (galerkin_builder.cpp:
+ * 308-327).  Not accepted by hbem_sigma_sweep_multi. */
 #define HBEM_FLAG_FAR_FIELD 2
 
 typedef struct hbem_geometry* hbem_geometry_t;
@@ -256,8 +253,8 @@ int hbem_sigma_sweep_der2(hbem_geometry_t g, const double* ks, int nk, double c_
  * be NULL) is set to 1; so is it when the refinement of an earlier solve does
  * not contract (its last correction above half the one before it, or above
  * half the unrefined solution after one step).  The assembly stays FP64 (on
- * a context created with HBEM_FLAG_FAR_FIELD, with its lower-order rules on
- * separated pairs).  No counterpart in the reference, which factorises in
+ * a context created with HBEM_FLAG_FAR_FIELD, with its tolerance on separated
+ * pairs).  No counterpart in the reference, which factorises in
  * FP64 only.
  */
 int hbem_sigma_sweep_mixed(hbem_geometry_t g, const double* ks, int nk, double c_o, double c_i, const void* R, int nc,
@@ -271,11 +268,11 @@ int hbem_sigma_sweep_mixed(hbem_geometry_t g, const double* ks, int nk, double c
  * wavenumbers ks[i nk .. i nk + nk - 1] with inner index c_i[i], outer c_o
  * and test matrix R[i] (2 N_i x nc, host); sigma[i nk + j] receives the
  * result.  The instances are grouped by their order 2 N_i rounded up to a
- * multiple of `bucket` (a multiple of 32; 0 = 256): every panel-pair class of
- * a group is one assembly launch, and the group's T matrices, padded with the
- * identity to the common order, are one batched LU and randomized SVD.  The
+ * multiple of `bucket` (a multiple of 32; 0 = 256): a group's T matrices,
+ * padded with the identity to the common order, are one batched LU and
+ * randomized SVD, its device phase replayed from a captured graph.  The
  * padding leaves every result equal bit for bit to hbem_sigma_sweep of the
- * instance alone (nk >= 32, whose sweep uses the same assembly kernel).
+ * instance alone.
  */
 int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double* ks, int nk, double c_o,
                            const double* c_i, const void* const* R, int nc, int q, int bucket, double* sigma);
@@ -284,22 +281,26 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
  * roofline figures.  enable != 0 clears and starts recording; the events are
  * only read by query (no host synchronisation inside the timed calls).  query
  * returns the accumulated milliseconds and launch count of phase `which`
- * (0 = general-pair assembly kernel, 1 = adjacent-pair kernel, 2 =
- * coinciding-pair kernel, 3 = LU factorisation, 4 = T formation, 5 = the
- * randomized SVD stage after the LU, 6 = the LU's matrix-core launches, its
- * trailing and sub-panel updates) and the algorithmic flop count (slots 0-2:
- * the frozen FP64 model of the assembly; 3: 8 n^3 / 3 per matrix; 6: the 3M
- * products' 6 m n k per update and matrix, in the precision of the
- * factorisation; 0 where none is defined). */
+ * (0 = general-pair assembly: the band products, or the node loops' general
+ * kernel where a wavenumber takes them; 1 = adjacent-pair kernel, 2 =
+ * coinciding-pair kernel, both of the node loops only; 3 = LU factorisation,
+ * 4 = T formation, 5 = the randomized SVD stage after the LU, 6 = the LU's
+ * matrix-core launches, its trailing and sub-panel updates) and the
+ * algorithmic flop count (0: 2 x 5 (d + 1) x 2 per band point, pair of hat
+ * functions and wavenumber slot for the band products; 0-2: the frozen FP64
+ * model for the node loops; 3: 8 n^3 / 3 per matrix; 6: the 3M products'
+ * 6 m n k per update and matrix, in the precision of the factorisation; 0
+ * where none is defined). */
 int hbem_profile_enable(hbem_geometry_t g, int enable);
 int hbem_profile_query(hbem_geometry_t g, int which, double* ms, long long* launches, double* flops);
 
-/* Wavenumbers per batch that hbem_sigma_sweep uses for a closed curve of
- * npanels panels at Gauss order `order`, derivative order d and nc random
- * columns when avail_bytes of device memory are usable and nk wavenumbers are
- * requested (at most 256, batches balanced; nk >= 32 real positive k use the
- * T-difference layout, half the local-matrix bytes).  Host-only: no device
- * is used.
+/* A lower estimate of the wavenumbers per batch that hbem_sigma_sweep takes for
+ * a closed curve of npanels panels at Gauss order `order`, derivative order d
+ * and nc random columns when avail_bytes of device memory are usable and nk
+ * wavenumbers are requested (at most 256, batches balanced).  It prices local
+ * matrices of 16 (d + 1) values per panel pair, which only the wavenumbers of
+ * the node loops need; the sweeps' records take a third of that, so a sweep's
+ * own batches are at least as large.  Host-only: no device is used.
  * (No counterpart in the reference, whose sweep runs one k per thread.) */
 int hbem_sweep_batch_size(int npanels, int order, int d, int nc, unsigned long long avail_bytes, int nk, int* B);
 
