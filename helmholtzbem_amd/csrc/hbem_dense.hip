@@ -182,130 +182,185 @@ __device__ __forceinline__ void row_map(const int* ip, int j0, int jb, int* src,
 // the factorisation runs): src[64], erow[32], nes.
 constexpr int kRowMapInts = 97;
 
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(const F& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<N, I + 1>(f);
+    }
+}
+
+// max of a non-negative or -1 value over a wavefront (W = 64, result in every
+// lane) or over its first sixteen lanes (W = 16), by DPP moves: the LDS shuffles
+// of a butterfly would cost ~5 times the latency
+template <int CTRL, int MASK>
+__device__ __forceinline__ double dpp_max(double x) {
+    const unsigned long long b = __double_as_longlong(x);
+    const unsigned lo = __builtin_amdgcn_update_dpp((int)b, (int)b, CTRL, MASK, 0xf, false);
+    const unsigned hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), CTRL, MASK, 0xf, false);
+    return fmax(x, __longlong_as_double(((unsigned long long)hi << 32) | lo));
+}
+template <int W>
+__device__ __forceinline__ double wave_max(double x) {
+    x = dpp_max<0x111, 0xf>(x);               // row_shr:1, 2, 4, 8: lane 15 of a row of 16 has its maximum
+    x = dpp_max<0x112, 0xf>(x);
+    x = dpp_max<0x114, 0xf>(x);
+    x = dpp_max<0x118, 0xf>(x);
+    if (W == 64) {
+        x = dpp_max<0x142, 0xa>(x);           // row_bcast:15, row_bcast:31
+        x = dpp_max<0x143, 0xc>(x);
+    }
+    const unsigned long long b = __double_as_longlong(x);
+    const unsigned lo = __builtin_amdgcn_readlane((int)b, W - 1), hi = __builtin_amdgcn_readlane((int)(b >> 32), W - 1);
+    return __longlong_as_double(((unsigned long long)hi << 32) | lo);
+}
+// the smallest index among the lanes that hold the maximum, and its lane
+__device__ __forceinline__ int first_index(unsigned long long mask, int index, int& lane) {
+    int p = 0x7fffffff;
+    lane = 0;
+    while (mask) {
+        const int l = __ffsll(mask) - 1, q = __builtin_amdgcn_readlane(index, l);
+        if (q < p) { p = q; lane = l; }
+        mask &= mask - 1;
+    }
+    return p;
+}
+
 // The same panel factorisation with the rows held in registers, CW panel
-// columns (a chunk) at a time, for panels of at most 1024 R rows: thread t owns
-// rows j0 + t + 1024 u, u < R.  Inside a chunk every column step -- pivot
-// search, exchange of the two rows' chunk values through LDS, scaling, rank-1
-// update -- works on registers; the interchange of the other panel columns
-// goes to memory, one thread per column.  After the chunk, its rows are
-// stored, U12 = L11^{-1} A12 is solved for the panel columns right of it (one
-// thread per column) and those columns receive A22 -= L21 U12 in one pass.
-// The panel is read and written about jb / CW + 1 times instead of once per
-// column step.  R x CW complex values stay in registers (at most 32 of the
-// 128 VGPRs a thread of a 1024-thread workgroup has).
-template <class C, int R, int CW>
-__global__ __launch_bounds__(1024) void k_lu_panel_rg(C* __restrict__ A, int n, int j0, int jb,
-                                                      int* __restrict__ ipiv, int* __restrict__ rmap) {
-    constexpr int YB = R >= 2 ? 4 : 8;           // trailing columns updated per round
+// columns (a chunk) at a time, for panels of at most TH R rows: thread t owns
+// rows j0 + t + blockDim.x u, u < R.  Rows do not move while the panel is
+// factorised: a thread keeps its rows' values and their current positions pos,
+// and an interchange only changes two positions.  A column step is the search
+// (each wavefront's candidate by DPP, handed over with its row's values of the
+// chunk through LDS, then the candidates in every wavefront: one barrier), the
+// scaling and the rank-1 update in registers.  After a chunk, its values are
+// stored to the rows' own places, U12 = L11^{-1} A12 is solved for the panel
+// columns right of it (one thread per column) and those columns receive A22 -=
+// L21 U12 in one pass; at the end the rows that changed place are moved.  A panel
+// that is one chunk (CW = 32) is read once and written once, in place.
+//
+// The column step's latency bounds it, not its 1 / CW reads of the panel.  With
+// the interchanges of the panel's other columns going to memory in every step and
+// three barriers a step, a panel of 32 columns took ## us.
+template <class C, int R, int CW, int TH>
+__global__ __launch_bounds__(TH) void k_lu_panel_rg(C* __restrict__ A, int n, int j0, int jb,
+                                                    int* __restrict__ ipiv, int* __restrict__ rmap) {
+    constexpr int YB = R >= 4 ? 1 : 2;   // trailing columns updated per round
+    constexpr int NW = TH / 64;
+    constexpr bool WHOLE = CW == 32;
     C* a = A + (size_t)blockIdx.x * n * n;
     int* ip = ipiv + (size_t)blockIdx.x * n;
-    __shared__ double sv[16];
-    __shared__ int si[16];
-    __shared__ int spiv;
-    __shared__ C prow[CW];                   // pivot row (chunk columns)
-    __shared__ C xrow[CW];                   // the row it displaces
-    __shared__ C L11[CW][CW];
-    __shared__ C U12[CW][32];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    int rowu[R];
+    __shared__ double sv[2][NW];
+    __shared__ int sp[2][NW];
+    __shared__ C cand[2][NW][CW];            // the wavefronts' candidate rows
+    __shared__ int spiv[32];
+    __shared__ C L11[WHOLE ? 1 : CW][CW];
+    __shared__ C U12[WHOLE ? 1 : CW][32];
+    __shared__ int srow[CW];                 // rows of the chunk's pivots
+    __shared__ int nmove, mfrom[64], mto[64];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
+    int rowu[R], pos[R];
 #pragma unroll
-    for (int u = 0; u < R; ++u) rowu[u] = j0 + tid + 1024 * u;
+    for (int u = 0; u < R; ++u) {
+        rowu[u] = j0 + tid + (int)blockDim.x * u;
+        pos[u] = rowu[u] < n ? rowu[u] : -1;  // -1: no row
+    }
+    if (tid == 0) nmove = 0;
     for (int c0 = 0; c0 < jb; c0 += CW) {
-        const int w = min(CW, jb - c0);
+        const int w = min(CW, jb - c0);          // below CW for the last chunk only
         const int cb = j0 + c0;                  // first column of the chunk = its first diagonal row
+        // (loads take clamped, in-range addresses so that they issue together; what
+        // lies outside the range is zero and never stored)
         C v[R][CW];
 #pragma unroll
         for (int u = 0; u < R; ++u) {
-            const bool own = rowu[u] < n && rowu[u] >= cb;
+            const bool own = pos[u] >= cb;
 #pragma unroll
-            for (int e = 0; e < CW; ++e) v[u][e] = (own && e < w) ? a[rowu[u] + (size_t)(cb + e) * n] : C{};
+            for (int e = 0; e < CW; ++e) {
+                const C t = a[min(rowu[u], n - 1) + (size_t)(cb + min(e, w - 1)) * n];
+                v[u][e] = own && e < w ? t : C{};
+            }
         }
-#pragma unroll
-        for (int c = 0; c < CW; ++c) {
-            if (c >= w) break;
-            const int col = cb + c;
+        // (unrolled by hand: the compiler gives up on sixteen and more columns and
+        // would keep the rows in scratch memory)
+        static_for<CW>([&](auto step) {
+            constexpr int c = decltype(step)::value;
+            if (c >= w) return;
+            const int col = cb + c, par = c & 1;
             double best = -1.0;
             int bi = n;
-            // rows ascending within a thread: strict > keeps the first index on ties
+            // largest |a|^2, smallest position on ties
 #pragma unroll
             for (int u = 0; u < R; ++u)
-                if (rowu[u] < n && rowu[u] >= col) {
+                if (pos[u] >= col) {
                     const double x = cabs2(v[u][c]);
-                    if (x > best) { best = x; bi = rowu[u]; }
+                    if (x > best || (x == best && pos[u] < bi)) { best = x; bi = pos[u]; }
                 }
+            double mx = wave_max<64>(best);
+            int l, piv = n;
+            if (mx >= 0.0) {
+                piv = first_index(__ballot(best == mx), bi, l);
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const double v2 = __shfl_xor(best, o, 64);
-                const int i2 = __shfl_xor(bi, o, 64);
-                if (v2 > best || (v2 == best && i2 < bi)) { best = v2; bi = i2; }
-            }
-            if (lane == 0) { sv[wv] = best; si[wv] = bi; }
-            __syncthreads();
-            if (tid < 64) {
-                best = lane < 16 ? sv[lane] : -1.0;
-                bi = lane < 16 ? si[lane] : n;
+                for (int u = 0; u < R; ++u)
+                    if (pos[u] == piv) {
 #pragma unroll
-                for (int o = 8; o > 0; o >>= 1) {
-                    const double v2 = __shfl_xor(best, o, 64);
-                    const int i2 = __shfl_xor(bi, o, 64);
-                    if (v2 > best || (v2 == best && i2 < bi)) { best = v2; bi = i2; }
-                }
-                // no candidate (a column of NaNs): keep the row, never index past n
-                if (tid == 0) { const int pv = bi < n ? bi : col; spiv = pv; ip[col] = pv; }
-            }
-            __syncthreads();
-            const int piv = spiv;
-#pragma unroll
-            for (int u = 0; u < R; ++u) {
-                if (rowu[u] == piv) {
-#pragma unroll
-                    for (int e = 0; e < CW; ++e) prow[e] = v[u][e];
-                }
-                if (rowu[u] == col) {
-#pragma unroll
-                    for (int e = 0; e < CW; ++e) xrow[e] = v[u][e];
-                }
-            }
-            if (piv != col && tid < jb && (tid < c0 || tid >= c0 + w)) {
-                C* pc = a + (size_t)(j0 + tid) * n;
-                const C t = pc[piv];
-                pc[piv] = pc[col];
-                pc[col] = t;
-            }
-            __syncthreads();
-            if (piv != col) {
-#pragma unroll
-                for (int u = 0; u < R; ++u) {
-                    if (rowu[u] == piv) {
-#pragma unroll
-                        for (int e = 0; e < CW; ++e) v[u][e] = xrow[e];
-                    } else if (rowu[u] == col) {
-#pragma unroll
-                        for (int e = 0; e < CW; ++e) v[u][e] = prow[e];
+                        for (int e = c; e < CW; ++e) cand[par][wv][e] = v[u][e];
                     }
-                }
             }
+            if (lane == 0) { sv[par][wv] = mx; sp[par][wv] = piv; }
+            __syncthreads();
+            best = lane < nw ? sv[par][lane] : -1.0;
+            bi = lane < nw ? sp[par][lane] : n;
+            mx = wave_max<16>(best);
+            piv = first_index(__ballot(lane < nw && best == mx), bi, l);
+            if (!(mx >= 0.0)) {
+                // no candidate (a column of NaNs): keep the row, never index past n
+                piv = col;
+                l = 0;
+#pragma unroll
+                for (int u = 0; u < R; ++u)
+                    if (pos[u] == col) {
+#pragma unroll
+                        for (int e = c; e < CW; ++e) cand[par][0][e] = v[u][e];
+                    }
+                __syncthreads();
+            }
+            if (tid == 0) spiv[c0 + c] = piv;
+            const C* prow = cand[par][l];
             const C d = prow[c];
             const C inv = (d.x == 0.0 && d.y == 0.0) ? C{} : crecip(d);
 #pragma unroll
-            for (int u = 0; u < R; ++u)
-                if (rowu[u] < n && rowu[u] > col) {
-                    const C l = cmulx(v[u][c], inv);
-                    v[u][c] = l;
+            for (int u = 0; u < R; ++u) {
+                pos[u] = pos[u] == piv ? col : (pos[u] == col ? piv : pos[u]);
+                if (pos[u] > col) {
+                    const C m = cmulx(v[u][c], inv);
+                    v[u][c] = m;
 #pragma unroll
-                    for (int e = c + 1; e < CW; ++e)
-                        if (e < w) cfms(v[u][e], l, prow[e]);
+                    for (int e = c + 1; e < CW; ++e) cfms(v[u][e], m, prow[e]);
                 }
+            }
+        });
+        if (WHOLE) {
+            __syncthreads();                     // every row has been read
+#pragma unroll
+            for (int u = 0; u < R; ++u)
+                if (pos[u] >= cb) {
+#pragma unroll
+                    for (int e = 0; e < CW; ++e)
+                        if (e < w) a[pos[u] + (size_t)(cb + e) * n] = v[u][e];
+                }
+            break;
         }
         // chunk rows back to memory; L11 of the chunk for the U12 solve
 #pragma unroll
         for (int u = 0; u < R; ++u) {
-            if (rowu[u] < n && rowu[u] >= cb) {
+            if (pos[u] >= cb) {
 #pragma unroll
                 for (int e = 0; e < CW; ++e)
                     if (e < w) a[rowu[u] + (size_t)(cb + e) * n] = v[u][e];
-                const int r = rowu[u] - cb;
+                const int r = pos[u] - cb;
                 if (r < w) {
+                    srow[r] = rowu[u];
 #pragma unroll
                     for (int e = 0; e < CW; ++e) L11[r][e] = v[u][e];
                 }
@@ -314,55 +369,72 @@ __global__ __launch_bounds__(1024) void k_lu_panel_rg(C* __restrict__ A, int n, 
         const int rem = jb - c0 - w;             // panel columns right of the chunk
         if (rem <= 0) break;
         __syncthreads();
-        // (loads below take clamped, in-range addresses so that they issue
-        // together; what lies outside the range is never used or stored)
         if (tid < rem) {
-            C* pc = a + (size_t)(cb + w + tid) * n + cb;
+            C* pc = a + (size_t)(cb + w + tid) * n;
             C x[CW];
 #pragma unroll
-            for (int r = 0; r < CW; ++r) x[r] = pc[min(r, w - 1)];
+            for (int r = 0; r < CW; ++r) x[r] = pc[srow[r]];
 #pragma unroll
             for (int r = 0; r < CW; ++r) {
-                if (r < w) {
+                pc[srow[r]] = x[r];
+                U12[r][tid] = x[r];
 #pragma unroll
-                    for (int e = 0; e < CW; ++e)
-                        if (e < r) cfms(x[r], L11[r][e], x[e]);
-                    pc[r] = x[r];
-                    U12[r][tid] = x[r];
-                }
+                for (int q = r + 1; q < CW; ++q) cfms(x[q], L11[q][r], x[r]);
             }
         }
         __syncthreads();
+        for (int cc0 = 0; cc0 < rem; cc0 += YB) {
+            C y[R][YB];
 #pragma unroll
-        for (int u = 0; u < R; ++u) {
-            const int row = rowu[u];
-            if (row >= n) break;                 // rows ascend with u
-            const bool upd = row >= cb + w;
-            for (int cc0 = 0; cc0 < rem; cc0 += YB) {
-                C y[YB];
+            for (int u = 0; u < R; ++u)
 #pragma unroll
-                for (int e = 0; e < YB; ++e) y[e] = a[row + (size_t)(cb + w + min(cc0 + e, rem - 1)) * n];
+                for (int e = 0; e < YB; ++e)
+                    y[u][e] = a[min(rowu[u], n - 1) + (size_t)(cb + w + min(cc0 + e, rem - 1)) * n];
 #pragma unroll
-                for (int e = 0; e < YB; ++e) {
-                    if (cc0 + e < rem) {
+            for (int e = 0; e < YB; ++e) {
+                if (cc0 + e < rem) {
 #pragma unroll
-                        for (int f = 0; f < CW; ++f)
-                            if (f < w) cfms(y[e], v[u][f], U12[f][cc0 + e]);
-                        if (upd) a[row + (size_t)(cb + w + cc0 + e) * n] = y[e];
+                    for (int f = 0; f < CW; ++f) {
+                        const C b = U12[f][cc0 + e];
+#pragma unroll
+                        for (int u = 0; u < R; ++u) cfms(y[u][e], v[u][f], b);
                     }
+#pragma unroll
+                    for (int u = 0; u < R; ++u)
+                        if (pos[u] >= cb + w) a[rowu[u] + (size_t)(cb + w + cc0 + e) * n] = y[u][e];
                 }
             }
         }
+    }
+    if (!WHOLE) {
+        // rows that changed place: at most two per interchange
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+            if (pos[u] != rowu[u] && pos[u] >= 0) {
+                const int k = atomicAdd(&nmove, 1);
+                mfrom[k] = rowu[u];
+                mto[k] = pos[u];
+            }
+        __syncthreads();
+        // eight threads a row, four columns each
+        const int k = tid >> 3;
+        const bool mv = k < nmove;
+        C t[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            t[e] = mv ? a[mfrom[k] + (size_t)(j0 + min((tid & 7) + 8 * e, jb - 1)) * n] : C{};
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (mv && (tid & 7) + 8 * e < jb) a[mto[k] + (size_t)(j0 + (tid & 7) + 8 * e) * n] = t[e];
+    } else {
         __syncthreads();
     }
-    // the interchange map for the row kernels (the pivots are in ip; every
-    // thread has passed a barrier since the last was written)
-    if (rmap) {
-        __syncthreads();
-        if (wv == 0) {
-            int* m = rmap + (size_t)blockIdx.x * n;
-            row_map(ip, j0, jb, m, m + 64, m + 96);
-        }
+    if (tid < jb) ip[j0 + tid] = spiv[tid];
+    // the interchange map for the row kernels
+    if (rmap && wv == 0) {
+        int* m = rmap + (size_t)blockIdx.x * n;
+        row_map(spiv - j0, j0, jb, m, m + 64, m + 96);
     }
 }
 
@@ -804,9 +876,12 @@ static void lu_factor_impl(C* A, int n, int batch, int* ipiv, int* perm, hipStre
         constexpr bool f32 = sizeof(C) == sizeof(cflt);   // half the registers per value: wider chunks
         int* m = n >= kRowMapInts ? perm : nullptr;
         rmap = rows <= 4096 ? m : nullptr;
-        if (rows <= 1024) hipLaunchKernelGGL((k_lu_panel_rg<C, 1, 8>), g, t, 0, st, A, n, j, jb, ipiv, m);
-        else if (rows <= 2048) hipLaunchKernelGGL((k_lu_panel_rg<C, 2, f32 ? 8 : 6>), g, t, 0, st, A, n, j, jb, ipiv, m);
-        else if (rows <= 4096) hipLaunchKernelGGL((k_lu_panel_rg<C, 4, f32 ? 8 : 4>), g, t, 0, st, A, n, j, jb, ipiv, m);
+        // as many columns at a time as 256 registers a thread hold
+        const dim3 tr((rows + 63) / 64 * 64), t5(512);
+        if (rows <= 512) hipLaunchKernelGGL((k_lu_panel_rg<C, 1, 32, 512>), g, tr, 0, st, A, n, j, jb, ipiv, m);
+        else if (rows <= 1024) hipLaunchKernelGGL((k_lu_panel_rg<C, 2, f32 ? 32 : 16, 512>), g, t5, 0, st, A, n, j, jb, ipiv, m);
+        else if (rows <= 2048) hipLaunchKernelGGL((k_lu_panel_rg<C, 4, f32 ? 16 : 8, 512>), g, t5, 0, st, A, n, j, jb, ipiv, m);
+        else if (rows <= 4096) hipLaunchKernelGGL((k_lu_panel_rg<C, 8, f32 ? 8 : 4, 512>), g, t5, 0, st, A, n, j, jb, ipiv, m);
         else hipLaunchKernelGGL((k_lu_panel<C>), g, t, 0, st, A, n, j, jb, ipiv);
     };
     for (int j0 = 0; j0 < n; j0 += S * sb) {
