@@ -557,6 +557,31 @@ __global__ __launch_bounds__(256) void k_radial_near(const RadialNear* __restric
 // doubles r_j and kappa r_j leave out of the argument enters by the derivatives
 // (A&S 9.1.27-28), as a phase kappa r of 100 rounded to 64 bits would put 1e-14 on
 // every pair of the band.
+// The four polynomials of horner4 by the compensated Horner scheme (Graillat,
+// Langlois and Louvet: each step's rounding errors, by fma and TwoSum, in a second
+// Horner recurrence).  Up to x = 8 the terms grow to 100 and cancel: plain Horner's
+// error of 1e-14 changes from point to point of a band, where the node loops
+// averaged it over a pair's nodes (V of the 400-panel star 2.9e-15 from theirs, 1e-16
+// at x > 8).
+template <int DEG>
+__device__ __forceinline__ void horner4_comp(ctab_ptr c, double z, double (&v)[4]) {
+#pragma clang fp contract(off)
+    double e[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int f = 0; f < 4; ++f) v[f] = c[4 * DEG + f];
+    for (int i = DEG - 1; i >= 0; --i) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            const double a = c[4 * i + f], p = v[f] * z, pe = fma(v[f], z, -p);
+            const double s = p + a, t = s - p, se = (p - (s - t)) + (a - t);
+            e[f] = fma(e[f], z, pe + se);
+            v[f] = s;
+        }
+    }
+#pragma unroll
+    for (int f = 0; f < 4; ++f) v[f] += e[f];
+}
+
 __global__ __launch_bounds__(256) void k_band_basis(RadialParams P, const Band* __restrict__ bands,
                                                     const double* __restrict__ costab, int nslots) {
     const int b = blockIdx.y;
@@ -595,31 +620,40 @@ __global__ __launch_bounds__(256) void k_band_basis(RadialParams P, const Band* 
         ol[nslots] = mk(-b1.y, b1.x);
         return;
     }
-    const double kap = P.kap[q], x = kap * r, y = x * x * (1.0 / 64.0), d = fma(kap, r, -x) + kap * dr;
-    if (b > 0) {
-        double j0, y0, j1, y1;
-        const double xi = 1.0 / x;
-        bessel_jy01_f<0>(x, y, kTwoOverPi * log(0.5 * x), xi, 1.0 / sqrt(kPi * x), j0, y0, j1, y1);
-        o[0] = mk(fma(-d, j1, j0), fma(-d, y1, y0));
-        o[nslots] = mk(fma(d, fma(-j1, xi, j0), j1), fma(d, fma(-y1, xi, y0), y1));
-        return;
-    }
+    const double kap = P.kap[q], x = kap * r, d = fma(kap, r, -x) + kap * dr, xi = 1.0 / x;
     double A, B, C, Dd;                        // J0 = A, J1 = x B, entire parts C of Y0 and x Dd of Y1
     if (x < 8.0) {
-        horner4<HBEM_SMALL_DEG>(bessel_table() + HBEM_TAB_SMALL, y, A, B, C, Dd);
+        // polynomials in y = x^2 / 64, whose rounding is one more residual of the
+        // argument: (x^2 - fl(x^2)) / (2 x)
+        const double x2 = x * x, t = (d + 0.5 * fma(x, x, -x2) * xi) * xi;
+        double v[4];
+        horner4_comp<HBEM_SMALL_DEG>(bessel_table() + HBEM_TAB_SMALL, x2 * (1.0 / 64.0), v);
+        A = fma(-x2 * t, v[1], v[0]);
+        B = fma(t, fma(-2.0, v[1], v[0]), v[1]);
+        C = fma(kTwoOverPi * t, 1.0 - v[0], fma(-x2 * t, v[3], v[2]));
+        Dd = fma(t, v[2] - 2.0 * v[3] - kTwoOverPi * v[1], v[3]);
+        if (b > 0) {
+            const double L2 = kTwoOverPi * fma(d, xi, log(0.5 * x)), xd = x + d, J1 = xd * B;
+            o[0] = mk(A, fma(L2, A, C));
+            o[nslots] = mk(J1, fma(L2, J1, fma(xd, Dd, -kTwoOverPi * fma(-d * xi, xi, xi))));
+            return;
+        }
     } else {
-        double y0, j1, y1;
-        const double L2 = kTwoOverPi * log(0.5 * x), xi = 1.0 / x;
-        bessel_jy01_f<0>(x, y, L2, xi, 1.0 / sqrt(kPi * x), A, y0, j1, y1);
-        C = fma(-L2, A, y0);
-        B = j1 * xi;
-        Dd = (fma(-L2, j1, y1) + kTwoOverPi * xi) * xi;
+        double j0, y0, j1, y1;
+        bessel_jy01_f<0>(x, 0.0, 0.0, xi, 1.0 / sqrt(kPi * x), j0, y0, j1, y1);
+        const double J0 = fma(-d, j1, j0), Y0 = fma(-d, y1, y0);
+        const double J1 = fma(d, fma(-j1, xi, j0), j1), Y1 = fma(d, fma(-y1, xi, y0), y1);
+        if (b > 0) {
+            o[0] = mk(J0, Y0);
+            o[nslots] = mk(J1, Y1);
+            return;
+        }
+        const double L2 = kTwoOverPi * fma(d, xi, log(0.5 * x)), xr = fma(-d * xi, xi, xi);
+        A = J0;
+        C = fma(-L2, J0, Y0);
+        B = J1 * xr;
+        Dd = (fma(-L2, J1, Y1) + kTwoOverPi * xr) * xr;
     }
-    const double t = d / x, a0 = A, b0 = B, c0 = C;
-    A = fma(-x * d, b0, A);
-    B = fma(t, fma(-2.0, b0, a0), B);
-    C = fma(kTwoOverPi * t, 1.0 - a0, fma(-x * d, Dd, C));
-    Dd = fma(t, c0 - 2.0 * Dd - kTwoOverPi * b0, Dd);
     const double lR = kTwoOverPi * log(0.5 * (kap * bd.a));
     o[0] = mk(A, fma(lR, A, C));
     o[nslots] = mk(kap * B, kap * fma(lR, B, Dd));
