@@ -11,6 +11,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -18,7 +19,7 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libhbem.so")
 ARCH = os.environ.get("HBEM_OFFLOAD_ARCH", "gfx950")
 
-HIP_SOURCES = ["hbem_assembly.hip", "hbem_radial.hip", "hbem_dense.hip", "hbem_capi.hip"]
+HIP_SOURCES = ["hbem_assembly.hip", "hbem_radial.hip", "hbem_dense.hip", "hbem_solve.hip", "hbem_capi.hip"]
 HOST_SOURCES = ["hbem_setup.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -38,17 +39,15 @@ def _run(cmd):
 
 def build(verbose: bool = False) -> str:
     os.makedirs(BUILD, exist_ok=True)
-    objs = []
-    for src in HOST_SOURCES:
-        obj = os.path.join(BUILD, src + ".o")
-        _run(["g++"] + HOST_FLAGS + ["-c", os.path.join(CSRC, src), "-o", obj])
-        objs.append(obj)
-    for src in HIP_SOURCES:
-        obj = os.path.join(BUILD, src + ".o")
-        out = _run([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, src), "-o", obj])
-        if verbose and out.strip():
-            print(out)
-        objs.append(obj)
+    cmds = [["g++"] + HOST_FLAGS + ["-c", os.path.join(CSRC, src), "-o", os.path.join(BUILD, src + ".o")]
+            for src in HOST_SOURCES]
+    cmds += [[HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, src), "-o", os.path.join(BUILD, src + ".o")]
+             for src in HIP_SOURCES]
+    with ThreadPoolExecutor(len(cmds)) as pool:
+        for out in pool.map(_run, cmds):
+            if verbose and out.strip():
+                print(out)
+    objs = [c[-1] for c in cmds]
     tmp = LIB + ".tmp"
     _run([HIPCC, "-shared", "-fPIC", "--offload-arch=" + ARCH, "-o", tmp] + objs)
     os.replace(tmp, LIB)

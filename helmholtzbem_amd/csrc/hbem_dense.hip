@@ -7,67 +7,15 @@
 //     32-column sub-panels; panel factorisation by one workgroup per matrix
 //     with the panel rows in registers, row interchanges, triangular solve of
 //     the U12 block, trailing update by a complex GEMM on the FP64 matrix cores;
-//   * lu.solve / lu.adjoint().solve on thin right-hand sides (n x nc), reading
-//     the factors in place: blocked substitution, the 64 x 64 diagonal blocks
-//     by one wavefront with cross-lane broadcasts, the off-diagonal updates by
-//     the whole workgroup;
+//   * (lu.solve / lu.adjoint().solve on thin right-hand sides: hbem_solve.hip;)
 //   * the projection factor's thin products in compressed-row form;
 //   * HouseholderQR's role (an orthonormal basis of the span): modified
 //     Gram-Schmidt applied twice;
 //   * JacobiSVD's role (largest singular value of the thin n x nc matrix):
 //     Gram matrix plus a Hermitian Jacobi eigensolver on one lane.
-#include "hbem_internal.hpp"
+#include "hbem_complex.hpp"
 
 namespace hbem {
-
-// Reciprocal and product with every multiply-add an explicit fma: the LU's
-// arithmetic per matrix entry is then fixed by the source, whichever kernel
-// instantiation (rows per thread, chunk width) performs it, so a matrix
-// factorised inside a larger zero-padded one gives the same bits.
-__device__ __forceinline__ cdbl crecip(cdbl d) {
-    const double s = 1.0 / fma(d.x, d.x, d.y * d.y);
-    return mk(d.x * s, -d.y * s);
-}
-__device__ __forceinline__ cdbl cmulx(cdbl a, cdbl b) { return mk(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x)); }
-__device__ __forceinline__ void cfms(cdbl& acc, cdbl a, cdbl b) {   // acc -= a * b
-    acc.x = fma(-a.x, b.x, fma(a.y, b.y, acc.x));
-    acc.y = fma(-a.x, b.y, fma(-a.y, b.x, acc.y));
-}
-__device__ __forceinline__ void cfma(cdbl& acc, cdbl a, cdbl b) {   // acc += a * b
-    acc.x = fma(a.x, b.x, fma(-a.y, b.y, acc.x));
-    acc.y = fma(a.x, b.y, fma(a.y, b.x, acc.y));
-}
-__device__ __forceinline__ cdbl shfl_c(cdbl v, int src) {
-    return mk(__shfl(v.x, src, 64), __shfl(v.y, src, 64));
-}
-// lane src's value in every lane, src the same for the whole wavefront:
-// v_readlane through a scalar register, no LDS round trip
-__device__ __forceinline__ double bcast_lane(double v, int src) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
-    return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ cdbl bcast_lane(cdbl v, int src) { return mk(bcast_lane(v.x, src), bcast_lane(v.y, src)); }
-
-// The same operations on single-precision complex values (the factors of the
-// mixed-precision LU).
-__device__ __forceinline__ float cabs2(cflt a) { return a.x * a.x + a.y * a.y; }
-__device__ __forceinline__ cflt operator*(cflt a, cflt b) { return cflt{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
-__device__ __forceinline__ cflt crecip(cflt d) {
-    const float s = 1.0f / fmaf(d.x, d.x, d.y * d.y);
-    return cflt{d.x * s, -d.y * s};
-}
-__device__ __forceinline__ cflt cmulx(cflt a, cflt b) {
-    return cflt{fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x)};
-}
-__device__ __forceinline__ void cfms(cflt& acc, cflt a, cflt b) {   // acc -= a * b
-    acc.x = fmaf(-a.x, b.x, fmaf(a.y, b.y, acc.x));
-    acc.y = fmaf(-a.x, b.y, fmaf(-a.y, b.x, acc.y));
-}
-__device__ __forceinline__ cflt shfl_c(cflt v, int src) { return cflt{__shfl(v.x, src, 64), __shfl(v.y, src, 64)}; }
-// widening load of a factor entry for double-precision arithmetic
-__device__ __forceinline__ cdbl to_cdbl(cdbl v) { return v; }
-__device__ __forceinline__ cdbl to_cdbl(cflt v) { return mk((double)v.x, (double)v.y); }
 
 // ---------------------------------------------------------------------------
 // LU with partial pivoting
@@ -181,14 +129,6 @@ __device__ __forceinline__ void row_map(const int* ip, int j0, int jb, int* src,
 // Map layout in memory (the caller's perm array doubles as its store while
 // the factorisation runs): src[64], erow[32], nes.
 constexpr int kRowMapInts = 97;
-
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void static_for(const F& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<N, I + 1>(f);
-    }
-}
 
 // max of a non-negative or -1 value over a wavefront (W = 64, result in every
 // lane) or over its first sixteen lanes (W = 16), by DPP moves: the LDS shuffles
@@ -918,630 +858,6 @@ void lu_factor_batched(cdbl* A, int n, int batch, int* ipiv, int* perm, hipStrea
 
 void lu_factor_batched_f32(cflt* A, int n, int batch, int* ipiv, int* perm, hipStream_t st, LaunchTimer* gemm) {
     lu_factor_impl(A, n, batch, ipiv, perm, st, gemm);
-}
-
-// ---------------------------------------------------------------------------
-// Thin triangular solves
-// ---------------------------------------------------------------------------
-// A = P^T L U with L (unit lower) and U in one column-major array LU.  All four
-// substitutions read LU in place, always down its columns:
-//   A x = b:    L y = P b forward, U x = y backward -- right-looking: once the
-//               block's unknowns are known, columns of L (below) / U (above)
-//               update the other rows;
-//   A^H x = b:  U^H y = b forward, L^H z = y backward, x = P^T z -- left-
-//               looking: (U^H y)_i = sum_j conj(U(j, i)) y_j runs down column
-//               i of U above the diagonal (of L below it for L^H), so each
-//               block first gathers its rows' sums from the finished unknowns.
-// Blocks of 64 rows; the diagonal block is staged in LDS (as the operator of
-// the pass) and solved by wavefront 0 with cross-lane broadcasts, while the
-// other wavefronts stage the next block.
-constexpr int kMaxNc = 8;
-constexpr int kSolveThreads = 1024;
-constexpr int kTS = 65;   // padded row stride of the 64 x 64 LDS diagonal block
-
-struct SolveLds {
-    cdbl tile[2][64 * kTS];   // the current diagonal block and the next one
-    cdbl xb[64 * kMaxNc];     // solution of the last block
-};
-
-// Stage the diagonal block [r0, r0 + bs)^2 of the pass operator with threads
-// t0, t0 + stride, ...: conj = false: op(i, j) = LU(i, j); conj = true:
-// op(i, j) = conj(LU(j, i)).
-template <class F>
-__device__ __forceinline__ void stage_diag(const F* M, int n, int r0, int bs, bool conj, cdbl* tile, int t0,
-                                           int stride) {
-    for (int e = t0; e < 64 * 64; e += stride) {
-        const int p = e & 63, q = e >> 6;   // p runs down a column of LU
-        const bool in = p < bs && q < bs;
-        const cdbl v = in ? to_cdbl(M[(r0 + p) + (size_t)(r0 + q) * n]) : mk(0, 0);
-        if (conj) tile[q * kTS + p] = cconj(v);
-        else tile[p * kTS + q] = v;
-    }
-}
-
-// Wavefront 0: solve the staged block for w[r0, r0 + bs) in place and leave
-// the solution in xb (zero beyond bs).  With a non-unit diagonal the block is
-// solved as (M D^-1) y = w, x = D^-1 y: the reciprocal pivots are formed by
-// all lanes at once and scale the tile entries as they are read, eight steps
-// ahead, and x = D^-1 y is formed at the end, so a step's dependence chain is
-// one broadcast (v_readlane: the step's lane is the same for the whole
-// wavefront) and one complex multiply-add.  Every complex product is written
-// as explicit FMAs, so the bits do not depend on how the compiler contracts
-// the code around each call site.
-template <int NC>
-__device__ __forceinline__ void diag_solve(int n, int r0, int bs, bool lower, bool unit, cdbl* w,
-                                           const cdbl* __restrict__ tile, cdbl* xb) {
-    const int lane = threadIdx.x & 63;
-    cdbl x[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) x[c] = lane < bs ? w[r0 + lane + (size_t)c * n] : mk(0, 0);
-    const cdbl dv = tile[lane * kTS + lane];
-    const cdbl dinv = (unit || lane >= bs) ? mk(1, 0) : crecip(dv);
-    for (int s0 = 0; s0 < bs; s0 += 8) {
-        cdbl lv[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int step = min(s0 + u, bs - 1);
-            const int j = lower ? step : bs - 1 - step;
-            lv[u] = tile[lane * kTS + j];
-            if (!unit) lv[u] = cmulx(lv[u], bcast_lane(dinv, j));
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int step = s0 + u;
-            if (step >= bs) break;
-            const int j = lower ? step : bs - 1 - step;
-            const bool other = lower ? (lane > j && lane < bs) : (lane < j);
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const cdbl xj = bcast_lane(x[c], j);
-                if (other) cfms(x[c], lv[u], xj);
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        if (!unit) x[c] = cmulx(x[c], dinv);
-        if (lane < bs) w[r0 + lane + (size_t)c * n] = x[c];
-        xb[lane * kMaxNc + c] = lane < bs ? x[c] : mk(0, 0);
-    }
-}
-
-// Right-looking pass with the column-major factor: L (lower, unit) forward or
-// U (upper) backward, over the rows [pb, pe) (the whole matrix, or one panel
-// of the panelled form).  After block b, the rows of the range outside it
-// (below / above) take w_i -= sum_j M(i, r0 + j) x_j: a wavefront covers RW
-// rows x 64 / RW groups
-// of columns (lane = row + RW group), each thread loading its columns in
-// batches of eight.  RW = 16 for FP64 factors, 32 for FP32 ones, so that a
-// load instruction reads runs of 256 bytes down the columns either way.
-template <int NC, class F, int RWT = 0>
-__device__ __forceinline__ void subst_right(const F* M, int n, bool lower, cdbl* w, SolveLds& S, int pb, int pe) {
-    // rows per wavefront, columns per group (RWT: chosen by the caller)
-    constexpr int RW = RWT ? RWT : (sizeof(F) == sizeof(cflt) ? 32 : 16), CW = RW;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
-    const int l16 = lane % RW, grp = lane / RW;
-    const int nblk = (pe - pb + 63) / 64;
-    auto rb = [&](int s) { return pb + 64 * (lower ? s : nblk - 1 - s); };   // first row of the s-th block solved
-    auto bsz = [&](int s) { return min(64, pe - rb(s)); };
-    stage_diag(M, n, rb(0), bsz(0), false, S.tile[0], tid, blockDim.x);
-    for (int s = 0; s < nblk; ++s) {
-        const int r0 = rb(s), bs = bsz(s);
-        __syncthreads();                          // block s staged, block s - 1's update done
-        if (wv == 0) {
-            diag_solve<NC>(n, r0, bs, lower, lower, w, S.tile[s & 1], S.xb);
-        } else if (s + 1 < nblk) {
-            stage_diag(M, n, rb(s + 1), bsz(s + 1), false, S.tile[(s + 1) & 1], tid - 64, blockDim.x - 64);
-        }
-        __syncthreads();
-        const int ia = lower ? r0 + bs : pb, ib = lower ? pe : r0;
-        for (int i0 = ia + RW * wv; i0 < ib; i0 += RW * nwv) {
-            const int i = i0 + l16;
-            cdbl acc[NC];
-#pragma unroll
-            for (int c = 0; c < NC; ++c) acc[c] = mk(0, 0);
-            {
-                // eight loads at a time from clamped (in-range) addresses, values
-                // beyond the block zeroed afterwards: no branch between the loads
-                const int ic = min(i, ib - 1);
-#pragma unroll 1
-                for (int u0 = 0; u0 < CW; u0 += 8) {
-                    F t[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        t[u] = M[ic + (size_t)(r0 + min(CW * grp + u0 + u, bs - 1)) * n];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        const int j = CW * grp + u0 + u;
-                        const cdbl tv = j < bs ? to_cdbl(t[u]) : mk(0, 0);
-#pragma unroll
-                        for (int c = 0; c < NC; ++c) cfma(acc[c], tv, S.xb[j * kMaxNc + c]);
-                    }
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < NC; ++c)
-#pragma unroll
-                for (int o = RW; o < 64; o <<= 1) {
-                    acc[c].x += __shfl_xor(acc[c].x, o, 64);
-                    acc[c].y += __shfl_xor(acc[c].y, o, 64);
-                }
-            if (grp == 0 && i < ib) {
-#pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    cdbl& y = w[i + (size_t)c * n];
-                    y = y - acc[c];
-                }
-            }
-        }
-    }
-    __syncthreads();
-}
-
-// Left-looking pass with the conjugate transpose of the factor: U^H (lower)
-// forward or L^H (upper, unit) backward, over the rows [pb, pe).  Block b
-// first takes w_i -= sum_j conj(M(j, i)) w_j over the finished unknowns j of
-// the range (above the block for U^H, below it for L^H; those outside the
-// range are gathered beforehand): wavefront v sums columns i = r0 + 4 v .. + 3
-// (CP of them per sweep down the column, CP = 4 / 2 / 1 for up to 2 / 4 / 8
-// right-hand sides) with its lanes down the column, then the diagonal block is
-// solved.
-template <int NC, class F, int TW = 1>
-__device__ __forceinline__ void subst_left(const F* M, int n, bool lower, cdbl* w, SolveLds& S, int pb, int pe) {
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int nblk = (pe - pb + 63) / 64;
-    auto rb = [&](int s) { return pb + 64 * (lower ? s : nblk - 1 - s); };
-    auto bsz = [&](int s) { return min(64, pe - rb(s)); };
-    stage_diag(M, n, rb(0), bsz(0), true, S.tile[0], tid, blockDim.x);
-    for (int s = 0; s < nblk; ++s) {
-        const int r0 = rb(s), bs = bsz(s);
-        const int ja = lower ? pb : r0 + bs, jb = lower ? r0 : pe;
-        constexpr int CP = NC <= 2 ? 4 : (NC <= 4 ? 2 : 1);
-        for (int q0 = 0; q0 < 4; q0 += CP) {
-            if (4 * wv + q0 >= bs) break;        // wave-uniform
-            const int i0 = r0 + 4 * wv + q0;
-            cdbl acc[CP][NC];
-#pragma unroll
-            for (int q = 0; q < CP; ++q)
-#pragma unroll
-                for (int c = 0; c < NC; ++c) acc[q][c] = mk(0, 0);
-            // the same number of sweeps for every lane, TW sweeps' loads in
-            // flight at once, at clamped addresses (values beyond the range
-            // replaced by zero afterwards; sweeps past the last add zeros)
-            const int T = (jb - ja + 63) >> 6;
-            const int qmax = bs - 1 - 4 * wv - q0;    // last column of the block for this wavefront
-            for (int tt = 0; tt < T; tt += TW) {
-                cdbl xj[TW][NC];
-                F mv[TW][CP];
-#pragma unroll
-                for (int h = 0; h < TW; ++h) {
-                    const int jc = min(ja + lane + 64 * (tt + h), jb - 1);
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) xj[h][c] = w[jc + (size_t)c * n];
-#pragma unroll
-                    for (int q = 0; q < CP; ++q) mv[h][q] = M[jc + (size_t)(i0 + min(q, qmax)) * n];
-                }
-#pragma unroll
-                for (int h = 0; h < TW; ++h) {
-                    const bool in = ja + lane + 64 * (tt + h) < jb;
-#pragma unroll
-                    for (int c = 0; c < NC; ++c)
-                        if (!in) xj[h][c] = mk(0, 0);
-#pragma unroll
-                    for (int q = 0; q < CP; ++q) {
-                        const cdbl t = q <= qmax ? cconj(to_cdbl(mv[h][q])) : mk(0, 0);
-#pragma unroll
-                        for (int c = 0; c < NC; ++c) cfma(acc[q][c], t, xj[h][c]);
-                    }
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < CP; ++q)
-#pragma unroll
-                for (int c = 0; c < NC; ++c)
-#pragma unroll
-                    for (int o = 32; o > 0; o >>= 1) {
-                        acc[q][c].x += __shfl_xor(acc[q][c].x, o, 64);
-                        acc[q][c].y += __shfl_xor(acc[q][c].y, o, 64);
-                    }
-            // lane q stores column i0 + q (register arrays are indexed with constants)
-#pragma unroll
-            for (int q = 0; q < CP; ++q)
-                if (lane == q && 4 * wv + q0 + q < bs) {
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) {
-                        cdbl& y = w[i0 + q + (size_t)c * n];
-                        y = y - acc[q][c];
-                    }
-                }
-        }
-        __syncthreads();                          // sums in, block s staged
-        if (wv == 0) {
-            diag_solve<NC>(n, r0, bs, lower, !lower, w, S.tile[s & 1], S.xb);
-        } else if (s + 1 < nblk) {
-            stage_diag(M, n, rb(s + 1), bsz(s + 1), true, S.tile[(s + 1) & 1], tid - 64, blockDim.x - 64);
-        }
-        __syncthreads();
-    }
-}
-
-// one workgroup of kSolveThreads threads per matrix
-template <class F, int NC>
-__global__ __launch_bounds__(kSolveThreads) void k_solve_thin(const F* __restrict__ LU, long long ms,
-                                                              const int* __restrict__ perm, int n,
-                                                              cdbl* __restrict__ X, int adj, cdbl* __restrict__ work) {
-    __shared__ SolveLds S;
-    const int b = blockIdx.x;
-    const int* p = perm + (size_t)b * n;
-    cdbl* x = X + (size_t)b * n * NC;
-    cdbl* w = work + (size_t)b * n * NC;
-    const F* lu = LU + (size_t)b * ms;
-    const int tid = threadIdx.x;
-    if (!adj) {
-        // A = P^T L U:  w = P x, L y = w, U z = y
-        for (int e = tid; e < n * NC; e += blockDim.x) {
-            const int i = e % n, c = e / n;
-            w[e] = x[p[i] + (size_t)c * n];
-        }
-        __syncthreads();
-        subst_right<NC>(lu, n, true, w, S, 0, n);
-        subst_right<NC>(lu, n, false, w, S, 0, n);
-        for (int e = tid; e < n * NC; e += blockDim.x) x[e] = w[e];
-    } else {
-        // A^H = U^H L^H P:  U^H y = x, L^H z = y, x = P^T z
-        for (int e = tid; e < n * NC; e += blockDim.x) w[e] = x[e];
-        __syncthreads();
-        subst_left<NC>(lu, n, true, w, S, 0, n);
-        subst_left<NC>(lu, n, false, w, S, 0, n);
-        for (int e = tid; e < n * NC; e += blockDim.x) {
-            const int i = e % n, c = e / n;
-            x[p[i] + (size_t)c * n] = w[e];
-        }
-    }
-}
-
-// Panelled form of the thin solves for orders above 2 kSolvePanel: the
-// passes run panel by panel of kSolvePanel rows.  A panel's triangle is solved
-// by one workgroup per matrix (k_solve_panel: the blocked substitution above,
-// restricted to the panel); the panel's coupling to the other rows runs on
-// many workgroups per matrix: a right-looking pass then updates every row
-// after the panel with the panel's columns (k_panel_update), a left-looking
-// pass first gathers into the panel's rows the sums over the unknowns finished
-// before it (k_panel_gather).  Each entry of the factors is still read once,
-// but the bulk of the reads no longer waits on one workgroup per matrix.
-constexpr int kSolvePanel = 512;
-
-// w = P x (A x = b) or w = x (A^H x = b)
-__global__ void k_thin_in(const int* __restrict__ perm, int n, int nc, const cdbl* __restrict__ X, int adj,
-                          cdbl* __restrict__ work) {
-    const int b = blockIdx.y;
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (long long)n * nc) return;
-    const int i = (int)(e % n), c = (int)(e / n);
-    const cdbl* x = X + (size_t)b * n * nc;
-    work[(size_t)b * n * nc + e] = adj ? x[e] : x[perm[(size_t)b * n + i] + (size_t)c * n];
-}
-
-// x = w (A x = b) or x = P^T w (A^H x = b)
-__global__ void k_thin_out(const int* __restrict__ perm, int n, int nc, cdbl* __restrict__ X, int adj,
-                           const cdbl* __restrict__ work) {
-    const int b = blockIdx.y;
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (long long)n * nc) return;
-    const int i = (int)(e % n), c = (int)(e / n);
-    cdbl* x = X + (size_t)b * n * nc;
-    const cdbl v = work[(size_t)b * n * nc + e];
-    if (adj) x[perm[(size_t)b * n + i] + (size_t)c * n] = v;
-    else x[e] = v;
-}
-
-// one workgroup of kSolveThreads threads per matrix: pass 0 (L, or U^H) or
-// pass 1 (U, or L^H) over the panel [pb, pe)
-// Right-looking coupling of the unknowns [cb, ce) (one panel, staged in xs)
-// onto row i: w_i -= sum_j M(i, j) w_j, the sum in column order.  A thread per
-// row (consecutive rows: the loads run down the columns), LR column loads in
-// flight.
-template <int NC>
-__device__ __forceinline__ void stage_unknowns(const cdbl* w, int n, int cb, int ce, cdbl* xs) {
-    const int pw = ce - cb;
-    for (int e = threadIdx.x; e < pw * NC; e += blockDim.x) {
-        const int j = e % pw, c = e / pw;
-        xs[j * NC + c] = w[cb + j + (size_t)c * n];
-    }
-}
-template <class F, int NC>
-__device__ __forceinline__ void couple_right_row(const F* M, int n, cdbl* w, int cb, int ce, int i, const cdbl* xs) {
-    constexpr int LR = sizeof(F) == sizeof(cflt) ? 16 : 8;
-    const int pw = ce - cb;
-    cdbl acc[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = mk(0, 0);
-    const F* mr = M + i + (size_t)cb * n;
-    for (int j0 = 0; j0 < pw; j0 += LR) {
-        F t[LR];
-#pragma unroll
-        for (int u = 0; u < LR; ++u) t[u] = mr[(size_t)min(j0 + u, pw - 1) * n];
-#pragma unroll
-        for (int u = 0; u < LR; ++u) {
-            if (j0 + u < pw) {
-                const cdbl tv = to_cdbl(t[u]);
-#pragma unroll
-                for (int c = 0; c < NC; ++c) cfma(acc[c], tv, xs[(j0 + u) * NC + c]);
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        cdbl& y = w[i + (size_t)c * n];
-        y = y - acc[c];
-    }
-}
-
-// Left-looking coupling of the unknowns [ja, jb) onto rows i0 .. i0 + 3 (those
-// below re): w_i -= sum_j conj(M(j, i)) w_j.  One wavefront, lanes down the
-// columns (lane j mod 64: ja is a multiple of 64), two sweeps' loads in
-// flight; the lane sums are reduced by shuffles in a fixed order.
-template <class F, int NC>
-__device__ __forceinline__ void couple_left_quad(const F* M, int n, cdbl* w, int ja, int jb, int i0, int re) {
-    const int lane = threadIdx.x & 63;
-    const int qmax = min(4, re - i0) - 1;
-    cdbl acc[4][NC];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) acc[q][c] = mk(0, 0);
-    const int T = (jb - ja + 63) >> 6;
-    for (int tt = 0; tt < T; tt += 2) {
-        cdbl xj[2][NC];
-        F mv[2][4];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int jc = min(ja + lane + 64 * (tt + h), jb - 1);
-#pragma unroll
-            for (int c = 0; c < NC; ++c) xj[h][c] = w[jc + (size_t)c * n];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) mv[h][q] = M[jc + (size_t)(i0 + min(q, qmax)) * n];
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const bool in = ja + lane + 64 * (tt + h) < jb;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const cdbl t = (in && q <= qmax) ? cconj(to_cdbl(mv[h][q])) : mk(0, 0);
-#pragma unroll
-                for (int c = 0; c < NC; ++c) cfma(acc[q][c], t, xj[h][c]);
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                acc[q][c].x += __shfl_xor(acc[q][c].x, o, 64);
-                acc[q][c].y += __shfl_xor(acc[q][c].y, o, 64);
-            }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        if (lane == q && q <= qmax) {
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                cdbl& y = w[i0 + q + (size_t)c * n];
-                y = y - acc[q][c];
-            }
-        }
-}
-
-// One panel [pb, pe) of a pass, blocks 0 .. batch - 1 (one per matrix), and
-// beside it, in blocks batch + cwg b + k, a coupling that does not touch the
-// panel: the unknowns [cb, ce) onto the rows [rb, re) of matrix b,
-// right-looking (a thread per row, 1024 rows a block) or, for adj, left-looking
-// (a wavefront per four rows, 64 rows a block).  The coupling blocks take the
-// CUs the batch's panel solves leave idle.  Up to kFuseNc right-hand sides:
-// with more, the left-looking sums do not fit the registers of a
-// 1024-thread block, and the couplings run as launches of their own.
-constexpr int kFuseNc = 3;
-template <class F, int NC>
-__global__ __launch_bounds__(kSolveThreads) void k_solve_panel(const F* __restrict__ LU, long long ms, int n, int pass,
-                                                               int adj, cdbl* __restrict__ work, int pb, int pe,
-                                                               int batch, int cwg, int cb, int ce, int rb, int re) {
-    __shared__ SolveLds S;
-    if ((int)blockIdx.x < batch) {
-        const int b = blockIdx.x;
-        cdbl* w = work + (size_t)b * n * NC;
-        const F* lu = LU + (size_t)b * ms;
-        // inside a panel the updates cover at most kSolvePanel - 64 rows: 16 rows
-        // per wavefront (more wavefronts busy, fewer load rounds each) and two
-        // sweeps' loads in flight in the left-looking sums
-        if (!adj) subst_right<NC, F, 16>(lu, n, pass == 0, w, S, pb, pe);
-        else subst_left<NC, F, NC <= 4 ? 2 : 1>(lu, n, pass == 0, w, S, pb, pe);
-        return;
-    }
-    if constexpr (NC <= kFuseNc) {
-        const int q = blockIdx.x - batch, b = q / cwg, k = q - b * cwg;
-        cdbl* w = work + (size_t)b * n * NC;
-        const F* M = LU + (size_t)b * ms;
-        if (!adj) {
-            cdbl* xs = reinterpret_cast<cdbl*>(&S);   // the panel solve's LDS is not used by this block
-            stage_unknowns<NC>(w, n, cb, ce, xs);
-            __syncthreads();
-            const int i = rb + k * blockDim.x + threadIdx.x;
-            if (i < re) couple_right_row<F, NC>(M, n, w, cb, ce, i, xs);
-        } else {
-            const int i0 = rb + (k * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 4;
-            if (i0 < re) couple_left_quad<F, NC>(M, n, w, cb, ce, i0, re);
-        }
-    }
-}
-
-// The same couplings on their own.  Right-looking, 64 rows a block: wavefront
-// v sums the unknowns cb + 128 v .. + 127 for the block's rows (lane = row,
-// so the loads still run down the columns in 64-row segments), and the four
-// partial sums are added in a fixed order, ((0 + 1) + (2 + 3)), by wavefront 0:
-// each thread's chain of dependent load rounds is a quarter as long as with
-// one thread per row over the whole panel.  The quarters are fixed column
-// ranges from the panel's start, so a panel padded with zero columns gives the
-// same sums.
-template <class F, int NC>
-__global__ __launch_bounds__(256) void k_panel_update(const F* __restrict__ LU, long long ms, int n,
-                                                      cdbl* __restrict__ work, int cb, int ce, int rb, int re) {
-    constexpr int LR = sizeof(F) == sizeof(cflt) ? 16 : 8;
-    constexpr int QW = kSolvePanel / 4;
-    __shared__ cdbl xs[kSolvePanel * NC];
-    __shared__ cdbl part[4][64][NC];
-    const int b = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    cdbl* w = work + (size_t)b * n * NC;
-    stage_unknowns<NC>(w, n, cb, ce, xs);
-    __syncthreads();
-    const int i = rb + blockIdx.x * 64 + lane;
-    const int q0 = wv * QW, q1 = min(ce - cb, q0 + QW);
-    cdbl acc[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = mk(0, 0);
-    if (i < re) {
-        const F* mr = LU + (size_t)b * ms + i + (size_t)cb * n;
-        for (int j0 = q0; j0 < q1; j0 += LR) {
-            F t[LR];
-#pragma unroll
-            for (int u = 0; u < LR; ++u) t[u] = mr[(size_t)min(j0 + u, q1 - 1) * n];
-#pragma unroll
-            for (int u = 0; u < LR; ++u) {
-                if (j0 + u < q1) {
-                    const cdbl tv = to_cdbl(t[u]);
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) cfma(acc[c], tv, xs[(j0 + u) * NC + c]);
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < NC; ++c) part[wv][lane][c] = acc[c];
-    __syncthreads();
-    if (wv == 0 && i < re) {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            cdbl& y = w[i + (size_t)c * n];
-            y = y - ((part[0][lane][c] + part[1][lane][c]) + (part[2][lane][c] + part[3][lane][c]));
-        }
-    }
-}
-
-// Left-looking, 16 rows a block.
-template <class F, int NC>
-__global__ __launch_bounds__(256) void k_panel_gather(const F* __restrict__ LU, long long ms, int n,
-                                                      cdbl* __restrict__ work, int ja, int jb, int rb, int re) {
-    const int b = blockIdx.y;
-    const int i0 = rb + (blockIdx.x * 4 + (threadIdx.x >> 6)) * 4;
-    if (i0 >= re) return;                     // whole wavefront; no barrier in this kernel
-    couple_left_quad<F, NC>(LU + (size_t)b * ms, n, work + (size_t)b * n * NC, ja, jb, i0, re);
-}
-
-// Panelled substitution (n > 2 kSolvePanel).  A pass solves its panels in
-// order; every row must have taken the couplings of all panels solved before
-// its own, in that order.  After panel p's solve, the next panel's rows take
-// p's coupling (a small launch); the rows beyond the next panel take it in
-// the launch that solves the next panel, beside that solve.  Left-looking
-// passes (adj) gather instead: the next panel's rows take the unknowns solved
-// before p beside p's solve, then p's own unknowns.  A row's sums are split
-// only at panel boundaries and at fixed offsets inside a panel, and which
-// launch serves a row depends only on its panel, so a matrix padded at the
-// end gives the same bits.  Above
-// kFuseNc right-hand sides: each panel's coupling as a launch of its own,
-// all rows at once, after its solve (right-looking) or before it (left).
-template <class F, int NC>
-static void solve_thin_nc(const F* LU, long long ms, const int* perm, int n, int batch, cdbl* X, bool adj, cdbl* work,
-                          hipStream_t st) {
-    const int a = adj ? 1 : 0;
-    if (n <= 2 * kSolvePanel) {
-        hipLaunchKernelGGL((k_solve_thin<F, NC>), dim3(batch), dim3(kSolveThreads), 0, st, LU, ms, perm, n, X, a, work);
-        return;
-    }
-    const dim3 gio((unsigned)(((long long)n * NC + 255) / 256), (unsigned)batch);
-    hipLaunchKernelGGL(k_thin_in, gio, dim3(256), 0, st, perm, n, NC, X, a, work);
-    const int np = (n + kSolvePanel - 1) / kSolvePanel;
-    auto first = [&](int p) { return p * kSolvePanel; };
-    auto last = [&](int p) { return min(n, (p + 1) * kSolvePanel); };
-    if constexpr (NC > kFuseNc) {
-        for (int pass = 0; pass < 2; ++pass) {
-            const bool lower = pass == 0;
-            for (int t = 0; t < np; ++t) {
-                const int p = lower ? t : np - 1 - t;
-                const int pb = first(p), pe = last(p);
-                if (adj && (lower ? pb > 0 : pe < n))
-                    hipLaunchKernelGGL((k_panel_gather<F, NC>), dim3((unsigned)((pe - pb + 15) / 16), (unsigned)batch),
-                                       dim3(256), 0, st, LU, ms, n, work, lower ? 0 : pe, lower ? pb : n, pb, pe);
-                hipLaunchKernelGGL((k_solve_panel<F, NC>), dim3((unsigned)batch), dim3(kSolveThreads), 0, st, LU, ms, n,
-                                   pass, a, work, pb, pe, batch, 1, 0, 0, 0, 0);
-                const int rb = lower ? pe : 0, re = lower ? n : pb;
-                if (!adj && re > rb)
-                    hipLaunchKernelGGL((k_panel_update<F, NC>), dim3((unsigned)((re - rb + 63) / 64), (unsigned)batch),
-                                       dim3(256), 0, st, LU, ms, n, work, pb, pe, rb, re);
-            }
-        }
-        hipLaunchKernelGGL(k_thin_out, gio, dim3(256), 0, st, perm, n, NC, X, a, work);
-        return;
-    }
-    for (int pass = 0; pass < 2; ++pass) {
-        const bool lower = pass == 0;
-        for (int t = 0; t < np; ++t) {
-            const int p = lower ? t : np - 1 - t;
-            const int pb = first(p), pe = last(p);
-            const bool next = t + 1 < np;
-            const int np_ = lower ? p + 1 : p - 1;             // the next panel of the pass
-            const int nb = next ? first(np_) : 0, ne = next ? last(np_) : 0;
-            int cb = 0, ce = 0, rb = 0, re = 0;                 // the coupling beside this solve
-            if (!adj && t > 0) {
-                const int pp = lower ? p - 1 : p + 1;          // the panel solved before
-                cb = first(pp);
-                ce = last(pp);
-                rb = lower ? pe : 0;                           // the rows beyond this panel
-                re = lower ? n : pb;
-            } else if (adj && next) {
-                cb = lower ? 0 : pe;
-                ce = lower ? pb : n;
-                rb = nb;
-                re = ne;
-            }
-            const bool cpl = ce > cb && re > rb;
-            const int cwg = !cpl ? 0 : (adj ? (re - rb + 63) / 64 : (re - rb + kSolveThreads - 1) / kSolveThreads);
-            hipLaunchKernelGGL((k_solve_panel<F, NC>), dim3((unsigned)(batch + batch * cwg)), dim3(kSolveThreads), 0, st,
-                               LU, ms, n, pass, a, work, pb, pe, batch, cwg > 0 ? cwg : 1, cb, ce, rb, re);
-            if (!next) continue;
-            if (!adj)
-                hipLaunchKernelGGL((k_panel_update<F, NC>), dim3((unsigned)((ne - nb + 63) / 64), (unsigned)batch),
-                                   dim3(256), 0, st, LU, ms, n, work, pb, pe, nb, ne);
-            else
-                hipLaunchKernelGGL((k_panel_gather<F, NC>), dim3((unsigned)((ne - nb + 15) / 16), (unsigned)batch),
-                                   dim3(256), 0, st, LU, ms, n, work, pb, pe, nb, ne);
-        }
-    }
-    hipLaunchKernelGGL(k_thin_out, gio, dim3(256), 0, st, perm, n, NC, X, a, work);
-}
-
-template <class F>
-static void solve_thin_impl(const F* LU, long long ms, const int* perm, int n, int batch, cdbl* X, int nc, bool adj,
-                            cdbl* work, hipStream_t st) {
-    switch (nc) {
-    case 1: solve_thin_nc<F, 1>(LU, ms, perm, n, batch, X, adj, work, st); break;
-    case 2: solve_thin_nc<F, 2>(LU, ms, perm, n, batch, X, adj, work, st); break;
-    case 3: solve_thin_nc<F, 3>(LU, ms, perm, n, batch, X, adj, work, st); break;
-    case 4: solve_thin_nc<F, 4>(LU, ms, perm, n, batch, X, adj, work, st); break;
-    case 5: solve_thin_nc<F, 5>(LU, ms, perm, n, batch, X, adj, work, st); break;
-    case 6: solve_thin_nc<F, 6>(LU, ms, perm, n, batch, X, adj, work, st); break;
-    case 7: solve_thin_nc<F, 7>(LU, ms, perm, n, batch, X, adj, work, st); break;
-    default: solve_thin_nc<F, 8>(LU, ms, perm, n, batch, X, adj, work, st); break;
-    }
-}
-
-void lu_solve_thin_batched(const cdbl* LU, long long ms, const int* perm, int n, int batch, cdbl* X, int nc, bool adj,
-                           cdbl* work, hipStream_t st) {
-    solve_thin_impl(LU, ms, perm, n, batch, X, nc, adj, work, st);
-}
-
-void lu_solve_thin_batched_f32(const cflt* LU, long long ms, const int* perm, int n, int batch, cdbl* X, int nc,
-                               bool adj, cdbl* work, hipStream_t st) {
-    solve_thin_impl(LU, ms, perm, n, batch, X, nc, adj, work, st);
 }
 
 // ---------------------------------------------------------------------------
