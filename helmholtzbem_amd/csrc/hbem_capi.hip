@@ -92,6 +92,44 @@ struct DCsr {
     }
 };
 
+// The same rows in slices of 64 of similar length, entries [k][64] (zero-padded).
+struct DSell {
+    DBuf mem;
+    const int *rows = nullptr, *off = nullptr, *col = nullptr;
+    const double* val = nullptr;
+    void build(const std::vector<double>& A, int n, hipStream_t st) {
+        std::vector<std::vector<std::pair<int, double>>> r(n);
+        for (int j = 0; j < n; ++j)
+            for (int i = 0; i < n; ++i)
+                if (A[i + (size_t)j * n] != 0.0) r[i].emplace_back(j, A[i + (size_t)j * n]);
+        std::vector<int> ord(n), o(1, 0), c;
+        std::vector<double> v;
+        for (int i = 0; i < n; ++i) ord[i] = i;
+        std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return r[a].size() > r[b].size(); });
+        for (int s = 0; s < n; s += 64) {
+            const size_t w = r[ord[s]].size();
+            for (size_t k = 0; k < w; ++k)
+                for (int l = 0; l < 64; ++l) {
+                    // (a shorter row repeats its last column with a zero)
+                    const auto& row = r[ord[std::min(s + l, n - 1)]];
+                    const bool in = s + l < n && k < row.size();
+                    c.push_back(row.empty() ? 0 : row[std::min(k, row.size() - 1)].first);
+                    v.push_back(in ? row[k].second : 0.0);
+                }
+            o.push_back((int)c.size());
+        }
+        Packed pk;
+        const size_t a = pk.add(ord), b = pk.add(o), d = pk.add(c), e = pk.add(v);
+        char* p = (char*)mem.get(pk.bytes.size());
+        HIPC(hipMemcpyAsync(p, pk.bytes.data(), pk.bytes.size(), hipMemcpyHostToDevice, st));
+        HIPC(hipStreamSynchronize(st));       // the upload reads a host vector
+        rows = (const int*)(p + a);
+        off = (const int*)(p + b);
+        col = (const int*)(p + d);
+        val = (const double*)(p + e);
+    }
+};
+
 // Algorithmic FP64 flops per node (frozen model): Hankel node (13 geometry + 171
 // Bessel) and accumulation for P1 x P1, three layers, derivative order d.
 double flops_per_node(int d) { return 184.0 + (d == 0 ? 108.0 : d == 1 ? 192.0 : 314.0); }
@@ -324,8 +362,9 @@ struct hbem_geometry {
         const int* recs = nullptr;
         Tier tier[kTiers];
     } rad;
-    DBuf d_M, d_Finvc;
+    DBuf d_M;
     DCsr s_F, s_FT, s_FinvT, s_Finv;   // F, F^T, Finv^T and Finv of the projection
+    DSell l_Finv;                      // Finv once more, in slices
     // work space
     DBuf w_Ao, w_U, w_rhs, w_flag;
     DBuf w_Tp, w_B, w_mv, w_bpiv, w_bperm, w_bvec, w_d2;   // bordered system of sv_der2 (sweeps)
@@ -1022,9 +1061,10 @@ void project_inplace(hbem_geometry* g, cdbl* T, int count, cdbl* tmp = nullptr) 
     const int n = 2 * g->N;
     const long long s = (long long)n * n;
     if (!tmp) tmp = g->w_tmp.as<cdbl>((size_t)s * count);
-    const cdbl* Fi = (const cdbl*)g->d_Finvc.p;
-    hbem::zgemm_batched(n, n, n, hbem::mk(1, 0), Fi, n, 0, T, n, s, false, hbem::mk(0, 0), tmp, n, s, count, g->st);
-    hbem::zgemm_batched(n, n, n, hbem::mk(1, 0), tmp, n, s, Fi, n, 0, true, hbem::mk(0, 0), T, n, s, count, g->st);
+    const DCsr& F = g->s_Finv;
+    const DSell& l = g->l_Finv;
+    hbem::sparse_congruence((const int*)F.rp.p, (const int*)F.ci.p, (const double*)F.v.p, l.rows, l.off, l.col, l.val, n, T, tmp,
+                            count, g->st);
 }
 
 // The linear system of tp::direct_second_kind::A_rhs (solvers.cpp:106-131) on
@@ -1051,7 +1091,7 @@ void tp_system(hbem_geometry* g, double k_re, double k_im, double c_o, double c_
     cdbl* dU = g->w_U.as<cdbl>((size_t)n * nrhs);
     HIPC(hipMemcpyAsync(dU, U, sizeof(cdbl) * (size_t)n * nrhs, hipMemcpyHostToDevice, g->st));
     rhs = g->w_rhs.as<cdbl>((size_t)n * nrhs);
-    hbem::zgemm_batched(n, nrhs, n, hbem::mk(1, 0), Ao, n, 0, dU, n, 0, false, hbem::mk(0, 0), rhs, n, 0, 1, g->st);
+    hbem::zgemm_batched(n, nrhs, n, hbem::mk(1, 0), Ao, n, 0, dU, n, 0, hbem::mk(0, 0), rhs, n, 0, 1, g->st);
     HIPC(hipGetLastError());
 }
 
@@ -1174,9 +1214,7 @@ int hbem_geometry_create(const double* panels, int npanels, const double* coefs,
         g->s_FT.build(g->F, n, true, st);
         g->s_FinvT.build(g->Finv, n, true, st);
         g->s_Finv.build(g->Finv, n, false, st);
-        std::vector<cdbl> Fic((size_t)n * n);
-        for (size_t e = 0; e < Fic.size(); ++e) Fic[e] = hbem::mk(g->Finv[e], 0.0);
-        upload(g->d_Finvc, Fic, st);
+        g->l_Finv.build(g->Finv, n, st);
     }
     HIPC(hipStreamSynchronize(st));
     *out = g;

@@ -501,9 +501,15 @@ __global__ void k_lu_perm(int n, const int* __restrict__ ipiv, int* __restrict__
 // block.  The product is formed transposed -- first operand B^T, second A^T --
 // so element v of lane l is C(r0 + (l & 15), c0 + 4 v + (l >> 4)): sixteen
 // consecutive rows of one column per lane group, for coalesced stores.
-// Workgroup = 64 x 64 tile of C as four wavefronts of 32 x 32 (2 x 2 blocks of
-// 16 x 16); k advances in steps of 16 through LDS while the next step's tile
-// is fetched into registers.  Workgroups are dealt to the eight XCDs in turn
+// Workgroup = a tile of C as WR x WC = four wavefronts of 32 x 32 (2 x 2 blocks of
+// 16 x 16): 64 x 64, or 128 x 32 / 32 x 128 for products with a side of at most 32,
+// where a square tile multiplies half of its columns or rows by zeros (the sub-panel
+// updates of an order-4000 LU, 64 matrices: 24.5 -> 33.6 TFLOP/s down the columns, 23.4 ->
+// 30.5 along the rows); k advances in steps of 16 through LDS while the next step's
+// tile is fetched into registers.  The matrix cores are busy 76% of the time in the
+// trailing updates (k = 256, 57 TFLOP/s at 2.26 GHz); two LDS buffers with one barrier a
+// step, operands loaded one group of MFMAs ahead, and the sums Re + Im laid out in
+// LDS instead of added per use each left 52-53.  Workgroups are dealt to the eight XCDs in turn
 // (id % 8); the grid is renumbered so that each XCD gets a contiguous run of
 // (matrix, tile) indices, i.e. whole matrices, whose A and B panels then stay
 // in that XCD's L2 instead of being fetched by all eight.
@@ -526,11 +532,12 @@ __device__ __forceinline__ void grouped_tile(int t, int tm, int tn, int& tr, int
     tc = r / rows;
 }
 
-template <bool TB>
+template <int WR, int WC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_zgemm(int m, int n, int k, cdbl alpha, const cdbl* __restrict__ A, int lda,
                                                long long sa, const cdbl* __restrict__ B, int ldb, long long sb,
                                                cdbl beta, cdbl* __restrict__ C, int ldc, long long sc, int batch) {
-    const int tm = (m + 63) >> 6, tn = (n + 63) >> 6;
+    constexpr int TR = 32 * WR, TC = 32 * WC;   // tile
+    const int tm = (m + TR - 1) / TR, tn = (n + TC - 1) / TC;
     const long long total = (long long)tm * tn * batch;
     const long long per = (total + 7) >> 3;
     const long long li = (long long)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -540,14 +547,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     A += bmat * sa;
     B += bmat * sb;
     C += bmat * sc;
-    __shared__ cdbl As[16][65];
-    __shared__ cdbl Bs[16][65];
+    __shared__ cdbl As[16][TR + 1];
+    __shared__ cdbl Bs[16][TC + 1];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int l16 = lane & 15, lk = lane >> 4;
-    const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32;
+    const int wr = (wv % WR) * 32, wc = (wv / WR) * 32;
     int tr, tc;
     grouped_tile(tile, tm, tn, tr, tc);
-    const int row0 = tr * 64, col0 = tc * 64;
+    const int row0 = tr * TR, col0 = tc * TC;
+    const bool full = row0 + TR <= m && col0 + TC <= n && (k & 15) == 0;
     dbl4 p1[2][2], p2[2][2], p3[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -557,30 +565,59 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             p2[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
             p3[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
         }
-    cdbl pa[4], pb[4];
+    cdbl pa[2 * WR], pb[2 * WC];
+    // an element of the k step's A (row, k) and B (k, column) blocks
+    auto ae = [&](int u, int& r, int& kk) {
+        const int e = tid + 256 * u;
+        r = e % TR;
+        kk = e / TR;
+    };
+    auto be = [&](int u, int& cc, int& kk) {
+        const int e = tid + 256 * u;
+        kk = e & 15;
+        cc = e >> 4;
+    };
     auto fetch = [&](int kb) {
+        if (full) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u, r = e & 63, kk = e >> 6;
+            for (int u = 0; u < 2 * WR; ++u) {
+                int r, kk;
+                ae(u, r, kk);
+                pa[u] = A[(row0 + r) + (size_t)(kb + kk) * lda];
+            }
+#pragma unroll
+            for (int u = 0; u < 2 * WC; ++u) {
+                int cc, kk;
+                be(u, cc, kk);
+                pb[u] = B[(kb + kk) + (size_t)(col0 + cc) * ldb];
+            }
+            return;
+        }
+#pragma unroll
+        for (int u = 0; u < 2 * WR; ++u) {
+            int r, kk;
+            ae(u, r, kk);
             pa[u] = (row0 + r < m && kb + kk < k) ? A[(row0 + r) + (size_t)(kb + kk) * lda] : mk(0, 0);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u;
-            const int kk = TB ? (e >> 6) : (e & 15), cc = TB ? (e & 63) : (e >> 4);
-            cdbl v = mk(0, 0);
-            if (col0 + cc < n && kb + kk < k)
-                v = TB ? B[(col0 + cc) + (size_t)(kb + kk) * ldb] : B[(kb + kk) + (size_t)(col0 + cc) * ldb];
-            pb[u] = v;
+        for (int u = 0; u < 2 * WC; ++u) {
+            int cc, kk;
+            be(u, cc, kk);
+            pb[u] = (col0 + cc < n && kb + kk < k) ? B[(kb + kk) + (size_t)(col0 + cc) * ldb] : mk(0, 0);
         }
     };
     fetch(0);
     for (int kb = 0; kb < k; kb += 16) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u;
-            As[e >> 6][e & 63] = pa[u];
-            const int kk = TB ? (e >> 6) : (e & 15), cc = TB ? (e & 63) : (e >> 4);
+        for (int u = 0; u < 2 * WR; ++u) {
+            int r, kk;
+            ae(u, r, kk);
+            As[kk][r] = pa[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 2 * WC; ++u) {
+            int cc, kk;
+            be(u, cc, kk);
             Bs[kk][cc] = pb[u];
         }
         __syncthreads();
@@ -637,16 +674,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 void zgemm_batched(int m, int n, int k, cdbl alpha, const cdbl* A, int lda, long long sa, const cdbl* B, int ldb,
-                   long long sb, bool transB, cdbl beta, cdbl* C, int ldc, long long sc, int batch, hipStream_t st) {
+                   long long sb, cdbl beta, cdbl* C, int ldc, long long sc, int batch, hipStream_t st) {
     if (m <= 0 || n <= 0 || batch <= 0) return;
-    const long long total = (long long)((m + 63) / 64) * ((n + 63) / 64) * batch;
-    const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
-    if (transB)
-        hipLaunchKernelGGL(k_zgemm<true>, grid, dim3(256), 0, st, m, n, k, alpha, A, lda, sa, B, ldb, sb, beta, C, ldc, sc,
+    auto run = [&](auto tile) {
+        constexpr int WR = decltype(tile)::value, WC = 4 / WR;
+        const long long total = (long long)((m + 32 * WR - 1) / (32 * WR)) * ((n + 32 * WC - 1) / (32 * WC)) * batch;
+        const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
+        hipLaunchKernelGGL((k_zgemm<WR, WC>), grid, dim3(256), 0, st, m, n, k, alpha, A, lda, sa, B, ldb, sb, beta, C, ldc, sc,
                            batch);
-    else
-        hipLaunchKernelGGL(k_zgemm<false>, grid, dim3(256), 0, st, m, n, k, alpha, A, lda, sa, B, ldb, sb, beta, C, ldc, sc,
-                           batch);
+    };
+    // products with one side of at most 32 (the sub-panels' updates): a square tile
+    // would multiply half of its columns or rows by zeros
+    if (n <= 32 && m > 32) run(std::integral_constant<int, 4>{});
+    else if (m <= 32 && n > 32) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 2>{});
 }
 
 // C -= A B on the FP32 matrix cores for the mixed-precision LU (single-
@@ -660,10 +701,12 @@ void zgemm_batched(int m, int n, int k, cdbl alpha, const cdbl* A, int lda, long
 // D(4 (l >> 4) + v, l & 15) (the transposed product's row, i.e. C's column).
 typedef float flt4 __attribute__((ext_vector_type(4)));
 
+template <int WR, int WC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_cgemm32_sub(
     int m, int n, int k, const cflt* __restrict__ A, const cflt* __restrict__ B, cflt* __restrict__ C, int ld,
     long long sm, int batch) {
-    const int tm = (m + 63) >> 6, tn = (n + 63) >> 6;
+    constexpr int TR = 32 * WR, TC = 32 * WC;   // tile
+    const int tm = (m + TR - 1) / TR, tn = (n + TC - 1) / TC;
     const long long total = (long long)tm * tn * batch;
     const long long per = (total + 7) >> 3;
     const long long li = (long long)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -673,14 +716,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     A += bmat * sm;
     B += bmat * sm;
     C += bmat * sm;
-    __shared__ cflt As[16][65];
-    __shared__ cflt Bs[16][65];
+    __shared__ cflt As[16][TR + 1];
+    __shared__ cflt Bs[16][TC + 1];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int l16 = lane & 15, lk = lane >> 4;
-    const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32;
+    const int wr = (wv % WR) * 32, wc = (wv / WR) * 32;
     int tr, tc;
     grouped_tile(tile, tm, tn, tr, tc);
-    const int row0 = tr * 64, col0 = tc * 64;
+    const int row0 = tr * TR, col0 = tc * TC;
     flt4 p1[2][2], p2[2][2], p3[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -690,15 +733,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             p2[i][j] = flt4{0.f, 0.f, 0.f, 0.f};
             p3[i][j] = flt4{0.f, 0.f, 0.f, 0.f};
         }
-    cflt pa[4], pb[4];
+    cflt pa[2 * WR], pb[2 * WC];
     auto fetch = [&](int kb) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u, r = e & 63, kk = e >> 6;
+        for (int u = 0; u < 2 * WR; ++u) {
+            const int e = tid + 256 * u, r = e % TR, kk = e / TR;
             pa[u] = (row0 + r < m && kb + kk < k) ? A[(row0 + r) + (size_t)(kb + kk) * ld] : cflt{0.f, 0.f};
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < 2 * WC; ++u) {
             const int e = tid + 256 * u, kk = e & 15, cc = e >> 4;
             pb[u] = (col0 + cc < n && kb + kk < k) ? B[(kb + kk) + (size_t)(col0 + cc) * ld] : cflt{0.f, 0.f};
         }
@@ -706,9 +749,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     fetch(0);
     for (int kb = 0; kb < k; kb += 16) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < 2 * WR; ++u) {
             const int e = tid + 256 * u;
-            As[e >> 6][e & 63] = pa[u];
+            As[e / TR][e % TR] = pa[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 2 * WC; ++u) {
+            const int e = tid + 256 * u;
             Bs[e & 15][e >> 4] = pb[u];
         }
         __syncthreads();
@@ -760,14 +807,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 // C -= A B for the blocked LU: FP64 on k_zgemm, FP32 on k_cgemm32_sub
 static void gemm_sub(int m, int n, int k, const cdbl* A, const cdbl* B, cdbl* C, int ld, long long s, int batch,
                      hipStream_t st) {
-    zgemm_batched(m, n, k, mk(-1, 0), A, ld, s, B, ld, s, false, mk(1, 0), C, ld, s, batch, st);
+    zgemm_batched(m, n, k, mk(-1, 0), A, ld, s, B, ld, s, mk(1, 0), C, ld, s, batch, st);
 }
 static void gemm_sub(int m, int n, int k, const cflt* A, const cflt* B, cflt* C, int ld, long long s, int batch,
                      hipStream_t st) {
     if (m <= 0 || n <= 0 || batch <= 0) return;
-    const long long total = (long long)((m + 63) / 64) * ((n + 63) / 64) * batch;
-    hipLaunchKernelGGL(k_cgemm32_sub, dim3((unsigned)(8 * ((total + 7) / 8))), dim3(256), 0, st, m, n, k, A, B, C, ld, s,
-                       batch);
+    auto run = [&](auto tile) {               // tiles as in zgemm_batched
+        constexpr int WR = decltype(tile)::value, WC = 4 / WR;
+        const long long total = (long long)((m + 32 * WR - 1) / (32 * WR)) * ((n + 32 * WC - 1) / (32 * WC)) * batch;
+        hipLaunchKernelGGL((k_cgemm32_sub<WR, WC>), dim3((unsigned)(8 * ((total + 7) / 8))), dim3(256), 0, st, m, n, k, A, B, C,
+                           ld, s, batch);
+    };
+    if (n <= 32 && m > 32) run(std::integral_constant<int, 4>{});
+    else if (m <= 32 && n > 32) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 2>{});
 }
 
 // Blocked right-looking LU in steps of S 32-column sub-panels (S = 2; above
@@ -1172,6 +1225,110 @@ void csr_apply_batched(const int* rowptr, const int* colidx, const double* val, 
     if (total <= 0) return;
     hipLaunchKernelGGL(k_csr_apply, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, rowptr, colidx, val, n, X,
                        Y, ncols);
+}
+
+// Y = S X for n x n matrices X (count of them, columns in succession), S with its rows
+// in slices of 64 of similar length (sell_rows, sorted by it), the slice's entries
+// [k][64] so that a wavefront's loads of them coalesce.  A workgroup holds CW columns
+// of X in LDS, where the gathers run; kSellLds entries leave two workgroups a CU.
+constexpr int kSellLds = 4608;
+template <int CW>
+__global__ __launch_bounds__(512) void k_sell_left(const int* __restrict__ rows, const int* __restrict__ off,
+                                                   const int* __restrict__ col, const double* __restrict__ val, int n,
+                                                   const cdbl* __restrict__ X, cdbl* __restrict__ Y, long long ncols) {
+    __shared__ cdbl S[kSellLds];
+    __shared__ cdbl part[8][64];
+    const long long c0 = (long long)blockIdx.x * CW;
+    const int cw = (int)min((long long)CW, ncols - c0), lane = threadIdx.x & 63;
+    const cdbl* x = X + c0 * n;
+    for (int e = threadIdx.x; e < cw * n; e += 512) S[e] = x[e];
+    __syncthreads();
+    const int wv = threadIdx.x >> 6;
+    auto sums = [&](cdbl (&acc)[CW], int sl, int first, int step) {
+#pragma unroll
+        for (int c = 0; c < CW; ++c) acc[c] = mk(0, 0);
+        for (int p = off[sl] + 64 * first + lane; p < off[sl + 1]; p += 64 * step) {
+            const int j = col[p];
+            const double f = val[p];
+#pragma unroll
+            for (int c = 0; c < CW; ++c) axpy(acc[c], f, S[(c < cw ? c : 0) * n + j]);
+        }
+    };
+    // long slices (they come first) by all wavefronts together: a few rows have up to
+    // n / 2 entries
+    int sl0 = 0;
+    for (; 64 * sl0 < n && off[sl0 + 1] - off[sl0] > 64 * 64; ++sl0) {
+        cdbl acc[CW];
+        sums(acc, sl0, wv, 8);
+        const int r = 64 * sl0 + lane < n ? rows[64 * sl0 + lane] : -1;
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+            part[wv][lane] = acc[c];
+            __syncthreads();
+            if (wv == 0 && r >= 0 && c < cw) {
+                cdbl t = part[0][lane];
+                for (int k = 1; k < 8; ++k) t = t + part[k][lane];
+                Y[(c0 + c) * n + r] = t;
+            }
+            __syncthreads();
+        }
+    }
+    for (int sl = sl0 + wv; 64 * sl < n; sl += 8) {
+        cdbl acc[CW];
+        sums(acc, sl, 0, 1);
+        const int r = 64 * sl + lane < n ? rows[64 * sl + lane] : -1;
+        if (r < 0) continue;
+#pragma unroll
+        for (int c = 0; c < CW; ++c)
+            if (c < cw) Y[(c0 + c) * n + r] = acc[c];
+    }
+}
+
+// Y = X S^T for n x n matrices X, S in compressed rows: a thread per row of X, four
+// columns of Y a workgroup, S's entries uniform.
+__global__ __launch_bounds__(256) void k_csr_right(const int* __restrict__ rowptr, const int* __restrict__ colidx,
+                                                   const double* __restrict__ val, int n, const cdbl* __restrict__ X,
+                                                   cdbl* __restrict__ Y) {
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= n) return;
+    const cdbl* x = X + (size_t)blockIdx.z * n * n + r;
+    cdbl* y = Y + (size_t)blockIdx.z * n * n + r;
+    for (int i = 4 * blockIdx.y; i < min(n, 4 * (int)blockIdx.y + 4); ++i) {
+        cdbl s = mk(0, 0);
+        const int p1 = rowptr[i + 1];
+        int p = rowptr[i];
+        for (; p + 8 <= p1; p += 8) {            // eight loads in flight
+            cdbl t[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) t[u] = x[(size_t)colidx[p + u] * n];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) axpy(s, val[p + u], t[u]);
+        }
+        for (; p < p1; ++p) axpy(s, val[p], x[(size_t)colidx[p] * n]);
+        y[(size_t)i * n] = s;
+    }
+}
+
+// T <- S T S^T through tmp, for count n x n matrices.  The dense products of the
+// projection factor's inverse, which has 33 nonzeros a row, took 3.7 + 3.3 ms for 32
+// matrices of order 1000 on the matrix cores; these take 0.9 + 2.0 ms, and the context
+// keeps no dense inverse on the device.
+void sparse_congruence(const int* rowptr, const int* colidx, const double* val, const int* srows, const int* soff,
+                       const int* scol, const double* sval, int n, cdbl* T, cdbl* tmp, int count, hipStream_t st) {
+    const long long ncols = (long long)n * count;
+    auto left = [&](auto w) {
+        constexpr int CW = decltype(w)::value;
+        hipLaunchKernelGGL(k_sell_left<CW>, dim3((unsigned)((ncols + CW - 1) / CW)), dim3(512), 0, st, srows, soff, scol, sval,
+                           n, T, tmp, ncols);
+    };
+    // as many columns as fit, since they share the entries' loads
+    if (8 * n <= kSellLds) left(std::integral_constant<int, 8>{});
+    else if (4 * n <= kSellLds) left(std::integral_constant<int, 4>{});
+    else if (2 * n <= kSellLds) left(std::integral_constant<int, 2>{});
+    else if (n <= kSellLds) left(std::integral_constant<int, 1>{});
+    else csr_apply_batched(rowptr, colidx, val, n, T, tmp, ncols, st);
+    hipLaunchKernelGGL(k_csr_right, dim3((unsigned)((n + 255) / 256), (unsigned)((n + 3) / 4), (unsigned)count), dim3(256), 0,
+                       st, rowptr, colidx, val, n, tmp, T);
 }
 
 __global__ __launch_bounds__(256) void k_csr_apply_multi(const CsrDesc* __restrict__ desc, int n_pad,

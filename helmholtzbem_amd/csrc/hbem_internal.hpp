@@ -185,6 +185,8 @@ struct CsrDesc {
     const double* v;
     int n;
 };
+void sparse_congruence(const int* rowptr, const int* colidx, const double* val, const int* srows, const int* soff,
+                       const int* scol, const double* sval, int n, cdbl* T, cdbl* tmp, int count, hipStream_t st);
 void csr_apply_multi(const CsrDesc* desc, int n_pad, const cdbl* X, cdbl* Y, int ncols, int batch, hipStream_t st);
 // X_b (n_pad x nc) = the n_b x nc block at src + off[b] (column-major, ld
 // n_b) padded with zero rows, n_b = nrow[b]
@@ -229,7 +231,7 @@ void copy_blocks_batched(const cdbl* src, long long sstride, long long soff, cdb
                          long long doff, int len, int nb, hipStream_t st);
 // C = alpha * A * op(B) + beta * C   (complex, column-major, batched with strides)
 void zgemm_batched(int m, int n, int k, cdbl alpha, const cdbl* A, int lda, long long sa, const cdbl* B, int ldb,
-                   long long sb, bool transB, cdbl beta, cdbl* C, int ldc, long long sc, int batch, hipStream_t st);
+                   long long sb, cdbl beta, cdbl* C, int ldc, long long sc, int batch, hipStream_t st);
 
 // host setup (hbem_setup.cpp)
 void gauss_rule(double a, double b, int n, double* x, double* w);
