@@ -76,6 +76,13 @@ __device__ __forceinline__ void stage_column(cdbl v, cdbl d, int q, int bs, bool
     tile[(rev ? i : ti) * kTS + (rev ? j : tj)] = in ? v : mk(0, 0);
 }
 
+// Element at byte offset 16 or 8 (c n + i) of a column block, c < 64: a uniform base and
+// a 32-bit offset, one register an address where 64-bit ones spilled.
+template <class F>
+__device__ __forceinline__ F at(const F* block, int i, int c, int n) {
+    return *reinterpret_cast<const F*>(reinterpret_cast<const char*>(block) + (unsigned)(sizeof(F) * ((unsigned)c * (unsigned)n + (unsigned)i)));
+}
+
 template <int J>
 __device__ __forceinline__ double row_bcast(double x) {
     const unsigned long long b = __double_as_longlong(x);
@@ -232,8 +239,9 @@ __device__ __forceinline__ void subst_right(const F* M, int n, bool lower, cdbl*
     auto bsz = [&](int s) { return min(64, pe - rb(s)); };
     // sixteen columns of the block [r0, r0 + bs) at row i (clamped addresses)
     auto load16 = [&](auto& t, int i, int r0, int bs) {
+        const F* B = M + (size_t)r0 * n;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) t[u] = M[i + (size_t)(r0 + min(16 * grp + u, bs - 1)) * n];
+        for (int u = 0; u < 16; ++u) t[u] = at(B, i, min(16 * grp + u, bs - 1), n);
     };
     // rows i of a wavefront minus the block's columns times its unknowns
     auto apply16 = [&](const auto& t, int i, bool live, int bs, const cdbl* xb) {
@@ -294,10 +302,10 @@ __device__ __forceinline__ void subst_right(const F* M, int n, bool lower, cdbl*
                     load16(pre, rn + min(16 * (wv - 1) + l16, bn - 1), r0, bs);
                 } else {
                     const int p = min(lane, bn - 1);
-                    if (!lower) dg = M[(rn + p) + (size_t)(rn + p) * n];
+                    const F* B = M + (size_t)rn * n;
+                    if (!lower) dg = at(B, rn + p, p, n);
 #pragma unroll
-                    for (int u = 0; u < 22; ++u)
-                        pre[u] = M[(rn + p) + (size_t)(rn + min(wv - 5 + 3 * u, bn - 1)) * n];
+                    for (int u = 0; u < 22; ++u) pre[u] = at(B, rn + p, min(wv - 5 + 3 * u, bn - 1), n);
                 }
             }
         }
@@ -348,6 +356,7 @@ __device__ __forceinline__ void subst_left(const F* M, int n, bool lower, cdbl* 
         if (wv == 0) {
             diag_solve<NC>(r0 - pb, bs, lower, !lower, w, S.tile, S.dinv, S.xb[s & 1]);
         } else if (next) {
+            const F* B = M + (size_t)rn * n;
             if (s > 0) {
                 const int ja = lower ? pb : r0 + bs, jb = lower ? r0 : pe;   // finished before block s
                 const int T = (jb - ja + 63) >> 6;
@@ -363,7 +372,7 @@ __device__ __forceinline__ void subst_left(const F* M, int n, bool lower, cdbl* 
                         for (int h = 0; h < TW; ++h) {
                             const int jc = min(ja + lane + 64 * (tt + h), jb - 1);
 #pragma unroll
-                            for (int q = 0; q < CB; ++q) mv[h][q] = M[jc + (size_t)(rn + min(q0 + q, bn - 1)) * n];
+                            for (int q = 0; q < CB; ++q) mv[h][q] = at(B, jc, min(q0 + q, bn - 1), n);
                         }
 #pragma unroll
                         for (int h = 0; h < TW; ++h) {
@@ -384,13 +393,12 @@ __device__ __forceinline__ void subst_left(const F* M, int n, bool lower, cdbl* 
             }
             if (wv <= 4) {
 #pragma unroll
-                for (int u = 0; u < 16; ++u)
-                    pre[u] = M[(r0 + min(lane, bs - 1)) + (size_t)(rn + min(16 * (wv - 1) + u, bn - 1)) * n];
+                for (int u = 0; u < 16; ++u) pre[u] = at(B, r0 + min(lane, bs - 1), min(16 * (wv - 1) + u, bn - 1), n);
             } else {
                 const int p = min(lane, bn - 1);
-                if (lower) dg = M[(rn + p) + (size_t)(rn + p) * n];
+                if (lower) dg = at(B, rn + p, p, n);
 #pragma unroll
-                for (int u = 0; u < 22; ++u) pre[u] = M[(rn + p) + (size_t)(rn + min(wv - 5 + 3 * u, bn - 1)) * n];
+                for (int u = 0; u < 22; ++u) pre[u] = at(B, rn + p, min(wv - 5 + 3 * u, bn - 1), n);
             }
         }
         __syncthreads();                          // block s solved, the older sums in
@@ -445,6 +453,7 @@ __global__ __launch_bounds__(kSolveThreads) void k_solve_thin(const F* __restric
         w[i * NC + c] = x[(adj ? i : p[i]) + (size_t)c * n];
     }
     __syncthreads();
+#pragma unroll 1
     for (int pass = 0; pass < 2; ++pass) {
         if (!adj) subst_right<NC>(lu, n, pass == 0, w, S, 0, n);
         else subst_left<NC>(lu, n, pass == 0, w, S, 0, n);
