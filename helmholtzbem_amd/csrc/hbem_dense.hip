@@ -823,12 +823,13 @@ static void gemm_sub(int m, int n, int k, const cflt* A, const cflt* B, cflt* C,
     else run(std::integral_constant<int, 2>{});
 }
 
-// Blocked right-looking LU in steps of S 32-column sub-panels (S = 2; above
-// order 2048, 8 for FP64 factors and 4 for FP32 ones: at order 4000 the
-// FP64 LU took 391 ms at S = 8 against 412 at S = 4 for 128 matrices, while
-// the FP32 LU at S = 8 left the mixed-precision sigma ten times farther from
-// FP64 -- 2e-9 against 2e-10 -- for 14 of its 230 ms).  Within a step,
-// sub-panel s is first brought up to date with the step's earlier sub-panels
+// Blocked right-looking LU in steps of S 32-column sub-panels: S = 2; FP64 factors above
+// order 1024 4 (order 1200, 64 matrices: a sweep's pass 16.0 -> 15.0 ms, order 1800 25.0
+// -> 23.2; order 800 in batches of one 4.0 -> 4.25 ms, so not below), above 2048 8
+// (order 4000: 391 ms at S = 8 against 412 at S = 4 for 128 matrices; S = 16 another 1%
+// there and 1% slower at 2060); FP32 ones above 2048 4 (S = 8 left the mixed-precision
+// sigma ten times farther from FP64 -- 2e-9 against 2e-10 -- for 14 of its 230 ms).
+// Within a step, sub-panel s is first brought up to date with the step's earlier sub-panels
 // (k = 32 s), factorised, its row interchanges applied to every other column,
 // and its U rows right of it formed; the trailing matrix then receives one
 // k = 32 S update per step.
@@ -846,7 +847,8 @@ static void gemm_sub(int m, int n, int k, const cflt* A, const cflt* B, cflt* C,
 template <class C>
 static void lu_factor_impl(C* A, int n, int batch, int* ipiv, int* perm, hipStream_t st, LaunchTimer* tm) {
     const int sb = 32;
-    const int S = n > 2048 ? (sizeof(C) == sizeof(cdbl) ? 8 : 4) : 2;
+    constexpr bool f64 = sizeof(C) == sizeof(cdbl);
+    const int S = n > 2048 ? (f64 ? 8 : 4) : (f64 && n > 1024 ? 4 : 2);
     const long long s = (long long)n * n;
     auto at = [&](int r, int c) { return A + r + (size_t)c * n; };
     auto update = [&](int m, int nn, int k, const C* a, const C* b, C* c) {
