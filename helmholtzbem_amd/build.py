@@ -19,7 +19,8 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libhbem.so")
 ARCH = os.environ.get("HBEM_OFFLOAD_ARCH", "gfx950")
 
-HIP_SOURCES = ["hbem_assembly.hip", "hbem_radial.hip", "hbem_dense.hip", "hbem_solve.hip", "hbem_capi.hip"]
+HIP_SOURCES = ["hbem_assembly.hip", "hbem_radial.hip", "hbem_dense.hip", "hbem_solve.hip", "hbem_solve_f32.hip",
+               "hbem_capi.hip"]
 HOST_SOURCES = ["hbem_setup.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -475,7 +475,7 @@ __global__ __launch_bounds__(kSolveThreads) void k_solve_thin(const F* __restric
 // but the bulk of the reads no longer waits on one workgroup per matrix.
 
 // w = P x (A x = b) or w = x (A^H x = b)
-__global__ void k_thin_in(const int* __restrict__ perm, int n, int nc, const cdbl* __restrict__ X, int adj,
+static __global__ void k_thin_in(const int* __restrict__ perm, int n, int nc, const cdbl* __restrict__ X, int adj,
                           cdbl* __restrict__ work) {
     const int b = blockIdx.y;
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -486,7 +486,7 @@ __global__ void k_thin_in(const int* __restrict__ perm, int n, int nc, const cdb
 }
 
 // x = w (A x = b) or x = P^T w (A^H x = b)
-__global__ void k_thin_out(const int* __restrict__ perm, int n, int nc, cdbl* __restrict__ X, int adj,
+static __global__ void k_thin_out(const int* __restrict__ perm, int n, int nc, cdbl* __restrict__ X, int adj,
                            const cdbl* __restrict__ work) {
     const int b = blockIdx.y;
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -799,14 +799,17 @@ static void solve_thin_impl(const F* LU, long long ms, const int* perm, int n, i
     }
 }
 
+// (the instances for FP32 factors are compiled by hbem_solve_f32.hip)
+#ifndef HBEM_SOLVE_F32
 void lu_solve_thin_batched(const cdbl* LU, long long ms, const int* perm, int n, int batch, cdbl* X, int nc, bool adj,
                            cdbl* work, hipStream_t st) {
     solve_thin_impl(LU, ms, perm, n, batch, X, nc, adj, work, st);
 }
-
+#else
 void lu_solve_thin_batched_f32(const cflt* LU, long long ms, const int* perm, int n, int batch, cdbl* X, int nc,
                                bool adj, cdbl* work, hipStream_t st) {
     solve_thin_impl(LU, ms, perm, n, batch, X, nc, adj, work, st);
 }
+#endif
 
 }  // namespace hbem
