@@ -49,7 +49,12 @@ struct DBuf {
         return p;
     }
     template <class T> T* as(size_t count) { return (T*)get(count * sizeof(T)); }
-    ~DBuf() { if (p) (void)hipFree(p); }
+    void release() {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        n = 0;
+    }
+    ~DBuf() { release(); }
 };
 
 template <class T>
@@ -446,7 +451,9 @@ int class_nodes(const hbem_geometry* g, int cls) {
 
 long long tri_index(int i, int j) { return i >= j ? (long long)i * (i + 1) / 2 + j : (long long)j * (j + 1) / 2 + i; }
 
-// Bands and tiles of the geometry (independent of kappa), built on first use.
+// Bands and tiles of the geometry (independent of kappa), built on first use; not
+// usable with fewer than 8 panels or where consecutive panels lie so far apart that
+// a pair of hats leaves its band (hbem_radial.hip).
 hbem_geometry::Radial& radial_base(hbem_geometry* g) {
     auto& r = g->rad;
     if (r.built) return r;
@@ -475,7 +482,8 @@ hbem_geometry::Radial& radial_base(hbem_geometry* g) {
     const size_t obf = al256(band.size() * sizeof(band[0]));
     unsigned short* db = (unsigned short*)r.flagmem.get(obf + g->npairs);
     HIPC(hipMemcpyAsync(db, band.data(), band.size() * sizeof(band[0]), hipMemcpyHostToDevice, g->st));
-    hbem::launch_radial_band((const double*)g->d_gtab.p, N, g->ns, (int)g->npairs, r.R, r.first, r.step, db, g->st);
+    hbem::launch_radial_band((const double*)g->d_gtab.p, N, g->ns, (int)g->npairs, r.R, r.first, r.step, r.width, db,
+                             g->st);
     unsigned char* fl = (unsigned char*)db + obf;
     r.flags = fl;
     HIPC(hipMemcpyAsync(band.data(), db, band.size() * sizeof(band[0]), hipMemcpyDeviceToHost, g->st));
@@ -484,6 +492,14 @@ hbem_geometry::Radial& radial_base(hbem_geometry* g) {
     HIPC(hipGetLastError());
     int top = 0;
     for (unsigned short b : band) top = std::max<int>(top, b);
+    if (top == hbem::kBandOutside) {
+        // panels that do not follow one another: every call of this context takes
+        // the node loops, which sum each panel pair by itself
+        HIPC(hipStreamSynchronize(g->st));
+        r.flagmem.release();
+        r.built = true;
+        return r;
+    }
     r.nbands = top + 1;
     // tiles of 16 pairs, band by band (the last of a band padded with -1)
     std::vector<long long> count(r.nbands, 0), pos(r.nbands, 0);
@@ -1252,11 +1268,7 @@ int hbem_geometry_release_work(hbem_geometry_t g) {
                              &g->w_rec.tab,
                              &g->w_scr.E, &g->w_scr.L, &g->w_scr.part};
     for (auto& b : g->w_rec.lslots) bs.push_back(b.get());
-    for (DBuf* b : bs) {
-        if (b->p) (void)hipFree(b->p);
-        b->p = nullptr;
-        b->n = 0;
-    }
+    for (DBuf* b : bs) b->release();
     API_END
 }
 

@@ -93,7 +93,8 @@ struct RadialParams {
     cdbl* out;
 };
 int band_order(double c, double a, double kmax, double tol, bool near);
-void launch_radial_band(const double* gtab, int N, int ns, int npairs, double R, double first, double step,
+constexpr int kBandOutside = 0xffff;   // a pair whose distances leave every band's interval
+void launch_radial_band(const double* gtab, int N, int ns, int npairs, double R, double first, double step, double width,
                         unsigned short* band, hipStream_t st);
 void launch_radial_flags(const double* gtab, int ns, int npairs, unsigned char* flags, hipStream_t st);
 void launch_radial_far(const int* recs, const BandTile* tiles, int tile0, int ntile, const Band* bands, int pmax,

@@ -67,10 +67,14 @@ __device__ __forceinline__ void tri_mn(int rec, int& m, int& n) {
 // distances of its four panel pairs: 0 (near) when hi <= R or the pair touches a
 // singular panel pair (band[rec] != 0 on entry), else 1 + floor((lo - first) /
 // step); band b covers [first + (b - 1) step, first + b step + W], W the largest
-// width an interval can have, so it holds the whole interval.
+// width an interval can have where a hat's two panels meet, so it holds the whole
+// interval.  Consecutive panels of a mesh need not meet (several curves in one
+// mesh, an open arc): a pair over such a seam may leave its band, where the
+// polynomials grow without bound, and is marked kBandOutside.
 // Four lanes a pair, one panel pair each.
 __global__ __launch_bounds__(256) void k_radial_band(const double* __restrict__ gtab, int N, int ns, int npairs, double R,
-                                                     double first, double step, unsigned short* __restrict__ band) {
+                                                     double first, double step, double width,
+                                                     unsigned short* __restrict__ band) {
     const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int rec = (int)(id >> 2) < npairs ? (int)(id >> 2) : npairs - 1, ab = (int)id & 3;
     const bool touch = band[rec] != 0;
@@ -79,7 +83,7 @@ __global__ __launch_bounds__(256) void k_radial_band(const double* __restrict__ 
     double lo = 1e300, hi = 0.0;
     const int P = (ab & 1) ? m : (m == 0 ? N - 1 : m - 1);
     const int Q = (ab >> 1) ? n : (n == 0 ? N - 1 : n - 1);
-    for (int i = 0; i < ns && !touch; ++i) {
+    for (int i = 0; i < ns; ++i) {
         const double* gi = gtab + ((size_t)P * ns + i) * 5;
         const double x = gi[0], y = gi[1];
         for (int j = 0; j < ns; ++j) {
@@ -97,8 +101,16 @@ __global__ __launch_bounds__(256) void k_radial_band(const double* __restrict__ 
     }
     lo = sqrt(lo);
     hi = sqrt(hi);
-    if (ab == 0 && (id >> 2) < npairs)
-        band[rec] = touch || hi <= R ? 0 : (unsigned short)(1 + (int)fmin(fmax(floor((lo - first) / step), 0.0), 65533.0));
+    if (ab == 0 && (id >> 2) < npairs) {
+        unsigned short b = 0;
+        bool in = hi <= R;
+        if (!touch && !in) {
+            b = (unsigned short)(1 + (int)fmin(fmax(floor((lo - first) / step), 0.0), kBandOutside - 2.0));
+            const double end = first + b * step;
+            in = lo >= end - step && hi <= end + width;
+        }
+        band[rec] = in ? b : (unsigned short)kBandOutside;
+    }
 }
 
 // Skip flags of the general panel pairs (the reference's isArrayZero tests,
@@ -1157,9 +1169,10 @@ int band_order(double c, double a, double kmax, double tol, bool near) {
     return 0;
 }
 
-void launch_radial_band(const double* gtab, int N, int ns, int npairs, double R, double first, double step,
+void launch_radial_band(const double* gtab, int N, int ns, int npairs, double R, double first, double step, double width,
                         unsigned short* band, hipStream_t st) {
-    hipLaunchKernelGGL(k_radial_band, dim3(grid_of(4LL * npairs)), dim3(256), 0, st, gtab, N, ns, npairs, R, first, step, band);
+    hipLaunchKernelGGL(k_radial_band, dim3(grid_of(4LL * npairs)), dim3(256), 0, st, gtab, N, ns, npairs, R, first, step,
+                       width, band);
 }
 
 void launch_radial_flags(const double* gtab, int ns, int npairs, unsigned char* flags, hipStream_t st) {
