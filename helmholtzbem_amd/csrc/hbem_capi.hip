@@ -355,7 +355,7 @@ struct hbem_geometry {
     };
     static constexpr int kTiers = 6;
     struct Radial {
-        bool built = false, usable = false;
+        bool usable = false;
         int nbands = 0, ntile = 0, ntile_near = 0;
         long long nfar = 0;
         double R = 0.0, first = 0.0, step = 0.0, width = 0.0;
@@ -366,7 +366,8 @@ struct hbem_geometry {
         const hbem::RadialNear* d_near = nullptr;
         const int* recs = nullptr;
         Tier tier[kTiers];
-    } rad;
+    };
+    std::unique_ptr<Radial> rad;           // null until it is complete
     DBuf d_M;
     DCsr s_F, s_FT, s_FinvT, s_Finv;   // F, F^T, Finv^T and Finv of the projection
     DSell l_Finv;                      // Finv once more, in slices
@@ -455,13 +456,14 @@ long long tri_index(int i, int j) { return i >= j ? (long long)i * (i + 1) / 2 +
 // usable with fewer than 8 panels or where consecutive panels lie so far apart that
 // a pair of hats leaves its band (hbem_radial.hip).
 hbem_geometry::Radial& radial_base(hbem_geometry* g) {
-    auto& r = g->rad;
-    if (r.built) return r;
+    if (g->rad) return *g->rad;
+    // (an allocation that fails on the way leaves the context without a plan)
+    auto plan_ptr = std::make_unique<hbem_geometry::Radial>();
+    auto& r = *plan_ptr;
+    auto done = [&]() -> hbem_geometry::Radial& { return *(g->rad = std::move(plan_ptr)); };
     const int N = g->N;
-    if (N < 8 || g->npairs > 0x7fffffffLL || !(g->dmax > 0.0)) {
-        r.built = true;                       // too few panels for disjoint supports: the node loops
-        return r;
-    }
+    // too few panels for disjoint supports: the node loops
+    if (N < 8 || g->npairs > 0x7fffffffLL || !(g->dmax > 0.0)) return done();
     r.R = kNearRadius * g->dmax;
     r.width = kBandWidth * g->dmax * (1.0 + 1e-12);
     r.step = kBandStep * g->dmax;
@@ -497,8 +499,7 @@ hbem_geometry::Radial& radial_base(hbem_geometry* g) {
         // the node loops, which sum each panel pair by itself
         HIPC(hipStreamSynchronize(g->st));
         r.flagmem.release();
-        r.built = true;
-        return r;
+        return done();
     }
     r.nbands = top + 1;
     // tiles of 16 pairs, band by band (the last of a band padded with -1)
@@ -538,8 +539,7 @@ hbem_geometry::Radial& radial_base(hbem_geometry* g) {
     r.recs = (const int*)(plan + orec);
     HIPC(hipStreamSynchronize(g->st));        // the upload reads a host vector
     r.usable = true;
-    r.built = true;
-    return r;
+    return done();
 }
 
 // Points and coefficient tables of tier t, built on first use (null: a band
@@ -598,11 +598,12 @@ hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
     }
     std::vector<hbem::BandTile> tiles(r.ntile);
     long long off = 0;
+    double npoints = 0.0;
     for (int i = 0; i < r.ntile; ++i) {
         const int b = r.tile_band[i];
         tiles[i] = {off, b, 0};
         off += (long long)bands[b].p * (b == 0 ? 10 : 5) * 16;
-        if (b) T.points += 16.0 * bands[b].p;
+        if (b) npoints += 16.0 * bands[b].p;
     }
     std::vector<int> cent;
     for (int i = 0; i < g->N; ++i) cent.insert(cent.end(), {i, i, 0});
@@ -649,6 +650,7 @@ hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
                             g->ns, r.flags, dc, tab, g->st);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(g->st));        // the uploads above read host vectors; other streams may use the tables
+    T.points = npoints;
     T.pmax = pmax;
     T.pnear = pn;
     T.basis = basis;
@@ -702,7 +704,7 @@ constexpr double kNearImag = 0.5;
 int record_tier(hbem_geometry* g, double lo, double hi, double im) {
     const int t = lo > 0.0 ? tier_of(hi * g->dmax) : -1;
     if (t < 0 || !radial_tier(g, t)) return -1;
-    if (im > 0.0 && (im * g->rad.R > kNearImag || hi * g->rad.R > hbem::kEntireMax)) return -1;
+    if (im > 0.0 && (im * g->rad->R > kNearImag || hi * g->rad->R > hbem::kEntireMax)) return -1;
     return t;
 }
 
@@ -843,7 +845,7 @@ RecJob prepare_records(hbem_geometry* g, RecBufs& b, RecScratch& w, hipStream_t 
         r.count = (int)kv.second.size();
         cols.insert(cols.end(), kv.second.begin(), kv.second.end());
         if (r.tier >= 0)
-            nbasis = std::max(nbasis, (size_t)(g->rad.tier[r.tier].basis + (J.cplx ? 2 * g->rad.tier[r.tier].pnear : 0)) *
+            nbasis = std::max(nbasis, (size_t)(g->rad->tier[r.tier].basis + (J.cplx ? 2 * g->rad->tier[r.tier].pnear : 0)) *
                                           r.count * (diff ? 2 : 1));
         if (r.tier < 0) {
             // the group's slots: blocks of 32 wavenumbers, inner and outer in turn
@@ -908,7 +910,7 @@ cdbl* launch_records(const RecJob& J) {
     cdbl* E = (cdbl*)J.w->E.p;
     for (const RecGroup& r : J.groups) {
         if (r.tier >= 0) {
-            const auto& R = g->rad;
+            const auto& R = *g->rad;
             const auto& T = R.tier[r.tier];
             hbem::RadialParams P;
             P.kap = J.kap;
