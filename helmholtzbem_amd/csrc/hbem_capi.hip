@@ -956,15 +956,20 @@ cdbl* assemble_records(hbem_geometry* g, const std::vector<double>& kap, const s
 }
 
 // Device bytes per column of a call with these kappa (the larger one of each
-// column): its records, and where one of them takes the node loops for every
-// pair their local matrices and partials too.  Builds the tiers the call needs,
-// so that the free memory seen afterwards is what its batches can use.
-size_t records_bytes_per_k(hbem_geometry* g, const std::vector<double>& kap, int D, int lcols) {
+// column) and `slots` kappa a column: its records and basis, and where one of them
+// takes the node loops for every pair their local matrices and partials too.  Builds
+// the tables the call needs, so that the free memory seen afterwards is what its
+// batches can use.
+size_t records_bytes_per_k(hbem_geometry* g, const std::vector<double>& kap, int D, int lcols, int slots) {
     bool loops = false;
+    size_t basis = 0;
     for (double v : kap) {
-        loops = loops || record_tier(g, std::fabs(v), std::fabs(v), 0.0) < 0;
+        const int t = D >= 1 && record_values(g, D) != hbem::kRecValues ? -1 : record_tier(g, std::fabs(v), std::fabs(v), 0.0);
+        if (t < 0) loops = true;
+        else basis = std::max(basis, (size_t)(g->rad->tier[t].basis + 2 * g->rad->tier[t].pnear) * slots * sizeof(cdbl));
     }
-    return (size_t)g->npairs * record_values(g, D) * (D + 1) * sizeof(cdbl) +
+    if (loops) node_loops(g);
+    return (size_t)g->npairs * record_values(g, D) * (D + 1) * sizeof(cdbl) + basis +
            (loops ? locals_bytes_per_k(g->npairs, (long long)g->aent.size() / 3, g->N, g->nc, D, lcols) : 0);
 }
 
@@ -1323,7 +1328,7 @@ int hbem_assemble_dense_batch(hbem_geometry_t g, const double* ks, int nk, doubl
     // one wavenumber slot per k: its records, and its local matrices where it takes the node loops
     std::vector<double> all(nk);
     for (int i = 0; i < nk; ++i) all[i] = ks[i] * sc;
-    const size_t per = records_bytes_per_k(g, all, d, 1);
+    const size_t per = records_bytes_per_k(g, all, d, 1, 1);
     const int B = sweep_batch(per, usable_device_bytes(g->w_scr.E.n + g->w_scr.L.n + g->w_scr.part.n), nk);
     for (int k0 = 0; k0 < nk; k0 += B) {
         const int nb = std::min(B, nk - k0);
@@ -1834,7 +1839,7 @@ void sweep_run(hbem_geometry* g, const double* ks, int nk, double c_o, double c_
     const double si = std::sqrt(c_i), so = std::sqrt(c_o);
     std::vector<double> all;
     for (int i = 0; i < nk; ++i) all.push_back(ks[i] * std::max(si, so));
-    const size_t per = records_bytes_per_k(g, all, D, tdiff ? 1 : 2) + dense_bytes_per_k(n, D, nc) +
+    const size_t per = records_bytes_per_k(g, all, D, tdiff ? 1 : 2, 2) + dense_bytes_per_k(n, D, nc) +
                        (d2sigma ? der2_bytes_per_k(n) : 0) + (mx ? mixed_bytes_per_k(n, nc) : 0);
     const int B = sweep_batch(per, usable_device_bytes(g->work_held()), nk);
     cdbl* dR = g->w_R.as<cdbl>((size_t)n * nc);
@@ -2229,6 +2234,16 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
     std::vector<std::pair<int, int>> key(ninst);
     for (int i = 0; i < ninst; ++i) key[i] = {(2 * G[i]->N + gran - 1) / gran * gran, i};
     std::sort(key.begin(), key.end());
+    // (the instances' tables first: the free memory is what is left beside them)
+    std::vector<size_t> need(ninst);
+    for (int i = 0; i < ninst; ++i) {
+        const double cm = std::sqrt(std::max(c_i[i], c_o));
+        std::vector<double> kap;
+        for (int j = 0; j < nk; ++j) kap.push_back(ks[(size_t)i * nk + j] * cm);
+        const size_t n_pad = (2 * (size_t)G[i]->N + gran - 1) / gran * gran;
+        need[i] = (size_t)nk * records_bytes_per_k(G[i], kap, 0, 1, 2) +
+                  (size_t)nk * (n_pad * n_pad * sizeof(cdbl) + n_pad * (8 + (4 * nc + 4) * sizeof(cdbl)));
+    }
     size_t held = 0;
     {
         MultiWork& w = g_multi;
@@ -2242,16 +2257,10 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
         std::vector<int> ids;
         size_t used = 0;
         while (a < key.size() && key[a].first == n_pad) {
-            hbem_geometry* g = G[key[a].second];
-            const double* kg = ks + (size_t)key[a].second * nk;
-            const double cm = std::sqrt(std::max(c_i[key[a].second], c_o));
-            std::vector<double> kap;
-            for (int j = 0; j < nk; ++j) kap.push_back(kg[j] * cm);
-            const size_t need = (size_t)nk * records_bytes_per_k(g, kap, 0, 1) +
-                                (size_t)nk * ((size_t)n_pad * n_pad * sizeof(cdbl) + (size_t)n_pad * (8 + (4 * nc + 4) * sizeof(cdbl)));
-            if (!ids.empty() && used + need > avail) break;
-            ids.push_back(key[a].second);
-            used += need;
+            const int i = key[a].second;
+            if (!ids.empty() && used + need[i] > avail) break;
+            ids.push_back(i);
+            used += need[i];
             ++a;
         }
         multi_subset(G, ids, n_pad, ks, nk, c_o, c_i, R, nc, q, sigma);

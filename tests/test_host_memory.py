@@ -104,3 +104,46 @@ def test_failed_allocation_leaves_no_trace(stub, what, least, flags):
 
 def test_failed_allocation_leaves_no_trace_complex(stub):
     print(run(stub, FAILING % dict(what="layers", least=5, flags=0, k="3.0 + 0.05j")))
+
+
+BUDGET_MULTI = """
+stub.hip_stub_capacity(12 << 30)
+items = []
+for i in range(14):
+    mesh = H.polygon_mesh([(0, 0), (1, 0), (1.2, 0.7 + 0.01 * i), (0.1, 1)], 400)
+    bd = H.BuilderData(mesh, SP, SP, 8)
+    items.append((bd, np.linspace(20.0, 60.0, 32), 1.0, 9.0, H.gaussian_test_matrix(800, 2, i)))
+H.sigma_sweep_batched(items, 2)
+launches()
+first = stub.hip_stub_peak()
+H.sigma_sweep_batched(items, 2)
+print("device phases", sum("k_replicate_padded" in x for x in launches()), "peak", first >> 20, "MiB")
+assert first <= 12 << 30
+"""
+
+BUDGET_SWEEP = """
+stub.hip_stub_capacity(%(gib)d << 30)
+mesh = H.polygon_mesh([(0, 0), (1, 0), (1.2, 0.7), (0.1, 1)], 600)
+bd = H.BuilderData(mesh, SP, SP, 16, flags=%(flags)d)
+ks = np.linspace(1.0, 40.0, 256) * %(scale)g
+%(call)s
+print("peak", stub.hip_stub_peak() >> 20, "MiB")
+"""
+
+SWEEP1 = "H.sigma_sweep(bd, ks, 1.0, 9.0, H.gaussian_test_matrix(1200, 2, 0), 2, der=1)"
+# (without the host matrices, whose copies would be resident)
+BATCH1 = "_lib.check(L.hbem_assemble_dense_batch(bd._geo.h, ks.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), 256, 9.0, 7, 1, None, None, None))"
+
+
+def test_multi_sweep_budgets_its_tables(stub):
+    """Fourteen instances whose tables and matrices together exceed the device: the
+    tables are built before the free memory is read, so the subsets fit what is left."""
+    print(run(stub, BUDGET_MULTI))
+
+
+@pytest.mark.parametrize("call", [SWEEP1, BATCH1])
+@pytest.mark.parametrize("what,flags,scale", [("quirk", 1, 1.0), ("beyond_the_tiers", 0, 1000.0), ("bands", 0, 1.0)])
+def test_sweeps_budget_their_tables(stub, call, what, flags, scale):
+    """The node tables of 180 000 panel pairs (3.3 GB) or the bands' tables are part of
+    the device memory when a sweep sizes its batches."""
+    print(run(stub, BUDGET_SWEEP % dict(gib=16, flags=flags, scale=scale, call=call)))
