@@ -2070,11 +2070,11 @@ bool graphs_enabled() {
 }
 
 // One bucket subset of hbem_sigma_sweep_multi: instances `ids` (all padded to
-// order n_pad), their nk wavenumbers each.  The panel pairs of every class of
-// all these instances are assembled by one launch; T of instance i, k j is
-// matrix i_local nk + j of one batch of order n_pad (identity in the
-// padding), factorised and reduced to sigma by the batched dense stage.
-void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& ids, int n_pad, const double* ks, int nk,
+// order n_pad, all factorised in steps of `panels` sub-panels by their own order),
+// their nk wavenumbers each.  T of instance i, k j is matrix i_local nk + j of one
+// batch of order n_pad (identity in the padding), factorised and reduced to sigma by
+// the batched dense stage.
+void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& ids, int n_pad, int panels, const double* ks, int nk,
                   double c_o, const double* c_i, const void* const* R, int nc, int q, double* sigma) {
     MultiWork& w = g_multi;
     hbem_geometry* g0 = G[ids[0]];
@@ -2083,7 +2083,6 @@ void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& 
     const size_t nn = (size_t)n_pad * n_pad;
     const int batch = m * nk;
     // ---- host side: every table the device phase reads, uploaded first ----
-    const bool tdiff = true;                  // the difference layout of hbem_sigma_sweep (nk >= 32)
     std::vector<RecJob> jobs;
     while ((int)w.rec.size() < m) w.rec.push_back(std::make_unique<RecBufs>());
     for (int a = 0; a < m; ++a) {
@@ -2094,7 +2093,8 @@ void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& 
             kap[j] = k * std::sqrt(c_i[i]); kr[j] = k; cv[j] = c_i[i];
             kap[nk + j] = k * std::sqrt(c_o); kr[nk + j] = k; cv[nk + j] = c_o;
         }
-        jobs.push_back(prepare_records(G[i], *w.rec[a], w.scr, st, kap, kr, cv, 0, true, {}, {}, tdiff));
+        jobs.push_back(prepare_records(G[i], *w.rec[a], w.scr, st, kap, kr, cv, 0, true, {}, {},
+                                       sweep_tdiff(ks + (size_t)i * nk, nk)));
     }
     std::vector<hbem::CsrDesc> desc(batch), descT(batch);
     std::vector<long long> roff(batch);
@@ -2140,7 +2140,7 @@ void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& 
                                 nullptr, st, n_pad);
             if (n < n_pad) hbem::launch_pad_identity(T + (size_t)a * nk * nn, n, n_pad, nk, st);
         }
-        hbem::lu_factor_batched(T, n_pad, batch, piv, perm, st);
+        hbem::lu_factor_batched(T, n_pad, batch, piv, perm, st, nullptr, panels);
         DenseCtx c;
         c.st = st; c.n = n_pad; c.batch = batch; c.nc = nc; c.q = q; c.LU = T; c.ms = (long long)nn; c.perm = perm;
         c.F = nullptr;
@@ -2160,10 +2160,12 @@ void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& 
         key.push_back((const void*)(size_t)nc);
         key.push_back((const void*)(size_t)q);
         key.push_back((const void*)(size_t)n_pad);
+        key.push_back((const void*)(size_t)panels);
         const void* bufs[] = {dF, dFT, dRall, droff, dnrow, T, piv, perm, X, Y, work, dsig, w.scr.E.p, w.scr.L.p,
                               w.scr.part.p};
         // the ways its columns take, and the tables each reads
         for (const RecJob& J : jobs) {
+            key.push_back((const void*)(size_t)J.tdiff);
             for (const void* p : {(const void*)J.kap, (const void*)J.kr, (const void*)J.cv, (const void*)J.cols}) key.push_back(p);
             for (const RecGroup& r : J.groups)
                 for (const void* p : {(const void*)(size_t)(r.tier + 1), (const void*)(size_t)r.start, (const void*)(size_t)r.count,
@@ -2229,10 +2231,13 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
     for (auto* g : order) locks.emplace_back(g->mu);
     std::lock_guard<std::mutex> lk(g_multi.mu);
     HIPC(hipSetDevice(G[0]->dev));
-    // buckets of equal padded order, in increasing order; a bucket is split
-    // into subsets whose work space fits the free device memory
-    std::vector<std::pair<int, int>> key(ninst);
-    for (int i = 0; i < ninst; ++i) key[i] = {(2 * G[i]->N + gran - 1) / gran * gran, i};
+    // buckets of equal padded order, in increasing order; a bucket is split by the
+    // LU's step width, which follows the instance's own order (1024 and 2048 may lie
+    // inside a bucket), and into subsets whose work space fits the free device memory
+    typedef std::pair<std::pair<int, int>, int> Key;
+    std::vector<Key> key(ninst);
+    for (int i = 0; i < ninst; ++i)
+        key[i] = {{(2 * G[i]->N + gran - 1) / gran * gran, hbem::lu_step_panels(2 * G[i]->N, true)}, i};
     std::sort(key.begin(), key.end());
     // (the instances' tables first: the free memory is what is left beside them)
     std::vector<size_t> need(ninst);
@@ -2241,7 +2246,7 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
         std::vector<double> kap;
         for (int j = 0; j < nk; ++j) kap.push_back(ks[(size_t)i * nk + j] * cm);
         const size_t n_pad = (2 * (size_t)G[i]->N + gran - 1) / gran * gran;
-        need[i] = (size_t)nk * records_bytes_per_k(G[i], kap, 0, 1, 2) +
+        need[i] = (size_t)nk * records_bytes_per_k(G[i], kap, 0, sweep_tdiff(ks + (size_t)i * nk, nk) ? 1 : 2, 2) +
                   (size_t)nk * (n_pad * n_pad * sizeof(cdbl) + n_pad * (8 + (4 * nc + 4) * sizeof(cdbl)));
     }
     size_t held = 0;
@@ -2253,17 +2258,17 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
     const size_t avail = usable_device_bytes(held);
     size_t a = 0;
     while (a < key.size()) {
-        const int n_pad = key[a].first;
+        const std::pair<int, int> form = key[a].first;
         std::vector<int> ids;
         size_t used = 0;
-        while (a < key.size() && key[a].first == n_pad) {
+        while (a < key.size() && key[a].first == form) {
             const int i = key[a].second;
             if (!ids.empty() && used + need[i] > avail) break;
             ids.push_back(i);
             used += need[i];
             ++a;
         }
-        multi_subset(G, ids, n_pad, ks, nk, c_o, c_i, R, nc, q, sigma);
+        multi_subset(G, ids, form.first, form.second, ks, nk, c_o, c_i, R, nc, q, sigma);
     }
     API_END
 }

@@ -842,13 +842,13 @@ static void gemm_sub(int m, int n, int k, const cflt* A, const cflt* B, cflt* C,
 //           Us = Lss^{-1} A[js:js+32, js+32:]
 //   then:   A[jE:, jE:] -= L[jE:, j0:jE] U[j0:jE, jE:]
 // C = cdbl: the FP64 factorisation; C = cflt: the same steps in FP32.  The
-// step width depends on n and the precision only, so a matrix gives the same
-// bits in any batch.
+// step width depends on the order and the precision only (of a matrix padded to n: on
+// its order without the padding), so a matrix gives the same bits in any batch.
+int lu_step_panels(int n, bool f64) { return n > 2048 ? (f64 ? 8 : 4) : (f64 && n > 1024 ? 4 : 2); }
+
 template <class C>
-static void lu_factor_impl(C* A, int n, int batch, int* ipiv, int* perm, hipStream_t st, LaunchTimer* tm) {
+static void lu_factor_impl(C* A, int n, int batch, int* ipiv, int* perm, hipStream_t st, LaunchTimer* tm, int S) {
     const int sb = 32;
-    constexpr bool f64 = sizeof(C) == sizeof(cdbl);
-    const int S = n > 2048 ? (f64 ? 8 : 4) : (f64 && n > 1024 ? 4 : 2);
     const long long s = (long long)n * n;
     auto at = [&](int r, int c) { return A + r + (size_t)c * n; };
     auto update = [&](int m, int nn, int k, const C* a, const C* b, C* c) {
@@ -907,12 +907,12 @@ static void lu_factor_impl(C* A, int n, int batch, int* ipiv, int* perm, hipStre
     hipLaunchKernelGGL(k_lu_perm, dim3(batch), dim3(64), 0, st, n, ipiv, perm);
 }
 
-void lu_factor_batched(cdbl* A, int n, int batch, int* ipiv, int* perm, hipStream_t st, LaunchTimer* gemm) {
-    lu_factor_impl(A, n, batch, ipiv, perm, st, gemm);
+void lu_factor_batched(cdbl* A, int n, int batch, int* ipiv, int* perm, hipStream_t st, LaunchTimer* gemm, int panels) {
+    lu_factor_impl(A, n, batch, ipiv, perm, st, gemm, panels > 0 ? panels : lu_step_panels(n, true));
 }
 
 void lu_factor_batched_f32(cflt* A, int n, int batch, int* ipiv, int* perm, hipStream_t st, LaunchTimer* gemm) {
-    lu_factor_impl(A, n, batch, ipiv, perm, st, gemm);
+    lu_factor_impl(A, n, batch, ipiv, perm, st, gemm, lu_step_panels(n, false));
 }
 
 // ---------------------------------------------------------------------------

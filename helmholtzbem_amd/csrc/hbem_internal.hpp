@@ -144,7 +144,11 @@ struct LaunchTimer {
     virtual void end(hipStream_t st, double flops) = 0;
     virtual ~LaunchTimer() = default;
 };
-void lu_factor_batched(cdbl* A, int n, int batch, int* ipiv, int* perm, hipStream_t st, LaunchTimer* gemm = nullptr);
+// panels: sub-panels of 32 columns per step; 0: lu_step_panels(n), the form of a matrix
+// that is not padded
+int lu_step_panels(int n, bool f64);
+void lu_factor_batched(cdbl* A, int n, int batch, int* ipiv, int* perm, hipStream_t st, LaunchTimer* gemm = nullptr,
+                       int panels = 0);
 // X (n x nc, stride n*nc per matrix) <- op(A)^{-1} X with A = P^T L U from
 // lu_factor_batched (factors of matrix b at LU + b * ms); adj = false solves
 // A X = B, adj = true solves A^H X = B.  work: n * nc * batch.

@@ -270,9 +270,10 @@ int hbem_sigma_sweep_mixed(hbem_geometry_t g, const double* ks, int nk, double c
  * result.  The instances are grouped by their order 2 N_i rounded up to a
  * multiple of `bucket` (a multiple of 32; 0 = 256): a group's T matrices,
  * padded with the identity to the common order, are one batched LU and
- * randomized SVD, its device phase replayed from a captured graph.  The
- * padding leaves every result equal bit for bit to hbem_sigma_sweep of the
- * instance alone.
+ * randomized SVD, its device phase replayed from a captured graph.  For real
+ * positive wavenumbers every result equals hbem_sigma_sweep of the instance
+ * alone bit for bit: an instance is assembled by the same kernels and its LU
+ * takes the steps of its own order, whatever the padding and nk.
  */
 int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double* ks, int nk, double c_o,
                            const double* c_i, const void* const* R, int nc, int q, int bucket, double* sigma);
