@@ -325,7 +325,7 @@ struct hbem_geometry {
     int dev = 0;
     hipStream_t st = nullptr;
     int N = 0, order = 0, ns = 0, nc = 0, flags = 0;
-    bool lines = true, proj = true;
+    bool lines = true, straight = true, proj = true;   // straight: line and arc panels only
     long long npairs = 0;
     std::vector<double> panels, coefs, xg, wg, xc, wc;
     std::vector<double> M, F, Finv;
@@ -353,7 +353,7 @@ struct hbem_geometry {
         const hbem::BandTile* tiles = nullptr;
         const double *costab = nullptr, *tab = nullptr, *ext = nullptr;
     };
-    static constexpr int kTiers = 6;
+    static constexpr int kTiers = 6, kFarTiers = kTiers;   // then the same edges at the separated pairs' tolerance
     struct Radial {
         bool usable = false;
         int nbands = 0, ntile = 0, ntile_near = 0;
@@ -365,7 +365,7 @@ struct hbem_geometry {
         const unsigned char* flags = nullptr;
         const hbem::RadialNear* d_near = nullptr;
         const int* recs = nullptr;
-        Tier tier[kTiers];
+        Tier tier[kTiers + kFarTiers];
     };
     std::unique_ptr<Radial> rad;           // null until it is complete
     DBuf d_M;
@@ -429,8 +429,8 @@ bool real_positive(double k_re, double k_im) { return k_im == 0.0 && k_re > 0.0;
 // no rule resolves the panels, the node loops take over.
 constexpr double kTierEdge[hbem_geometry::kTiers] = {0.625, 1.25, 2.5, 5.0, 10.0, 20.0};
 // Interpolation error of the far bands relative to the radial function, and of
-// separated line and arc panels on contexts with HBEM_FLAG_FAR_FIELD (up to
-// kappa dmax = 5: half of the flag's 1e-13).
+// separated line and arc panels on contexts with HBEM_FLAG_FAR_FIELD at real positive
+// wavenumbers (up to kappa dmax = 5: half of the flag's 1e-13).
 constexpr double kBandTol = 1e-16, kBandTolFar = 5e-14, kNearTol = 1e-17;
 // Near radius, band step and largest interval width in units of dmax.  A hat's
 // support is at most 2 dmax wide, so a pair's distances spread over 4 dmax at
@@ -542,17 +542,19 @@ hbem_geometry::Radial& radial_base(hbem_geometry* g) {
     return done();
 }
 
-// Points and coefficient tables of tier t, built on first use (null: a band
-// would need more than kBandMaxP points).
+// Whether a wavenumber of tier t takes the separated pairs' tolerance: real positive
+// ones of contexts with HBEM_FLAG_FAR_FIELD on line and arc panels.
+bool far_tolerance(const hbem_geometry* g, int t, bool cplx) { return g->straight && (g->flags & HBEM_FLAG_FAR_FIELD) && !cplx && kTierEdge[t] <= 5.0; }
+
+// Points and coefficient tables of tier t (kTiers + t: at the separated pairs'
+// tolerance), built on first use (null: a band would need more than kBandMaxP points).
 hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
     auto& r = radial_base(g);
     if (!r.usable || t < 0) return nullptr;
     auto& T = r.tier[t];
     if (T.built) return T.pmax > 0 ? &T : nullptr;
-    bool straight = true;                     // line and arc panels only
-    for (int i = 0; i < g->N; ++i) straight = straight && g->panels[8 * (size_t)i] < 2.0;
-    const double tol = (g->flags & HBEM_FLAG_FAR_FIELD) && straight && kTierEdge[t] <= 5.0 ? kBandTolFar : kBandTol;
-    const double kmax = kTierEdge[t] / g->dmax;
+    const double tol = t >= hbem_geometry::kTiers ? kBandTolFar : kBandTol;
+    const double kmax = kTierEdge[t % hbem_geometry::kTiers] / g->dmax;
     std::vector<hbem::Band> bands(r.nbands);
     std::vector<double> cosv;
     std::map<int, int> cosoff;
@@ -700,9 +702,11 @@ hbem_geometry::Loops& node_loops(hbem_geometry* g) {
 // for the node loops: kappa = 0, beyond the last tier, or so far from the real
 // axis that J and iY of the near band, each of size e^{Im kappa r}, would leave
 // H with fewer digits (kNearImag: e^{2 Im kappa R} below 3).
+// cplx: it is evaluated as a complex one.
 constexpr double kNearImag = 0.5;
-int record_tier(hbem_geometry* g, double lo, double hi, double im) {
-    const int t = lo > 0.0 ? tier_of(hi * g->dmax) : -1;
+int record_tier(hbem_geometry* g, double lo, double hi, double im, bool cplx) {
+    int t = lo > 0.0 ? tier_of(hi * g->dmax) : -1;
+    if (t >= 0 && far_tolerance(g, t, cplx)) t += hbem_geometry::kTiers;
     if (t < 0 || !radial_tier(g, t)) return -1;
     if (im > 0.0 && (im * g->rad->R > kNearImag || hi * g->rad->R > hbem::kEntireMax)) return -1;
     return t;
@@ -833,7 +837,7 @@ RecJob prepare_records(hbem_geometry* g, RecBufs& b, RecScratch& w, hipStream_t 
             hi = std::max(hi, m);
             if (J.cplx) im = std::max(im, kapi[q]);
         }
-        by[quirk ? -1 : record_tier(g, lo, hi, im)].push_back(c);
+        by[quirk ? -1 : record_tier(g, lo, hi, im, J.cplx)].push_back(c);
     }
     std::vector<int> cols;
     size_t nL = 0, npart = 0, nbasis = 0;
@@ -961,10 +965,15 @@ cdbl* assemble_records(hbem_geometry* g, const std::vector<double>& kap, const s
 // the tables the call needs, so that the free memory seen afterwards is what its
 // batches can use.
 size_t records_bytes_per_k(hbem_geometry* g, const std::vector<double>& kap, int D, int lcols, int slots) {
-    bool loops = false;
+    const bool quirk = record_values(g, D) != hbem::kRecValues;
+    bool loops = false, cplx = false;
     size_t basis = 0;
+    // (a batch with a wavenumber that is not positive is evaluated as complex)
+    for (double v : kap) cplx = cplx || !(v > 0.0);
     for (double v : kap) {
-        const int t = D >= 1 && record_values(g, D) != hbem::kRecValues ? -1 : record_tier(g, std::fabs(v), std::fabs(v), 0.0);
+        const double m = std::fabs(v);
+        if (cplx && !quirk) record_tier(g, m, m, 0.0, true);
+        const int t = quirk ? -1 : record_tier(g, m, m, 0.0, false);
         if (t < 0) loops = true;
         else basis = std::max(basis, (size_t)(g->rad->tier[t].basis + 2 * g->rad->tier[t].pnear) * slots * sizeof(cdbl));
     }
@@ -1181,7 +1190,10 @@ int hbem_geometry_create(const double* panels, int npanels, const double* coefs,
     g->panels.assign(panels, panels + 8 * (size_t)npanels);
     if (ncoefs > 0) g->coefs.assign(coefs, coefs + 3 * (size_t)ncoefs);
     g->lines = true;
-    for (int i = 0; i < npanels; ++i) if ((int)panels[8 * i] != 0) g->lines = false;
+    for (int i = 0; i < npanels; ++i) {
+        if ((int)panels[8 * i] != 0) g->lines = false;
+        if ((int)panels[8 * i] >= 2) g->straight = false;
+    }
     g->xg.resize(g->ns); g->wg.resize(g->ns); g->xc.resize(g->nc); g->wc.resize(g->nc);
     hbem::gauss_rule(0.0, 1.0, g->ns, g->xg.data(), g->wg.data());
     hbem::composite_rule(order, g->xc.data(), g->wc.data());

@@ -57,13 +57,13 @@ extern "C" {
  * derivative order, which is what the k-derivative of V requires. */
 #define HBEM_FLAG_QUIRK_SLP_COINC_DER 1
 /* Separated panel pairs to 5e-14 instead of rounding.  On meshes of line and
- * arc panels only, every assembly through the context (matrices, T, sweeps)
- * interpolates the kernels of separated pairs over their distance bands with
- * as many points as keep them within 5e-14 of the largest value on the band
- * (1e-16 without the flag), for the wavenumbers with kappa times the largest
- * panel diameter up to 5.  Pairs closer than ten panel diameters, meshes with
- * trigonometric-curve or spline panels, wavenumbers the bands do not serve and
- * kappa d > 5 are those of the plain context.  Off by default: the reference
+ * arc panels only, every assembly through the context at real positive
+ * wavenumbers (matrices, T, sweeps) interpolates the kernels of separated pairs
+ * over their distance bands with as many points as keep them within 5e-14 of
+ * the largest value on the band (1e-16 without the flag), where kappa times
+ * the largest panel diameter is at most 5.  Pairs closer than ten panel
+ * diameters, meshes with trigonometric-curve or spline panels, complex
+ * wavenumbers and kappa d > 5 are those of the plain context.  Off by default: the reference
  * integrates every general pair with the same rule (galerkin_builder.cpp:
  * 308-327).  Not accepted by hbem_sigma_sweep_multi. */
 #define HBEM_FLAG_FAR_FIELD 2
