@@ -546,6 +546,43 @@ hbem_geometry::Radial& radial_base(hbem_geometry* g) {
 // ones of contexts with HBEM_FLAG_FAR_FIELD on line and arc panels.
 bool far_tolerance(const hbem_geometry* g, int t, bool cplx) { return g->straight && (g->flags & HBEM_FLAG_FAR_FIELD) && !cplx && kTierEdge[t] <= 5.0; }
 
+// The power of two with R^2 near_scale(R) in [1, 4).
+double near_scale(double R) { return std::ldexp(1.0, -2 * std::ilogb(R)); }
+// r^2 near_scale(R) of point j of the near band's p, Chebyshev in r^2 on [0, R^2]; the
+// point is the one this double names, whose last bit is clear (near_node).
+double near_u(double R, int p, int j) {
+    const long double x = R * cosl(acosl(-1.0L) * (2 * j + 1) / (4.0L * p));
+    const double u = (double)(x * x * near_scale(R));
+    unsigned long long b;
+    std::memcpy(&b, &u, sizeof(b));
+    b &= ~1ull;
+    double v;
+    std::memcpy(&v, &b, sizeof(v));
+    return v;
+}
+
+// The power series of series_comp (hbem_radial.hip) in y = x^2 / 64, A&S 9.1.10-9.1.13:
+// J0, J1 / x, the entire part of Y0 and that of Y1 over x; doubles, then residuals.
+std::vector<double> entire_series() {
+    constexpr int n = hbem::kSeriesDeg + 1;
+    const long double g = 0.57721566490153286060651209008240243L, pi = acosl(-1.0L);
+    std::vector<double> out(8 * n);
+    long double a = 1.0L, b = 0.5L, h = 0.0L;            // (-16)^k / k!^2, half of (-16)^k / (k! (k + 1)!), H_k
+    for (int k = 0; k < n; ++k) {
+        if (k > 0) {
+            a *= -16.0L / ((long double)k * k);
+            b *= -16.0L / ((long double)k * (k + 1));
+            h += 1.0L / k;
+        }
+        const long double c[4] = {a, b, 2.0L / pi * (g - h) * a, -b / pi * (2.0L * h + 1.0L / (k + 1) - 2.0L * g)};
+        for (int f = 0; f < 4; ++f) {
+            out[4 * k + f] = (double)c[f];
+            out[4 * (n + k) + f] = (double)(c[f] - (double)c[f]);
+        }
+    }
+    return out;
+}
+
 // Points and coefficient tables of tier t (kTiers + t: at the separated pairs'
 // tolerance), built on first use (null: a band would need more than kBandMaxP points).
 hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
@@ -556,7 +593,7 @@ hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
     const double tol = t >= hbem_geometry::kTiers ? kBandTolFar : kBandTol;
     const double kmax = kTierEdge[t % hbem_geometry::kTiers] / g->dmax;
     std::vector<hbem::Band> bands(r.nbands);
-    std::vector<double> cosv;
+    std::vector<double> cosv = entire_series();
     std::map<int, int> cosoff;
     std::map<int, std::vector<long double>> points;
     int pmax = 0, basis = 0;
@@ -576,20 +613,35 @@ hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
             return nullptr;
         }
         const int p = B.p;
+        if (b == 0) {
+            // the points' r^2 in units of a power of two, and the reciprocal
+            // products of their differences
+            const int P = hbem::near_stride(p);
+            B.cos = (int)cosv.size();
+            cosv.resize(B.cos + (size_t)P, -1.0);
+            cosv.resize(B.cos + 2 * (size_t)P, 0.0);
+            double* u = &cosv[B.cos];
+            for (int j = 0; j < p; ++j) u[j] = near_u(r.R, p, j);
+            for (int j = 0; j < p; ++j) {
+                long double v = 1.0L;
+                for (int k = 0; k < p; ++k)
+                    if (k != j) v *= (long double)u[j] - u[k];
+                u[P + j] = (double)(1.0L / v);
+            }
+        }
         auto it = cosoff.find(p);
-        if (it == cosoff.end()) {
+        if (b > 0 && it == cosoff.end()) {
             it = cosoff.emplace(p, (int)cosv.size()).first;
             for (int j = 0; j < p; ++j) points[p].push_back(cosl(acosl(-1.0L) * (2 * j + 1) / (2.0L * p)));
             for (int j = 0; j < p; ++j)
                 for (int q = 0; q < p; ++q)
                     cosv.push_back((q == 0 ? 1.0 : 2.0) / p * std::cos(M_PI * (double)((long long)q * (2 * j + 1) % (4 * p)) / (2.0 * p)));
         }
-        B.cos = it->second;
+        if (b > 0) B.cos = it->second;
         B.rad = (int)cosv.size();
         std::vector<double> res;              // the points' radii, then what rounding took from them
         for (int j = 0; j < p; ++j) {
-            const long double s = points[p][j];
-            const long double x = b == 0 ? B.a * sqrtl(0.5L * (s + 1.0L)) : B.c + B.a * s;
+            const long double x = b == 0 ? sqrtl(near_u(r.R, p, j) / (long double)near_scale(r.R)) : B.c + B.a * points[p][j];
             cosv.push_back((double)x);
             res.push_back((double)(x - (double)x));
         }
@@ -628,7 +680,7 @@ hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
     for (int cls = 0; cls < 2; ++cls) {
         const size_t cnt = ents[cls]->size() / 3 * (1 + cls);
         omom[cls] = place(cnt * pn * hbem::kRadialMoments * sizeof(double));
-        oext[cls] = place(cnt * 8 * sizeof(double));
+        oext[cls] = place(cnt * hbem::kRadialSums * sizeof(double));
     }
     char* plan = (char*)T.mem.get(need);
     HIPC(hipMemcpyAsync(plan, pk.bytes.data(), pk.bytes.size(), hipMemcpyHostToDevice, g->st));
@@ -640,14 +692,24 @@ hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
     T.ext = ext;
     const double* gtab = (const double*)g->d_gtab.p;
     const double *xg = (const double*)g->d_xg.p, *wg = (const double*)g->d_wg.p;
+    const double iS = near_scale(r.R);
+    // the quadrature rules' integrals of 1 over a panel pair, less one
+    long double c0 = 0.0L, c1 = 0.0L, gs = 0.0L;
+    for (int i = 0; i < g->nc; ++i) {
+        c0 += g->wc[i];
+        c1 += (long double)g->xc[i] * g->wc[i];
+    }
+    for (int i = 0; i < g->ns; ++i) gs += g->wg[i];
+    const double curl_s = (double)(2.0L * c0 * c1 - 1.0L), curl_g = (double)(gs * gs - 1.0L);
     for (int cls = 0; cls < 2; ++cls)
         hbem::launch_radial_moments(cls, (const int*)(plan + oe[cls]), (int)ents[cls]->size() / 3,
                                     (const double*)g->d_panels.p, (const double*)g->d_coefs.p, (const double*)g->d_xc.p,
-                                    (const double*)g->d_wc.p, g->nc, r.R, pn, (double*)(plan + omom[cls]),
+                                    (const double*)g->d_wc.p, g->nc, r.R, iS, dc + bands[0].cos, pn, (double*)(plan + omom[cls]),
                                     (double*)(plan + oext[cls]), g->st);
     hbem::launch_radial_near(r.d_near, (int)r.near.size(), dt, db, pn, gtab, xg, wg, g->N, g->ns,
                              r.flags, (const double*)(plan + omom[0]), (const double*)(plan + oext[0]),
-                             (const double*)(plan + omom[1]), (const double*)(plan + oext[1]), dc, tab, ext, g->st);
+                             (const double*)(plan + omom[1]), (const double*)(plan + oext[1]), dc, iS, curl_s, curl_g, tab,
+                             ext, g->st);
     hbem::launch_radial_far(r.recs, dt, r.ntile_near, r.ntile - r.ntile_near, db, pmax, gtab, xg, wg, g->N,
                             g->ns, r.flags, dc, tab, g->st);
     HIPC(hipGetLastError());

@@ -325,7 +325,12 @@ __device__ inline void hankel01_cplx(cdbl z, cdbl& h0, cdbl& h1) {
 // kEntireMax: the ascending series (A&S 9.1.10-9.1.13) for |z| <= 2; above it J
 // by Miller's backward recurrence J_{n-1} = (2n / z) J_n - J_{n+1} normalised by
 // e^{-iz} = J0 + 2 sum (-i)^n J_n (A&S 9.1.27, 9.1.41-45), whose left side is not
-// small for Im z >= 0, and the parts from H0, H1.
+// small for Im z >= 0, and C, D from the same J_n by Neumann's series (A&S 9.1.88-89),
+// from |z| = 8 on, where the continued fraction of H0, H1 is good to 1e-15, from these,
+// so that J's error drops out again where the logarithm is added.
+// The recurrence multiplies by the rounded reciprocal of z, so it runs at z + e, e the
+// reciprocal's residual: everything is formed there and carried back by the
+// derivatives (9.1.28); without that the phase is off by |z| units of rounding.
 constexpr double kEntireMax = 200.0;
 __device__ inline void bessel_entire_cplx(cdbl z, cdbl& j0, cdbl& c0, cdbl& j1, cdbl& c1) {
     if (cabsd(z) <= 2.0) {
@@ -349,27 +354,49 @@ __device__ inline void bessel_entire_cplx(cdbl z, cdbl& j0, cdbl& c0, cdbl& j1, 
         return;
     }
     const cdbl zi = recip(z);
+    // 1 - z zi, exact to its own rounding
+    const double p = z.x * zi.x, q = z.y * zi.y, g = z.x * zi.y, h = z.y * zi.x;
+    const cdbl rs = mk(((1.0 - p) + q) + (fma(z.y, zi.y, -q) - fma(z.x, zi.x, -p)),
+                       -((g + h) + (fma(z.x, zi.y, -g) + fma(z.y, zi.x, -h))));
+    const cdbl e = z * rs;                               // the recurrence's argument minus z
     int n = 2 * ((int)(0.5 * cabsd(z)) + 16 + (int)(2.0 * cbrt(cabsd(z))) * 2);
     cdbl hi = mk(0.0, 0.0), lo = mk(1e-60, 0.0), sum = mk(0.0, 0.0);   // J_{n+1}, J_n
+    cdbl sy0 = mk(0.0, 0.0), sy1 = mk(0.0, 0.0);         // sum (-1)^{k+1} J_2k / k, sum (-1)^{k+1} (2k + 1) J_{2k+1} / (k (k + 1))
     for (; n > 0; --n) {
         // (-i)^n = 1, -i, -1, i for n mod 4 = 0 .. 3
         const int m = n & 3;
         sum = sum + (m == 0 ? lo : (m == 1 ? mk(lo.y, -lo.x) : (m == 2 ? mk(-lo.x, -lo.y) : mk(-lo.y, lo.x))));
+        const int k = n >> 1;
+        const double s = (k & 1) ? 1.0 : -1.0;
+        if (n & 1) sy1 = sy1 + (k ? s * (2 * k + 1) / ((double)k * (k + 1)) : 0.0) * lo;
+        else sy0 = sy0 + (s / k) * lo;
         const cdbl nx = (2.0 * n) * (zi * lo) - hi;
         hi = lo;
         lo = nx;
     }
     const cdbl w = mk(z.y, -z.x);                        // -iz
-    const cdbl sc = cdiv(cexpd(w), lo + 2.0 * sum);
-    j0 = sc * lo;
-    const cdbl J1 = sc * hi;
-    j1 = J1 * zi;
-    cdbl h0, h1;
-    hankel01_cplx(z, h0, h1);
-    const cdbl y0 = mk(h0.y - j0.y, j0.x - h0.x), y1 = mk(h1.y - J1.y, J1.x - h1.x);   // -i (H - J)
-    const cdbl L2 = kTwoOverPi * clogd(0.5 * z);
-    c0 = y0 - L2 * j0;
-    c1 = zi * (y1 - L2 * J1 + kTwoOverPi * zi);
+    const cdbl ex = cexpd(w), sc = cdiv(ex - mk(-e.y, e.x) * ex, lo + 2.0 * sum);   // e^{-i (z + e)}
+    const cdbl a0 = sc * lo, a1 = sc * hi;               // J0, J1 at z + e
+    const cdbl b0 = kTwoOverPi * (kEuler * a0 + 2.0 * (sc * sy0));
+    const cdbl b1 = kTwoOverPi * (zi * (mk(1.0, 0.0) - a0) + (kEuler - 1.0) * a1 + sc * sy1);   // z D
+    // back to z: J0' = -J1, C' = -z D + (2/pi) (1 - J0) / z, J1' = J0 - J1 / z, (z D)' =
+    // C - D - (2/pi) J1 / z
+    j0 = a0 + e * a1;
+    const cdbl d1 = a0 - zi * a1, J1 = a1 - e * d1;
+    j1 = zi * J1;
+    j1 = j1 + rs * j1;                                   // (with the residual of 1 / z)
+    if (cabsd(z) >= 8.0) {
+        cdbl h0, h1;
+        hankel01_cplx(z, h0, h1);
+        const cdbl y0 = mk(h0.y - j0.y, j0.x - h0.x), y1 = mk(h1.y - J1.y, J1.x - h1.x);   // -i (H - J)
+        const cdbl L2 = kTwoOverPi * clogd(0.5 * z);
+        c0 = y0 - L2 * j0;
+        c1 = zi * (y1 - L2 * J1 + kTwoOverPi * zi);
+        return;
+    }
+    c0 = b0 + e * (b1 - kTwoOverPi * (zi * (mk(1.0, 0.0) - a0)));
+    c1 = zi * (b1 - e * (b0 - zi * b1 - kTwoOverPi * (zi * a1)));
+    c1 = c1 + rs * c1;
 }
 
 // ---------------------------------------------------------------------------

@@ -64,8 +64,9 @@ void launch_pad_identity(cdbl* T, int n, int ld, int nb, hipStream_t st);
 constexpr int kBandMaxP = 200;   // most points of a band (320 bytes of LDS each while its tables are built)
 constexpr int kRecValues = 5;    // values of a record and order (6 with the quirk)
 // A distance band: its interval is [c - a, c + a] (near band, band 0: [0, a]);
-// p points, their basis at record offset `basis`, the weights (2 - delta_q0) / p
-// T_q(s_j) of their transform at costab + cos, [j][q], their radii at costab + rad.
+// p points, their basis at record offset `basis`, at costab + cos the weights (2 -
+// delta_q0) / p T_q(s_j) of their transform, [j][q] (near band: what its Lagrange
+// weights take, see hbem_radial.hip), their radii at costab + rad.
 struct Band {
     double c, a;
     int p, basis, cos, rad;
@@ -92,6 +93,9 @@ struct RadialParams {
     cdbl* basis;
     cdbl* out;
 };
+// entries of the near band's point tables: a multiple of 32, six at least beyond p
+__host__ __device__ constexpr int near_stride(int p) { return (p + 37) & ~31; }
+constexpr int kSeriesDeg = 26;         // of the power series at the start of costab (see series_comp)
 int band_order(double c, double a, double kmax, double tol, bool near);
 constexpr int kBandOutside = 0xffff;   // a pair whose distances leave every band's interval
 void launch_radial_band(const double* gtab, int N, int ns, int npairs, double R, double first, double step, double width,
@@ -101,14 +105,17 @@ void launch_radial_far(const int* recs, const BandTile* tiles, int tile0, int nt
                        const double* gtab, const double* xg, const double* wg, int N, int ns, const unsigned char* flags,
                        const double* costab, double* tab, hipStream_t st);
 // moments of the cnt singular pairs of class cls: mom [pair][half][p][34], ext
-// [pair][half][8], two halves for adjacent pairs
+// [pair][half][25], two halves for adjacent pairs; pts, iS: the near band's points and
+// the scale of their u = r^2 iS
 void launch_radial_moments(int cls, const int* ent, int cnt, const double* panels, const double* coefs, const double* xc,
-                           const double* wc, int nc, double R, int p, double* mom, double* ext, hipStream_t st);
-constexpr int kRadialMoments = 34;
+                           const double* wc, int nc, double R, double iS, const double* pts, int p, double* mom,
+                           double* ext, hipStream_t st);
+constexpr int kRadialMoments = 34, kRadialSums = 25;
 void launch_radial_near(const RadialNear* ent, int nent, const BandTile* tiles, const Band* bands, int p,
                         const double* gtab, const double* xg, const double* wg, int N, int ns, const unsigned char* flags,
                         const double* mom_c, const double* ext_c, const double* mom_a, const double* ext_a,
-                        const double* costab, double* tab, double* ext, hipStream_t st);
+                        const double* costab, double iS, double curl_s, double curl_g, double* tab, double* ext,
+                        hipStream_t st);
 // basis of all bands (at most pmax points each) for the group
 void launch_band_basis(const RadialParams& P, bool diff, const Band* bands, int nbands, int pmax, const double* costab,
                        hipStream_t st);

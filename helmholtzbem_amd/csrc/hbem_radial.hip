@@ -26,7 +26,10 @@
 //               without ln x and 1/x -- are entire in r^2, so the transposition
 //               on [0, R^2] of the coefficients and of the coefficients times
 //               ln(r / R), plus the sums of c / r^2 and of c, reproduces the
-//               (singular) quadrature sums (k_radial_near).
+//               (singular) quadrature sums (k_radial_near).  The functions span
+//               orders of magnitude over [0, R], so every coefficient has to be
+//               right to its own last digits: the nodes' Lagrange weights are
+//               formed from the differences r^2 - r_j^2 (near_weight).
 //
 // The points being the band's, one Hankel pair per point and kappa serves every
 // pair of the band (k_band_basis), and the evaluation is a real x complex
@@ -271,24 +274,60 @@ __global__ __launch_bounds__(128) void k_radial_far(const int* __restrict__ recs
     }
 }
 
+// Lagrange weights of the near band's points at a node: l_j = prod_{k != j} (u -
+// u_k) / (u_j - u_k) with u = r^2 times a power of two (iS, near 1 / R^2), u_j doubles
+// (the points are defined by them) and lam[j] = prod_{k != j} 1 / (u_j - u_k); pts:
+// [u_j][lam], near_stride(p) each (-1 and 0 beyond p).  Products of differences, each
+// good to a few rounding errors of itself: the weights are too, also those a thousand
+// times smaller than the largest.  (Sums of Chebyshev polynomials, which the far bands
+// take, leave every weight with the rounding of the largest: at kappa d = 20, where
+// J1 / r falls by 10^4 over the band, K of a 64-panel polygon was off by 2.0e-13 and V
+// by 5.7e-14; these leave 3.8e-14 and 8.1e-15, the node loops 4.5e-14 and 2.2e-14.)
+// u's last bit is made one, up or down, and the points' are zero: no node names a point.
+__device__ __forceinline__ double near_node(double r2, double iS) {
+    const long long b = __double_as_longlong(r2 * iS);
+    return __longlong_as_double(b & 1 ? b : (b & 2 ? b - 1 : b + 1));
+}
+__device__ __forceinline__ double near_product(const double* __restrict__ pts, int p, double u) {
+    double w = 1.0;
+    for (int k = 0; k < p; ++k) w *= u - pts[k];
+    return w;
+}
+// 1 / d by two Newton steps
+__device__ __forceinline__ double fast_recip(double d) {
+    double y = __builtin_amdgcn_rcp(d);
+    y = fma(fma(-d, y, 1.0), y, y);
+    return fma(fma(-d, y, 1.0), y, y);
+}
+
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+// s + x, what rounding takes from it added to e (Knuth's TwoSum)
+__device__ __forceinline__ void two_sum(dbl4& s, dbl4 x, dbl4& e) {
+#pragma clang fp contract(off)
+    const dbl4 t = s + x, b = t - s;
+    e += (s - (t - b)) + (x - b);
+    s = t;
+}
+
 // Moments of the singular panel pairs for the near band (composite rules,
 // galerkin_builder.cpp:17-306, 553-832): local functionals of a pair (i, j), entry
 // q = a + 2 b: double layer test i (local a) / trial j (b) [0..3] and test j (a) /
 // trial i (b) [4..7], curl weight [8], weak part [9..12] and single layer [13..16]
-// test i (a) / trial j (b); times T_q(2 r^2 / R^2 - 1), and that times (2/pi)
-// ln(r / R) [17..33].  A pair's table serves the four pairs of hats over it;
-// adjacent pairs have one table per node half.  ext[8]: sums of c / r^2 of the
-// double-layer functionals.
+// test i (a) / trial j (b); times the Lagrange weight of point q, and that times
+// (2/pi) ln(r / R) [17..33].  A pair's table serves the four pairs of hats over it;
+// adjacent pairs have one table per node half.  ext[25]: sums of c / r^2 of the
+// double-layer functionals, then the sums of c of the seventeen (0 for the curl
+// weight, see k_radial_near).
 //
-// Sixteen of the seventeen functionals and the polynomials are the operands of a
+// Sixteen of the seventeen functionals and the weights are the operands of a
 // matrix product over the nodes, [16 x nodes] [nodes x 32 q] and the same with the
 // logarithm, so a wavefront evaluates 64 nodes (a lane each), hands them through
 // LDS to the lanes that v_mfma_f64_16x16x4f64 wants them in, and multiplies; the
 // curl weight and ext ride along as multiply-adds.  The product bounds it: one
 // workgroup (pair, half) reads nothing but its two panels.  Node tables in memory
 // read by one workgroup per two q took 0.55 ms for a 200-panel polygon's pairs
-// (order 11) and 5.2 ms for the 400-panel star's (order 16); this form 0.21 and
-// 1.95 ms.
+// (order 11) and 5.2 ms for the 400-panel star's (order 16); this form 0.29 and
+// 2.53 ms.
 constexpr int kMomLocal = kRadialMoments;
 constexpr int kMomQ = 32;                     // q per workgroup
 __device__ __forceinline__ void wave_lds_fence() {
@@ -299,9 +338,8 @@ template <int CLS>
 __global__ __launch_bounds__(256) void k_radial_moments(const int* __restrict__ ent, const double* __restrict__ panels,
                                                         const double* __restrict__ coefs,
                                                         const double* __restrict__ xc, const double* __restrict__ wc, int nc,
-                                                        double R, int p, double* __restrict__ mom,
-                                                        double* __restrict__ ext) {
-    typedef double dbl4 __attribute__((ext_vector_type(4)));
+                                                        double R, double iS, const double* __restrict__ pts, int p,
+                                                        double* __restrict__ mom, double* __restrict__ ext) {
     constexpr int LD = 17, WAVE = 64 * LD + 3 * 64;   // doubles of a wavefront
     __shared__ double sh[4 * WAVE];
     __shared__ int nz[3];
@@ -313,12 +351,13 @@ __global__ __launch_bounds__(256) void k_radial_moments(const int* __restrict__ 
     const double* gi = panels + 8 * (size_t)pi;
     const double* gj = panels + 8 * (size_t)pj;
     const double iR2 = 1.0 / (R * R);
+    const int P = near_stride(p);
     double* buf = sh + wv * WAVE;
     double *sln = buf + 64 * LD, *scu = sln + 64, *sir = scu + 64;
     if (tid < 3) nz[tid] = 0;
     __syncthreads();
-    dbl4 acc[2][2] = {};                      // [16 q][without, with the logarithm]
-    double curl[2][2] = {}, ex = 0.0;
+    dbl4 tot[2][2] = {}, err[2][2] = {};      // [16 q][without, with the logarithm]: sums and their rounding errors
+    double curl[2][2] = {}, ex = 0.0, ec = 0.0;
     bool any[3] = {false, false, false};
     for (int n0 = 64 * wv; n0 < nn; n0 += 256) {
         const int nd = n0 + lane < nn ? n0 + lane : nn - 1, a = nd / nc, b = nd - a * nc;
@@ -350,7 +389,7 @@ __global__ __launch_bounds__(256) void k_radial_moments(const int* __restrict__ 
         any[0] = any[0] || (in && !(fabs(vd) < kDblEps));
         any[1] = any[1] || (in && !(fabs(vt) < kDblEps));
         any[2] = any[2] || (in && !(fabs(td) < kDblEps));
-        const double u = r2 * iR2, x = fma(2.0, u, -1.0), x2 = x + x;
+        const double u = near_node(r2, iS);
         double* o = buf + lane * LD;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -361,7 +400,7 @@ __global__ __launch_bounds__(256) void k_radial_moments(const int* __restrict__ 
             o[8 + q] = w * (2.0 * td) * pw;
             o[12 + q] = w * (ni * nj) * pw;
         }
-        sln[lane] = r2 > 0.0 ? 0.5 * kTwoOverPi * log(u) : 0.0;
+        sln[lane] = r2 > 0.0 ? 0.5 * kTwoOverPi * log(r2 * iR2) : 0.0;
         scu[lane] = CLS == 1 ? w : 2.0 * w;
         sir[lane] = r2 > 0.0 ? 1.0 / r2 : 0.0;
         wave_lds_fence();
@@ -369,42 +408,43 @@ __global__ __launch_bounds__(256) void k_radial_moments(const int* __restrict__ 
 #pragma unroll
         for (int s = 0; s < 16; ++s) fa[s] = buf[(4 * s + lk) * LD + l16];
         wave_lds_fence();
-        double tp = x, tc = 1.0;
-        for (int q = 0; q < q0; ++q) {
-            const double tn = fma(x2, tc, -tp);
-            tp = tc;
-            tc = tn;
-        }
+        const double wp = near_product(pts, p, u);
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
-                o[q] = tc;
-                const double tn = fma(x2, tc, -tp);
-                tp = tc;
-                tc = tn;
+                const int j = q0 + 16 * c + q;
+                o[q] = (wp * pts[P + j]) * fast_recip(u - pts[j]);
             }
             wave_lds_fence();
+            dbl4 acc[2] = {};                 // this chunk's 64 nodes
 #pragma unroll
             for (int s = 0; s < 16; ++s) {
                 const double t = buf[(4 * s + lk) * LD + l16], tl = t * sln[4 * s + lk], cu = scu[4 * s + lk];
-                acc[c][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s], t, acc[c][0], 0, 0, 0);
-                acc[c][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s], tl, acc[c][1], 0, 0, 0);
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s], t, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s], tl, acc[1], 0, 0, 0);
                 curl[c][0] = fma(cu, t, curl[c][0]);
                 curl[c][1] = fma(cu, tl, curl[c][1]);
-                if (c == 0) ex = fma(fa[s], sir[4 * s + lk], ex);
+                if (c == 0) {
+                    ex = fma(fa[s], sir[4 * s + lk], ex);
+                    ec += fa[s];
+                }
             }
+            // a singular pair's nodes fill many chunks, whose running sum would leave
+            // the coefficients with three times the rounding error of one
+#pragma unroll
+            for (int g = 0; g < 2; ++g) two_sum(tot[c][g], acc[g], err[c][g]);
             wave_lds_fence();
         }
     }
     for (int k = 0; k < 3; ++k)
         if (any[k]) nz[k] = 1;
     // the four wavefronts' sums through LDS, added in order: [c][log][16][16],
-    // then curl [c][log][16], then ext [16]
+    // then curl [c][log][16], then the sums of c / r^2 [16] and of c [16]
     __syncthreads();
     for (int c = 0; c < 2; ++c)
         for (int g = 0; g < 2; ++g) {
-            for (int v = 0; v < 4; ++v) buf[((c * 2 + g) * 16 + 4 * v + lk) * 16 + l16] = acc[c][g][v];
+            for (int v = 0; v < 4; ++v) buf[((c * 2 + g) * 16 + 4 * v + lk) * 16 + l16] = tot[c][g][v] + err[c][g][v];
             double t = curl[c][g];
             t += __shfl_xor(t, 16, 64);
             t += __shfl_xor(t, 32, 64);
@@ -412,58 +452,68 @@ __global__ __launch_bounds__(256) void k_radial_moments(const int* __restrict__ 
         }
     ex += __shfl_xor(ex, 16, 64);
     ex += __shfl_xor(ex, 32, 64);
-    if (lk == 0) buf[1088 + l16] = ex;
+    ec += __shfl_xor(ec, 16, 64);
+    ec += __shfl_xor(ec, 32, 64);
+    if (lk == 0) {
+        buf[1088 + l16] = ex;
+        buf[1104 + l16] = ec;
+    }
     __syncthreads();
     auto total = [&](int k) { return (sh[k] + sh[WAVE + k]) + (sh[2 * WAVE + k] + sh[3 * WAVE + k]); };
     const bool f0 = nz[0] != 0, f1 = nz[1] != 0, f2 = nz[2] != 0;   // isArrayZero (galerkin_builder.cpp:470-495, 852-870)
     const size_t eh = (size_t)e * gridDim.y + h;
+    // functional kk of a table whose sixteen products lie at base, stride st
+    auto value = [&](int kk, int base, int st, double curl_sum) {
+        if (kk == 8) return curl_sum;
+        if (kk > 8) return kk > 12 || f2 ? total(base + st * (kk - 1)) : 0.0;
+        if (CLS == 1) return (kk < 4 ? f0 : f1) ? total(base + st * kk) : 0.0;
+        return kk < 4 ? (f0 ? total(base + st * kk) : 0.0) + (f1 ? total(base + st * (4 + kk)) : 0.0) : 0.0;
+    };
     for (int it = tid; it < kMomQ * kMomLocal; it += 256) {
-        const int q = it / kMomLocal, k = it - q * kMomLocal, kk = k % 17;
+        const int q = it / kMomLocal, k = it - q * kMomLocal, g = (q >> 4) * 2 + (k >= 17 ? 1 : 0);
         if (q0 + q >= p) break;
-        const int base = ((q >> 4) * 2 + (k >= 17 ? 1 : 0)) * 256 + (q & 15);
-        double v;
-        if (kk == 8) v = total(1024 + ((q >> 4) * 2 + (k >= 17 ? 1 : 0)) * 16 + (q & 15));
-        else if (kk > 8) v = kk > 12 || f2 ? total(base + 16 * (kk - 1)) : 0.0;
-        else if (CLS == 1) v = (kk < 4 ? f0 : f1) ? total(base + 16 * kk) : 0.0;
-        else v = kk < 4 ? (f0 ? total(base + 16 * kk) : 0.0) + (f1 ? total(base + 16 * (4 + kk)) : 0.0) : 0.0;
-        mom[(eh * p + q0 + q) * kMomLocal + k] = v;
+        mom[(eh * p + q0 + q) * kMomLocal + k] = value(k % 17, g * 256 + (q & 15), 16, total(1024 + g * 16 + (q & 15)));
     }
-    if (q0 == 0 && tid < 8) {
-        double v;
-        if (CLS == 1) v = (tid < 4 ? f0 : f1) ? total(1088 + tid) : 0.0;
-        else v = tid < 4 ? (f0 ? total(1088 + tid) : 0.0) + (f1 ? total(1088 + 4 + tid) : 0.0) : 0.0;
-        ext[eh * 8 + tid] = v;
-    }
+    if (q0 == 0 && tid < kRadialSums)
+        ext[eh * kRadialSums + tid] = tid < 8 ? value(tid, 1088, 1, 0.0) : value(tid - 8, 1104, 1, 0.0);
 }
 
 // Coefficients of the near band.  One wavefront per pair of hats: the Gauss nodes
-// of its general panel pairs over the lanes, the moments of its singular panel
-// pairs from their tables, then the transform to the points as for the far bands.
-// Table per point: the five coefficients, then those of (2/pi) ln(r / R); ext
-// [tile][7][16]: sum c / r^2 of the two double-layer functionals, the five sums
-// of c.
-__global__ __launch_bounds__(256) void k_radial_near(const RadialNear* __restrict__ ent, int nent,
+// of its general panel pairs over the lanes, six points at a time (60 register sums a
+// lane, totalled over the lanes together), and the moments of its singular panel
+// pairs from their tables.  Table per point: the five coefficients, then those of
+// (2/pi) ln(r / R); ext [tile][7][16]: sum c / r^2 of the two double-layer
+// functionals, the five sums of c, for the curl part less one: the constant that its
+// first k-derivative takes from the 1 / x of H1, -2i / (pi kappa) of every panel pair,
+// cancels in the hats (record_W), but for the quadrature rules' own defect of the
+// integral of 1 (curl_s of the singular pairs', curl_g of the general ones), and its
+// rounding errors would not, 1 / (kappa h)^2 times the entry's.  The far bands drop it
+// too (k_band_eval).
+__global__ __launch_bounds__(128) void k_radial_near(const RadialNear* __restrict__ ent, int nent,
                                                      const BandTile* __restrict__ tiles, const Band* __restrict__ bands,
                                                      const double* __restrict__ gtab, const double* __restrict__ xg,
                                                      const double* __restrict__ wg, int N, int ns,
                                                      const unsigned char* __restrict__ flags,
                                                      const double* __restrict__ mom_c, const double* __restrict__ ext_c,
                                                      const double* __restrict__ mom_a, const double* __restrict__ ext_a,
-                                                     const double* __restrict__ costab, double* __restrict__ tab,
-                                                     double* __restrict__ ext, int pmax) {
+                                                     const double* __restrict__ costab, double iS, double curl_s,
+                                                     double curl_g, double* __restrict__ tab, double* __restrict__ ext, int pmax, int cache) {
     constexpr int QC = 6;
-    extern __shared__ double mu_s[];          // [4 wavefronts][pmax][10]
+    extern __shared__ double mu_s[];          // [2 wavefronts]([pmax][10], [cache]{product, log} of the nodes)
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int x = blockIdx.x * 4 + wv;        // the grid covers the tiles' 16 pairs each, four a workgroup
+    const int x = blockIdx.x * 2 + wv;        // the grid covers the tiles' 16 pairs each, two a workgroup
     const int tile = x >> 4, row = x & 15;
-    double* mu = mu_s + (size_t)wv * pmax * 10;
+    double* mu = mu_s + (size_t)wv * (pmax * 10 + 2 * cache);
+    double* nodes = mu + pmax * 10;           // (a lane reads what it wrote)
     const BandTile bt = tiles[tile];
     const Band bd = bands[bt.band];
     const int p = bd.p, nn = ns * ns;
     const bool live = x < nent;               // else the padding of the last tile
     const RadialNear en = ent[live ? x : 0];
     const double iR2 = 1.0 / (bd.a * bd.a);   // near band: a = R
-    double ex[2] = {0.0, 0.0};
+    const double* pts = costab + bd.cos;
+    const int P = near_stride(p);
+    double ex[7] = {};                        // sums of c / r^2 (double layer), of c (not curl)
     for (int q0 = 0; q0 < p; q0 += QC) {
         double s[64];
 #pragma unroll
@@ -475,29 +525,38 @@ __global__ __launch_bounds__(256) void k_radial_near(const RadialNear* __restric
                 const int i = nd / ns, j = nd - i * ns;
                 double c[5];
                 const double r2 = gauss_node(pn, i, j, gtab, ns, xg, wg, c);
-                const double u = r2 * iR2, v = fma(2.0, u, -1.0), v2 = v + v;
-                const double lr = r2 > 0.0 ? 0.5 * kTwoOverPi * log(u) : 0.0;
-                if (q0 == 0 && r2 > 0.0) {
-                    ex[0] += c[0] / r2;
-                    ex[1] += c[1] / r2;
+                const double u = near_node(r2, iS);
+                double wp, lr;
+                const int at = ab * nn + nd;
+                if (q0 == 0 || !cache) {
+                    lr = r2 > 0.0 ? 0.5 * kTwoOverPi * log(r2 * iR2) : 0.0;
+                    wp = near_product(pts, p, u);
+                    if (cache) {
+                        nodes[2 * at] = wp;
+                        nodes[2 * at + 1] = lr;
+                    }
+                } else {
+                    wp = nodes[2 * at];
+                    lr = nodes[2 * at + 1];
                 }
-                double tp = v, tc = 1.0;
-                for (int q = 0; q < q0; ++q) {
-                    const double tn = fma(v2, tc, -tp);
-                    tp = tc;
-                    tc = tn;
+                if (q0 == 0) {
+                    if (r2 > 0.0) {
+                        ex[0] += c[0] / r2;
+                        ex[1] += c[1] / r2;
+                    }
+#pragma unroll
+                    for (int g = 0; g < 5; ++g)
+                        if (g != 2) ex[2 + g] += c[g];
                 }
 #pragma unroll
                 for (int q = 0; q < QC; ++q) {
-                    const double tl = tc * lr;
+                    const int k = q0 + q;     // < P, lam 0 beyond p
+                    const double t = (wp * pts[P + k]) * fast_recip(u - pts[k]), tl = t * lr;
 #pragma unroll
                     for (int g = 0; g < 5; ++g) {
-                        s[q * 10 + g] = fma(tc, c[g], s[q * 10 + g]);
+                        s[q * 10 + g] = fma(t, c[g], s[q * 10 + g]);
                         s[q * 10 + 5 + g] = fma(tl, c[g], s[q * 10 + 5 + g]);
                     }
-                    const double tn = fma(v2, tc, -tp);
-                    tp = tc;
-                    tc = tn;
                 }
             }
         }
@@ -505,7 +564,7 @@ __global__ __launch_bounds__(256) void k_radial_near(const RadialNear* __restric
         if (lane < QC * 10 && q0 * 10 + lane < p * 10) mu[q0 * 10 + lane] = s[0];
     }
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
+    for (int g = 0; g < 7; ++g)
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) ex[g] += __shfl_xor(ex[g], o, 64);
     __syncthreads();
@@ -521,38 +580,35 @@ __global__ __launch_bounds__(256) void k_radial_near(const RadialNear* __restric
         // one panel: entry (0, 1) = entry (1, 0) (galerkin_builder.cpp:571-573, 744-746)
         return (g == 3 ? 9 : 13) + (coi ? (q == 2 ? 1 : q) : (rev ? qt : q));
     };
-    if (live) {
-        for (int it = lane; it < p * 10; it += 64) {
-            const int q = it / 10, g = it - 10 * q, g5 = g % 5;
-            double v = mu[it];
-            for (int ab = 0; ab < 4; ++ab) {
-                const int cls = en.type[ab] & 3, e = en.type[ab] >> 2;
-                if (cls == 3 || (g5 == 2 && ab != 3)) continue;
-                const int k = q * kMomLocal + (g >= 5 ? 17 : 0) + local(ab, g5);
-                const size_t st = (size_t)p * kMomLocal;
-                v += cls == 0 ? mom_c[e * st + k] : mom_a[2 * e * st + k] + mom_a[(2 * e + 1) * st + k];
-            }
-            mu[it] = v;
-        }
-    }
-    __syncthreads();
     double* out = tab + bt.off;
-    const double* ct = costab + bd.cos;
     for (int it = lane; it < p * 10; it += 64) {
-        const int j = it / 10, g = it - 10 * j;
-        double v = 0.0;
-        for (int q = 0; q < p; ++q) v = fma(ct[j * p + q], mu[q * 10 + g], v);
+        const int j = it / 10, g = it - 10 * j, g5 = g % 5;
+        double v = mu[it];
+        for (int ab = 0; ab < 4 && live; ++ab) {
+            const int cls = en.type[ab] & 3, e = en.type[ab] >> 2;
+            if (cls == 3 || (g5 == 2 && ab != 3)) continue;
+            const int k = j * kMomLocal + (g >= 5 ? 17 : 0) + local(ab, g5);
+            const size_t st = (size_t)p * kMomLocal;
+            v += cls == 0 ? mom_c[e * st + k] : mom_a[2 * e * st + k] + mom_a[(2 * e + 1) * st + k];
+        }
         out[tile_elem(j, 10, g, row)] = v;
     }
     if (lane < 7) {
-        double v = lane < 2 ? (lane == 0 ? ex[0] : ex[1]) : mu[lane - 2];
-        if (lane < 2 && live)
-            for (int ab = 0; ab < 4; ++ab) {
-                const int cls = en.type[ab] & 3, e = en.type[ab] >> 2;
-                const int k = local(ab, lane);
-                if (cls != 3)
-                    v += cls == 0 ? ext_c[(size_t)e * 8 + k] : ext_a[(size_t)e * 16 + k] + ext_a[(size_t)e * 16 + 8 + k];
+        double v = 0.0;
+#pragma unroll
+        for (int g = 0; g < 7; ++g)
+            if (lane == g) v = ex[g];
+        for (int ab = 0; ab < 4 && live; ++ab) {
+            const int cls = en.type[ab] & 3, e = en.type[ab] >> 2;
+            if (lane == 4) {
+                if (ab == 3) v = cls == 3 ? curl_g : curl_s;
+                continue;
             }
+            if (cls == 3) continue;
+            const int k = lane < 2 ? local(ab, lane) : 8 + local(ab, lane - 2);
+            const size_t st = kRadialSums;
+            v += cls == 0 ? ext_c[e * st + k] : ext_a[2 * e * st + k] + ext_a[(2 * e + 1) * st + k];
+        }
         ext[((size_t)tile * 7 + lane) * 16 + row] = v;
     }
 }
@@ -569,24 +625,26 @@ __global__ __launch_bounds__(256) void k_radial_near(const RadialNear* __restric
 // doubles r_j and kappa r_j leave out of the argument enters by the derivatives
 // (A&S 9.1.27-28), as a phase kappa r of 100 rounded to 64 bits would put 1e-14 on
 // every pair of the band.
-// The four polynomials of horner4 by the compensated Horner scheme (Graillat,
-// Langlois and Louvet: each step's rounding errors, by fma and TwoSum, in a second
-// Horner recurrence).  Up to x = 8 the terms grow to 100 and cancel: plain Horner's
-// error of 1e-14 changes from point to point of a band, where the node loops
-// averaged it over a pair's nodes (V of the 400-panel star 2.9e-15 from theirs, 1e-16
-// at x > 8).
-template <int DEG>
-__device__ __forceinline__ void horner4_comp(ctab_ptr c, double z, double (&v)[4]) {
+// Up to x = 8 the entire parts A = J0, B = J1 / x, C, D of Y0 and Y1 by their power
+// series in y = x^2 / 64 (A&S 9.1.10-9.1.13), whose terms grow to 100 and cancel: by the
+// compensated Horner scheme (Graillat, Langlois and Louvet: each step's rounding errors,
+// by fma and TwoSum, in a second Horner recurrence), the coefficients in two doubles.
+// ser: [kSeriesDeg + 1][A, B, C, D], then the residuals.
+__device__ __forceinline__ void series_comp(const double* __restrict__ ser, double z, double (&v)[4]) {
 #pragma clang fp contract(off)
-    double e[4] = {0.0, 0.0, 0.0, 0.0};
+    const double* lo = ser + 4 * (kSeriesDeg + 1);
+    double e[4];
 #pragma unroll
-    for (int f = 0; f < 4; ++f) v[f] = c[4 * DEG + f];
-    for (int i = DEG - 1; i >= 0; --i) {
+    for (int f = 0; f < 4; ++f) {
+        v[f] = ser[4 * kSeriesDeg + f];
+        e[f] = lo[4 * kSeriesDeg + f];
+    }
+    for (int i = kSeriesDeg - 1; i >= 0; --i) {
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
-            const double a = c[4 * i + f], p = v[f] * z, pe = fma(v[f], z, -p);
+            const double a = ser[4 * i + f], p = v[f] * z, pe = fma(v[f], z, -p);
             const double s = p + a, t = s - p, se = (p - (s - t)) + (a - t);
-            e[f] = fma(e[f], z, pe + se);
+            e[f] = fma(e[f], z, (pe + se) + lo[4 * i + f]);
             v[f] = s;
         }
     }
@@ -609,7 +667,17 @@ __global__ __launch_bounds__(256) void k_band_basis(RadialParams P, const Band* 
         const cdbl d = mk(fma(r, kap.x, -z.x) + dr * kap.x, fma(r, kap.y, -z.y) + dr * kap.y);
         if (b > 0) {
             cdbl h0, h1;
-            hankel01_cplx(z, h0, h1);
+            if (cabsd(z) < 8.0) {
+                // (the continued fraction is slow next to |z| = 2 and leaves 2e-15)
+                cdbl c0, c1;
+                bessel_entire_cplx(z, h0, c0, h1, c1);
+                const cdbl L2 = kTwoOverPi * clogd(0.5 * z), y0 = c0 + L2 * h0;
+                const cdbl y1 = z * (c1 + L2 * h1) - kTwoOverPi * recip(z), J1 = z * h1;
+                h0 = mk(h0.x - y0.y, h0.y + y0.x);
+                h1 = mk(J1.x - y1.y, J1.y + y1.x);
+            } else {
+                hankel01_cplx(z, h0, h1);
+            }
             o[0] = h0 - d * h1;
             o[nslots] = h1 + d * (h0 - cdiv(h1, z));
             return;
@@ -639,7 +707,7 @@ __global__ __launch_bounds__(256) void k_band_basis(RadialParams P, const Band* 
         // argument: (x^2 - fl(x^2)) / (2 x)
         const double x2 = x * x, t = (d + 0.5 * fma(x, x, -x2) * xi) * xi;
         double v[4];
-        horner4_comp<HBEM_SMALL_DEG>(bessel_table() + HBEM_TAB_SMALL, x2 * (1.0 / 64.0), v);
+        series_comp(costab, x2 * (1.0 / 64.0), v);
         A = fma(-x2 * t, v[1], v[0]);
         B = fma(t, fma(-2.0, v[1], v[0]), v[1]);
         C = fma(kTwoOverPi * t, 1.0 - v[0], fma(-x2 * t, v[3], v[2]));
@@ -670,8 +738,6 @@ __global__ __launch_bounds__(256) void k_band_basis(RadialParams P, const Band* 
     o[0] = mk(A, fma(lR, A, C));
     o[nslots] = mk(kap * B, kap * fma(lR, B, Dd));
 }
-
-typedef double dbl4 __attribute__((ext_vector_type(4)));
 
 // One complex sum of four pairs (the accumulator rows of a lane).
 struct Sum4 {
@@ -744,6 +810,13 @@ __device__ __forceinline__ void load_slot(const RadialParams& P, int q, SlotScal
     s.nk2h = (-1.0) * s.k2h;
     s.nkap2 = -2.0 * s.kap;
     s.sqc = sqrt(s.c);
+}
+
+// sum v of s plus i k e
+__device__ __forceinline__ void add_i(Sum4& s, int v, double k, double e) { s.im[v] = fma(k, e, s.im[v]); }
+__device__ __forceinline__ void add_i(Sum4& s, int v, cdbl k, double e) {
+    s.re[v] = fma(-k.y, e, s.re[v]);
+    s.im[v] = fma(k.x, e, s.im[v]);
 }
 
 // Sums of NF functionals starting at f0 (all of one kind: KIND 0 double layer,
@@ -819,14 +892,7 @@ __device__ __forceinline__ void band_sums(const double* __restrict__ a, int f0, 
                 for (int v = 0; v < 4; ++v) {
                     const double e = ex[(size_t)(KIND == 0 && t == 0 ? f0 + f : 2 + f0 + f) * 16 + 4 * v + lk];
 #pragma unroll
-                    for (int h = 0; h < H; ++h) {
-                        if constexpr (CN) {
-                            S[t][f][h].re[v] = fma(-ikap[h].y, e, S[t][f][h].re[v]);
-                            S[t][f][h].im[v] = fma(ikap[h].x, e, S[t][f][h].im[v]);
-                        } else if constexpr (NEAR) {
-                            S[t][f][h].im[v] = fma(ikap[h], e, S[t][f][h].im[v]);
-                        }
-                    }
+                    for (int h = 0; h < H; ++h) add_i(S[t][f][h], v, ikap[h], e);
                 }
         }
     }
@@ -898,6 +964,13 @@ __global__ __launch_bounds__(256) void k_band_eval(RadialParams P, const int* __
     {
         Sum4 S[D + 1][2][H];
         band_sums<D, DIFF, NEAR, K, 1, 2>(a, 2, bs, nslots, cc, P.ncolg + cc, rj, bd.p, ex, ikap, bl, S);
+        if (D >= 1 && !NEAR) {
+            // the curl part's constant (see k_radial_near)
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) add_i(S[D >= 1 ? 1 : 0][0][h], v, ikap[h], -1.0);
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
@@ -1188,22 +1261,31 @@ void launch_radial_far(const int* recs, const BandTile* tiles, int tile0, int nt
 }
 
 void launch_radial_moments(int cls, const int* ent, int cnt, const double* panels, const double* coefs, const double* xc,
-                           const double* wc, int nc, double R, int p, double* mom, double* ext, hipStream_t st) {
+                           const double* wc, int nc, double R, double iS, const double* pts, int p, double* mom,
+                           double* ext, hipStream_t st) {
     if (cnt <= 0) return;
     const dim3 g((unsigned)cnt, cls == 1 ? 2 : 1, (unsigned)((p + kMomQ - 1) / kMomQ));
     if (cls == 1)
-        hipLaunchKernelGGL(k_radial_moments<1>, g, dim3(256), 0, st, ent, panels, coefs, xc, wc, nc, R, p, mom, ext);
+        hipLaunchKernelGGL(k_radial_moments<1>, g, dim3(256), 0, st, ent, panels, coefs, xc, wc, nc, R, iS, pts, p,
+                           mom, ext);
     else
-        hipLaunchKernelGGL(k_radial_moments<0>, g, dim3(256), 0, st, ent, panels, coefs, xc, wc, nc, R, p, mom, ext);
+        hipLaunchKernelGGL(k_radial_moments<0>, g, dim3(256), 0, st, ent, panels, coefs, xc, wc, nc, R, iS, pts, p,
+                           mom, ext);
 }
 
 void launch_radial_near(const RadialNear* ent, int nent, const BandTile* tiles, const Band* bands, int p,
                         const double* gtab, const double* xg, const double* wg, int N, int ns, const unsigned char* flags,
                         const double* mom_c, const double* ext_c, const double* mom_a, const double* ext_a,
-                        const double* costab, double* tab, double* ext, hipStream_t st) {
+                        const double* costab, double iS, double curl_s, double curl_g, double* tab, double* ext,
+                        hipStream_t st) {
     if (nent <= 0) return;
-    hipLaunchKernelGGL(k_radial_near, dim3((unsigned)((nent + 15) / 16 * 4)), dim3(256), 4 * p * 10 * sizeof(double), st,
-                       ent, nent, tiles, bands, gtab, xg, wg, N, ns, flags, mom_c, ext_c, mom_a, ext_a, costab, tab, ext, p);
+    // the nodes' products and logarithms are kept in LDS from the first points on
+    // where two wavefronts' fit in 64 KB (orders up to 20)
+    const size_t mu = (size_t)p * 10, nodes = (size_t)4 * ns * ns;
+    const int cache = 2 * (mu + 2 * nodes) * sizeof(double) <= 65536 ? (int)nodes : 0;
+    hipLaunchKernelGGL(k_radial_near, dim3((unsigned)((nent + 15) / 16 * 8)), dim3(128),
+                       2 * (mu + 2 * cache) * sizeof(double), st, ent, nent, tiles, bands, gtab, xg, wg, N, ns, flags, mom_c,
+                       ext_c, mom_a, ext_a, costab, iS, curl_s, curl_g, tab, ext, p, cache);
 }
 
 void launch_band_basis(const RadialParams& P, bool diff, const Band* bands, int nbands, int pmax, const double* costab,
