@@ -51,6 +51,8 @@ NC, Q = 2, 2
 MIXED_REFINE = 2            # FP64 refinement steps of the last solve of the randomized SVD
 MIXED_REFINE_INNER = 1      # ... and of the solves before it
 MIXED_TOL = 1e-8            # the mixed-precision bar: sigma within 1e-8 relative of FP64
+# (assembly_adjacent: the near band's products where the wavenumbers take the bands; a
+# phase without launches is null)
 PHASES = ("assembly_general", "assembly_adjacent", "assembly_coinciding", "lu", "form_T", "rsvd")
 
 
@@ -150,7 +152,7 @@ def run_workload(H, name, steps, warmup, mixed=False, bd=None, ref_sigma=None, f
         "config": {"workload": w["text"], "panels": N, "order": w["order"], "nk": w["nk"], "global_batch": w["nk"],
                    "parallelism": "single-gpu"},
         "panel_pair_evals_per_s": pairs_per_k * evals / asm_s if asm_s > 0 else None,
-        "phase_seconds_per_step": {ph: p[0] * 1e-3 / steps for ph, p in zip(PHASES, prof)},
+        "phase_seconds_per_step": {ph: p[0] * 1e-3 / steps if p[1] else None for ph, p in zip(PHASES, prof)},
         "lu_model_tflops": lu_tflops,
         "roofline_assembly": {"kernel": "k_band_eval<d=%d> (band functionals x Hankel basis, all pairs of hat functions, "
                                         "%d k)" % (der, w["nk"]),

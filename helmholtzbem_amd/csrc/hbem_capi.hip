@@ -1002,7 +1002,11 @@ cdbl* launch_records(const RecJob& J) {
                                    ext, J.st);
             if (J.prof)
                 g->plog.end(J.st, kProfGeneral, e0, 20.0 * (J.D + 1) * T.points * r.count * (J.diff ? 2.0 : 1.0));
+            if (J.prof) e0 = g->plog.begin(J.st);
             hbem::launch_band_eval(J.D, J.diff, true, P, recs, tiles, 0, R.ntile_near, bands, cs, tab, ext, J.st);
+            if (J.prof)
+                g->plog.end(J.st, kProfAdjacent, e0,
+                            (J.cplx ? 40.0 : 30.0) * (J.D + 1) * 16.0 * R.ntile_near * T.pnear * r.count * (J.diff ? 2.0 : 1.0));
         } else {
             launch_loops(J, r);
         }

@@ -282,14 +282,16 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
  * roofline figures.  enable != 0 clears and starts recording; the events are
  * only read by query (no host synchronisation inside the timed calls).  query
  * returns the accumulated milliseconds and launch count of phase `which`
- * (0 = general-pair assembly: the band products, or the node loops' general
- * kernel where a wavenumber takes them; 1 = adjacent-pair kernel, 2 =
- * coinciding-pair kernel, both of the node loops only; 3 = LU factorisation,
+ * (0 = general-pair assembly: the far bands' basis and products, or the node
+ * loops' general kernel where a wavenumber takes them; 1 = the near band's
+ * products, which hold the adjacent and coinciding pairs, or the node loops'
+ * adjacent-pair kernel; 2 = the node loops' coinciding-pair kernel, no launch
+ * where every wavenumber takes the bands; 3 = LU factorisation,
  * 4 = T formation, 5 = the randomized SVD stage after the LU, 6 = the LU's
  * matrix-core launches, its trailing and sub-panel updates) and the
- * algorithmic flop count (0: 2 x 5 (d + 1) x 2 per band point, pair of hat
- * functions and wavenumber slot for the band products; 0-2: the frozen FP64
- * model for the node loops; 3: 8 n^3 / 3 per matrix; 6: the 3M products'
+ * algorithmic flop count (0 and 1 for the band products: 20 (d + 1) and, with
+ * the logarithms, 30 (d + 1), complex 40 (d + 1), per point, pair of hat
+ * functions and wavenumber slot; 0-2: the frozen FP64 model for the node loops; 3: 8 n^3 / 3 per matrix; 6: the 3M products'
  * 6 m n k per update and matrix, in the precision of the factorisation; 0
  * where none is defined). */
 int hbem_profile_enable(hbem_geometry_t g, int enable);
