@@ -174,8 +174,7 @@ class BuilderData:
 
     def release_work(self):
         """Frees the device work buffers of this geometry's contexts (the
-        geometry and its node tables stay); the next call allocates them
-        again."""
+        geometry and its tables stay); the next call allocates them again."""
         for g in (self._geo, self._geo_noproj):
             if g is not None:
                 check(lib().hbem_geometry_release_work(g.h))

@@ -333,8 +333,7 @@ struct hbem_geometry {
     // device geometry
     DBuf d_panels, d_coefs, d_xg, d_wg, d_xc, d_wc, d_gtab;
     std::vector<int> aent;                 // adjacent panel pairs (i, j, swap), i > j
-    std::vector<double> disc;              // bounding disc of every panel: centre, radius
-    double dmax = 0.0;                     // largest disc diameter
+    double dmax = 0.0;                     // largest diameter of a panel's bounding disc
     // Panel pairs by class (coinciding, adjacent, general) with their node tables,
     // for the node-loop kernels; built on first use.
     struct Loops {
@@ -1268,10 +1267,10 @@ int hbem_geometry_create(const double* panels, int npanels, const double* coefs,
     // adjacent pairs (galerkin_builder.cpp:872-897; adjacency test 189-201)
     const double* cptr = g->coefs.empty() ? nullptr : g->coefs.data();
     std::vector<double> ends(4 * (size_t)N);
-    g->disc.resize(3 * (size_t)N);
+    std::vector<double> disc(3 * (size_t)N);   // bounding discs: centre, radius
     hbem::panel_endpoints(g->panels.data(), cptr, N, ends.data());
-    hbem::panel_bounds(g->panels.data(), cptr, N, g->disc.data());
-    for (int i = 0; i < N; ++i) g->dmax = std::max(g->dmax, 2.0 * g->disc[3 * (size_t)i + 2]);
+    hbem::panel_bounds(g->panels.data(), cptr, N, disc.data());
+    for (int i = 0; i < N; ++i) g->dmax = std::max(g->dmax, 2.0 * disc[3 * (size_t)i + 2]);
     const double tol = 100.0 * hbem::kDblEps;
     auto meet = [&](const double* a, const double* b) {
         return std::fabs(a[0] - b[0]) < tol && std::fabs(a[1] - b[1]) < tol && std::hypot(a[0] - b[0], a[1] - b[1]) < tol;

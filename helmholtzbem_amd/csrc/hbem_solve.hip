@@ -498,8 +498,6 @@ static __global__ void k_thin_out(const int* __restrict__ perm, int n, int nc, c
     else x[e] = v;
 }
 
-// one workgroup of kSolveThreads threads per matrix: pass 0 (L, or U^H) or
-// pass 1 (U, or L^H) over the panel [pb, pe)
 // Right-looking coupling of the unknowns [cb, ce) (one panel, staged in xs)
 // onto row i: w_i -= sum_j M(i, j) w_j, the sum in column order.  A thread per
 // row (consecutive rows: the loads run down the columns), LR column loads in
@@ -596,8 +594,8 @@ __device__ __forceinline__ void couple_left_quad(const F* M, int n, cdbl* w, int
         }
 }
 
-// One panel [pb, pe) of a pass, blocks 0 .. batch - 1 (one per matrix), and
-// beside it, in blocks batch + cwg b + k, a coupling that does not touch the
+// One panel [pb, pe) of a pass (0: L, or U^H; 1: U, or L^H), blocks 0 .. batch - 1
+// (one of kSolveThreads threads per matrix), and beside it, in blocks batch + cwg b + k, a coupling that does not touch the
 // panel: the unknowns [cb, ce) onto the rows [rb, re) of matrix b,
 // right-looking (a thread per row, 512 rows a block) or, for adj, left-looking
 // (a wavefront per four rows, 32 rows a block).  The coupling blocks take the

@@ -81,16 +81,15 @@ int hbem_init(int device);
  * (galerkin_builder.hpp:43-46, galerkin_builder.cpp:17-187;
  *  gen_sol_op.hpp:28, gen_sol_op.cpp:23-43).
  * Uploads the panels, builds the quadrature grids, classifies panel pairs
- * (coinciding / adjacent / general, galerkin_builder.cpp:189-201, 872-897),
- * precomputes the pair-node geometry on the device and, when proj != 0, the
- * mass matrix and the projection factor F = P^T L sqrt(D) of
+ * (coinciding / adjacent / general, galerkin_builder.cpp:189-201, 872-897) and
+ * computes, when proj != 0, the mass matrix and the projection factor F = P^T L sqrt(D) of
  * blockdiag(M, M^T).
  */
 int hbem_geometry_create(const double* panels, int npanels, const double* coefs, int ncoefs,
                          int order, int proj, int flags, hbem_geometry_t* out);
 int hbem_geometry_destroy(hbem_geometry_t g);
 /* Frees the context's per-call work buffers (local matrices, T, factor and
- * thin blocks; the geometry, node tables and projection factor stay); the
+ * thin blocks; the geometry, its tables and the projection factor stay); the
  * next call allocates them again.  For callers that keep many contexts alive.
  * (No counterpart in the reference, which allocates per call.) */
 int hbem_geometry_release_work(hbem_geometry_t g);
