@@ -33,6 +33,11 @@ sys.path.insert(0, HERE)
 PEAK_FP64_TFLOPS = 78.6     # MI355X dense FP64 (vector and matrix)
 PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense FP32 on the matrix cores
 
+# HBM bytes per launch of the far bands' products, averaged over the launches of a
+# sweep (rocprofv3 FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000, KiB per dispatch, scaled by
+# the counters' reading of a plain 1 GiB copy): profiles/k_band_eval_counters.txt,
+# k_cgemm32_sub_polygon2000_far_traffic.txt (128 k)
+TRAFFIC_BYTES = {"polygon2000": 2.3808e10, "star400": 2.55e9}
 # HBM bytes per launch of the LU's matrix-core updates, averaged over the 217
 # launches of one polygon2000 sweep (the same counters and factors; 4.268e11 B
 # per sweep against 3.900e11 B of algorithmic C, A and B traffic)
@@ -157,7 +162,7 @@ def run_workload(H, name, steps, warmup, mixed=False, bd=None, ref_sigma=None, f
         "roofline_assembly": {"kernel": "k_band_eval<d=%d> (band functionals x Hankel basis, all pairs of hat functions, "
                                         "%d k)" % (der, w["nk"]),
                               "bound": "fp64_mfma", "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
-                              "frac": achieved / PEAK_FP64_TFLOPS, "traffic": None,
+                              "frac": achieved / PEAK_FP64_TFLOPS, "traffic": TRAFFIC_BYTES.get(name),
                               "avg_launch_ms": avg_launch_s * 1e3, "launches": n_gen,
                               "flops_per_launch": fl_gen / max(n_gen, 1),
                               "seconds_per_step": ms_gen * 1e-3 / steps},

@@ -2014,7 +2014,7 @@ void sweep_run(hbem_geometry* g, const double* ks, int nk, double c_o, double c_
         if (d2sigma) {
             // randomized_svd::sv_der2's bordered system (randsvd.cpp:171-216) for
             // every k of the batch, on T_p formed explicitly: T again from the
-            // local matrices (T0 holds its LU factors), projected through the
+            // records (T0 holds its LU factors), projected through the
             // bordered matrix's storage.
             const int m2 = 2 * n;
             cdbl* Tp = g->w_Tp.as<cdbl>(nn * nb);
