@@ -1,5 +1,6 @@
 // hbem_capi.hip -- geometry contexts and the C-ABI of include/hbem.h.
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <complex>
 #include <cstdlib>
@@ -314,7 +315,6 @@ size_t usable_device_bytes(size_t held) {
 // Work space of an assembly call: the slots' tables and column lists ...
 struct RecBufs {
     DBuf tab;                                    // slots and columns, one upload
-    std::vector<std::unique_ptr<DBuf>> lslots;   // slot tables of the groups on the node loops
 };
 // ... and what the groups use in turn
 struct RecScratch {
@@ -762,11 +762,18 @@ hbem_geometry::Loops& node_loops(hbem_geometry* g) {
 // The tier of a column with |kappa| between lo and hi and Im kappa at most im, or -1
 // for the node loops: kappa = 0, beyond the last tier, or so far from the real
 // axis that J and iY of the near band, each of size e^{Im kappa r}, would leave
-// H with fewer digits (kNearImag: e^{2 Im kappa R} below 3).
-// cplx: it is evaluated as a complex one.
-constexpr double kNearImag = 0.5;
-int record_tier(hbem_geometry* g, double lo, double hi, double im, bool cplx) {
+// H with fewer digits (kNearImag: e^{2 Im kappa R} below 3).  cplx: it is evaluated as
+// a complex one.  sweep: of a sweep; the single matrices' calls at real wavenumbers take
+// the node loops from kappa dmax = 5 on (kBuilderEdge), where a panel holds most of a
+// wavelength and the tables' many points cost a context's first call far more than any
+// later call saves: made and called once, with the bands 400 panels at kappa dmax = 15
+// took 21.4 ms (node loops 12.5), 100 panels 2.4 (1.15); their second calls 0.84 (1.22) and
+// 0.22 (0.22).  At complex ones the loops are ten times as long (100 panels at 9 + 0.04 i:
+// 3.4 ms made and called once, with the bands 2.6).
+constexpr double kNearImag = 0.5, kBuilderEdge = 5.0;
+int record_tier(hbem_geometry* g, double lo, double hi, double im, bool cplx, bool sweep) {
     int t = lo > 0.0 ? tier_of(hi * g->dmax) : -1;
+    if (t >= 0 && !sweep && !cplx && kTierEdge[t] > kBuilderEdge) t = -1;
     if (t >= 0 && far_tolerance(g, t, cplx)) t += hbem_geometry::kTiers;
     if (t < 0 || !radial_tier(g, t)) return -1;
     if (im > 0.0 && (im * g->rad->R > kNearImag || hi * g->rad->R > hbem::kEntireMax)) return -1;
@@ -782,7 +789,7 @@ int record_tier(hbem_geometry* g, double lo, double hi, double im, bool cplx) {
 // tier; tier < 0: the node loops.
 struct RecGroup {
     int tier, start, count;
-    double *kap = nullptr, *kr = nullptr, *cv = nullptr, *kapi = nullptr, *kri = nullptr;   // node loops: the group's slots
+    const double *kap = nullptr, *kr = nullptr, *cv = nullptr, *kapi = nullptr, *kri = nullptr;   // node loops: the group's slots
     int nslots = 0;
 };
 // Values per order of the records of a call (see hbem_radial.hip).
@@ -792,7 +799,7 @@ struct RecJob {
     hbem_geometry* g = nullptr;
     RecScratch* w = nullptr;
     int D = 0, ncol = 0, nslot2 = 0, nv = 4;
-    bool diff = false, cplx = false, tdiff = false, prof = false;   // prof: time into the context's log
+    bool diff = false, cplx = false, tdiff = false, sweep = false, prof = false;   // prof: time into the context's log
     hipStream_t st = nullptr;
     const double *kap = nullptr, *kapi = nullptr, *kr = nullptr, *kri = nullptr, *cv = nullptr;
     const int* cols = nullptr;
@@ -801,9 +808,11 @@ struct RecJob {
 };
 
 // lanes per item of the node loops for ns slots: 0 = the paired-lane kernel
-// (32 wavenumbers x 2 nodes per wavefront), else groups of lanes per item
-void loop_lanes(int ns, bool cplx, bool tdiff, int& general, int& singular) {
-    general = cplx ? 16 : (ns >= 64 || tdiff ? 0 : (ns >= 16 ? 4 : 16));
+// (32 wavenumbers x 2 nodes per wavefront), else groups of lanes per item (in the
+// single matrices' calls one size, so that a matrix of a batch of fewer than 64 is the
+// one of a call of its own)
+void loop_lanes(int ns, bool cplx, bool tdiff, bool sweep, int& general, int& singular) {
+    general = cplx ? 16 : (ns >= 64 || tdiff ? 0 : (sweep && ns >= 16 ? 4 : 16));
     singular = (ns >= 64 || tdiff) && !cplx ? 0 : 64;
 }
 
@@ -841,7 +850,7 @@ void launch_loops(const RecJob& J, const RecGroup& r) {
     P.kapi = r.kapi;
     P.kri = r.kri;
     int Gg, Gs;
-    loop_lanes(r.nslots, J.cplx, J.tdiff, Gg, Gs);
+    loop_lanes(r.nslots, J.cplx, J.tdiff, J.sweep, Gg, Gs);
     const int which[3] = {kProfCoinciding, kProfAdjacent, kProfGeneral};
     for (int cls = 2; cls >= 0; --cls) {
         if (set.cnt[cls] == 0) continue;
@@ -870,11 +879,14 @@ void launch_loops(const RecJob& J, const RecGroup& r) {
 // inner slots then the outer, whose differences T is formed from.  tdiff: the
 // node loops take the paired-lane kernel in the difference layout whatever the
 // width (sweeps of >= 32 wavenumbers, so that a wavenumber's bits do not depend
-// on its batch).
+// on its batch).  sweep: see record_tier.  together: the columns are one system's and
+// take one way, that of the largest kappa.
 RecJob prepare_records(hbem_geometry* g, RecBufs& b, RecScratch& w, hipStream_t st, const std::vector<double>& kap,
                        const std::vector<double>& kr, const std::vector<double>& cv, int D, bool diff,
-                       const std::vector<double>& kapi = {}, const std::vector<double>& kri = {}, bool tdiff = false) {
+                       const std::vector<double>& kapi = {}, const std::vector<double>& kri = {}, bool sweep = false,
+                       bool tdiff = false, bool together = false) {
     RecJob J;
+    J.sweep = sweep;
     J.g = g;
     J.w = &w;
     J.st = st;
@@ -889,20 +901,26 @@ RecJob prepare_records(hbem_geometry* g, RecBufs& b, RecScratch& w, hipStream_t 
     J.nv = record_values(g, D);
     const bool quirk = J.nv != hbem::kRecValues;
     std::map<int, std::vector<int>> by;
+    double lo = 1e300, hi = 0.0, im = 0.0;
+    auto reach = [&](int q) {
+        const double m = J.cplx ? std::hypot(kap[q], kapi[q]) : std::fabs(kap[q]);
+        lo = std::min(lo, m);
+        hi = std::max(hi, m);
+        if (J.cplx) im = std::max(im, kapi[q]);
+    };
+    for (int q = 0; q < (int)kap.size() && together; ++q) reach(q);
     for (int c = 0; c < n; ++c) {
-        double lo = 1e300, hi = 0.0, im = 0.0;
-        for (int h = 0; h < (diff ? 2 : 1); ++h) {
-            const int q = c + h * n;
-            const double m = J.cplx ? std::hypot(kap[q], kapi[q]) : std::fabs(kap[q]);
-            lo = std::min(lo, m);
-            hi = std::max(hi, m);
-            if (J.cplx) im = std::max(im, kapi[q]);
+        if (!together) {
+            lo = 1e300;
+            hi = im = 0.0;
+            for (int h = 0; h < (diff ? 2 : 1); ++h) reach(c + h * n);
         }
-        by[quirk ? -1 : record_tier(g, lo, hi, im, J.cplx)].push_back(c);
+        by[quirk ? -1 : record_tier(g, lo, hi, im, J.cplx, sweep)].push_back(c);
     }
     std::vector<int> cols;
     size_t nL = 0, npart = 0, nbasis = 0;
-    size_t nl = 0;
+    Packed pk;
+    std::vector<std::array<size_t, 5>> places;   // of the groups' slot tables in pk
     for (auto& kv : by) {
         RecGroup r;
         r.tier = kv.first;
@@ -927,23 +945,20 @@ RecJob prepare_records(hbem_geometry* g, RecBufs& b, RecScratch& w, hipStream_t 
                     for (int c : kv.second) slot.push_back(c + h * n);
             }
             r.nslots = (int)slot.size();
-            auto table = [&](const std::vector<double>& v) -> double* {
-                if (v.empty()) return nullptr;
+            std::array<size_t, 5> at;
+            const std::vector<double>* tabs[5] = {&kap, &kr, &cv, &kapi, &kri};
+            for (int i = 0; i < 5; ++i) {
                 std::vector<double> x;
-                for (int q : slot) x.push_back(v[q]);
-                if (b.lslots.size() <= nl) b.lslots.push_back(std::make_unique<DBuf>());
-                return upload(*b.lslots[nl++], x, st);
-            };
-            r.kap = table(kap);
-            r.kr = table(kr);
-            r.cv = table(cv);
-            r.kapi = table(kapi);
-            r.kri = table(kri);
+                if (!tabs[i]->empty())
+                    for (int q : slot) x.push_back((*tabs[i])[q]);
+                at[i] = pk.add(x);
+            }
+            places.push_back(at);
             auto& set = node_loops(g);
             const size_t rows = (size_t)16 * (D + 1) * (J.tdiff ? r.count : r.nslots);
             nL = std::max(nL, rows * (size_t)g->npairs);
             int G[2];
-            loop_lanes(r.nslots, J.cplx, J.tdiff, G[0], G[1]);
+            loop_lanes(r.nslots, J.cplx, J.tdiff, J.sweep, G[0], G[1]);
             for (int cls = 0; cls < 3; ++cls) {
                 int chunk, nchunk;
                 loop_chunks(cls, cls == 2 ? G[0] : G[1], class_nodes(g, cls), chunk, nchunk);
@@ -952,7 +967,6 @@ RecJob prepare_records(hbem_geometry* g, RecBufs& b, RecScratch& w, hipStream_t 
         }
         J.groups.push_back(r);
     }
-    Packed pk;
     const std::vector<double>* tabs[5] = {&kap, &kr, &cv, &kapi, &kri};
     const double** dst[5] = {&J.kap, &J.kr, &J.cv, &J.kapi, &J.kri};
     size_t at[5];
@@ -962,6 +976,13 @@ RecJob prepare_records(hbem_geometry* g, RecBufs& b, RecScratch& w, hipStream_t 
     HIPC(hipMemcpyAsync(b.tab.p, pk.bytes.data(), pk.bytes.size(), hipMemcpyHostToDevice, st));
     for (int i = 0; i < 5; ++i) *dst[i] = tabs[i]->empty() ? nullptr : (const double*)(d + at[i]);
     J.cols = (const int*)(d + ocols);
+    size_t np = 0;
+    for (RecGroup& r : J.groups)
+        if (r.tier < 0) {
+            const std::array<size_t, 5>& p = places[np++];
+            const double** own[5] = {&r.kap, &r.kr, &r.cv, &r.kapi, &r.kri};
+            for (int i = 0; i < 5; ++i) *own[i] = tabs[i]->empty() ? nullptr : (const double*)(d + p[i]);
+        }
     J.obasis = al256((size_t)g->npairs * J.nv * (D + 1) * n * sizeof(cdbl));
     w.E.get(J.obasis + nbasis * sizeof(cdbl));
     if (nL) w.L.get(nL * sizeof(cdbl));
@@ -1016,8 +1037,8 @@ cdbl* launch_records(const RecJob& J) {
 // Records of a call on the context's own buffers and stream.
 cdbl* assemble_records(hbem_geometry* g, const std::vector<double>& kap, const std::vector<double>& kr,
                        const std::vector<double>& cv, int D, bool diff, const std::vector<double>& kapi = {},
-                       const std::vector<double>& kri = {}, bool tdiff = false) {
-    RecJob J = prepare_records(g, g->w_rec, g->w_scr, g->st, kap, kr, cv, D, diff, kapi, kri, tdiff);
+                       const std::vector<double>& kri = {}, bool sweep = false, bool tdiff = false, bool together = false) {
+    RecJob J = prepare_records(g, g->w_rec, g->w_scr, g->st, kap, kr, cv, D, diff, kapi, kri, sweep, tdiff, together);
     J.prof = g->prof;
     cdbl* E = launch_records(J);
     HIPC(hipGetLastError());
@@ -1029,7 +1050,7 @@ cdbl* assemble_records(hbem_geometry* g, const std::vector<double>& kap, const s
 // takes the node loops for every pair their local matrices and partials too.  Builds
 // the tables the call needs, so that the free memory seen afterwards is what its
 // batches can use.
-size_t records_bytes_per_k(hbem_geometry* g, const std::vector<double>& kap, int D, int lcols, int slots) {
+size_t records_bytes_per_k(hbem_geometry* g, const std::vector<double>& kap, int D, int lcols, int slots, bool sweep) {
     const bool quirk = record_values(g, D) != hbem::kRecValues;
     bool loops = false, cplx = false;
     size_t basis = 0;
@@ -1037,8 +1058,8 @@ size_t records_bytes_per_k(hbem_geometry* g, const std::vector<double>& kap, int
     for (double v : kap) cplx = cplx || !(v > 0.0);
     for (double v : kap) {
         const double m = std::fabs(v);
-        if (cplx && !quirk) record_tier(g, m, m, 0.0, true);
-        const int t = quirk ? -1 : record_tier(g, m, m, 0.0, false);
+        if (cplx && !quirk) record_tier(g, m, m, 0.0, true, sweep);
+        const int t = quirk ? -1 : record_tier(g, m, m, 0.0, false, sweep);
         if (t < 0) loops = true;
         else basis = std::max(basis, (size_t)(g->rad->tier[t].basis + 2 * g->rad->tier[t].pnear) * slots * sizeof(cdbl));
     }
@@ -1172,10 +1193,12 @@ void tp_system(hbem_geometry* g, double k_re, double k_im, double c_o, double c_
                cdbl*& T, cdbl*& rhs) {
     const double si = std::sqrt(c_i), so = std::sqrt(c_o);
     // the outer operators are wanted by themselves: one column per refraction index
-    cdbl* E = real_positive(k_re, k_im)
-                  ? assemble_records(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, 0, false)
-                  : assemble_records(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, 0, false,
-                                     {k_im * si, k_im * so}, {k_im, k_im});
+    std::vector<double> kapi, kri;
+    if (!real_positive(k_re, k_im)) {
+        kapi = {k_im * si, k_im * so};
+        kri = {k_im, k_im};
+    }
+    cdbl* E = assemble_records(g, {k_re * si, k_re * so}, {k_re, k_re}, {c_i, c_o}, 0, false, kapi, kri, false, false, true);
     const int N = g->N, n = 2 * N;
     const size_t nn = (size_t)n * n;
     const double* dM = (const double*)g->d_M.p;
@@ -1351,7 +1374,6 @@ int hbem_geometry_release_work(hbem_geometry_t g) {
                              &g->w_R, &g->w_u, &g->w_v, &g->w_a, &g->w_b, &g->w_sig, &g->w_dsig, &g->w_tmp, &g->w_out,
                              &g->w_rec.tab,
                              &g->w_scr.E, &g->w_scr.L, &g->w_scr.part};
-    for (auto& b : g->w_rec.lslots) bs.push_back(b.get());
     for (DBuf* b : bs) b->release();
     API_END
 }
@@ -1405,7 +1427,7 @@ int hbem_assemble_dense_batch(hbem_geometry_t g, const double* ks, int nk, doubl
     // one wavenumber slot per k: its records, and its local matrices where it takes the node loops
     std::vector<double> all(nk);
     for (int i = 0; i < nk; ++i) all[i] = ks[i] * sc;
-    const size_t per = records_bytes_per_k(g, all, d, 1, 1);
+    const size_t per = records_bytes_per_k(g, all, d, 1, 1, false);
     const int B = sweep_batch(per, usable_device_bytes(g->w_scr.E.n + g->w_scr.L.n + g->w_scr.part.n), nk);
     for (int k0 = 0; k0 < nk; k0 += B) {
         const int nb = std::min(B, nk - k0);
@@ -1916,7 +1938,7 @@ void sweep_run(hbem_geometry* g, const double* ks, int nk, double c_o, double c_
     const double si = std::sqrt(c_i), so = std::sqrt(c_o);
     std::vector<double> all;
     for (int i = 0; i < nk; ++i) all.push_back(ks[i] * std::max(si, so));
-    const size_t per = records_bytes_per_k(g, all, D, tdiff ? 1 : 2, 2) + dense_bytes_per_k(n, D, nc) +
+    const size_t per = records_bytes_per_k(g, all, D, tdiff ? 1 : 2, 2, true) + dense_bytes_per_k(n, D, nc) +
                        (d2sigma ? der2_bytes_per_k(n) : 0) + (mx ? mixed_bytes_per_k(n, nc) : 0);
     const int B = sweep_batch(per, usable_device_bytes(g->work_held()), nk);
     cdbl* dR = g->w_R.as<cdbl>((size_t)n * nc);
@@ -1933,7 +1955,7 @@ void sweep_run(hbem_geometry* g, const double* ks, int nk, double c_o, double c_
             kap[nb + b] = k * so; kr[nb + b] = k; cv[nb + b] = c_o;
         }
         const std::vector<double> zero(allpos ? 0 : kap.size(), 0.0);
-        cdbl* E = assemble_records(g, kap, kr, cv, D, true, zero, zero, tdiff);
+        cdbl* E = assemble_records(g, kap, kr, cv, D, true, zero, zero, true, tdiff);
         cdbl* T0 = g->w_T0.as<cdbl>(nn * nb);
         cdbl* T1 = D >= 1 ? g->w_T1.as<cdbl>(nn * nb) : nullptr;
         cdbl* T2 = D >= 2 ? g->w_T2.as<cdbl>(nn * nb) : nullptr;
@@ -2170,7 +2192,7 @@ void multi_subset(const std::vector<hbem_geometry*>& G, const std::vector<int>& 
             kap[j] = k * std::sqrt(c_i[i]); kr[j] = k; cv[j] = c_i[i];
             kap[nk + j] = k * std::sqrt(c_o); kr[nk + j] = k; cv[nk + j] = c_o;
         }
-        jobs.push_back(prepare_records(G[i], *w.rec[a], w.scr, st, kap, kr, cv, 0, true, {}, {},
+        jobs.push_back(prepare_records(G[i], *w.rec[a], w.scr, st, kap, kr, cv, 0, true, {}, {}, true,
                                        sweep_tdiff(ks + (size_t)i * nk, nk)));
     }
     std::vector<hbem::CsrDesc> desc(batch), descT(batch);
@@ -2323,7 +2345,7 @@ int hbem_sigma_sweep_multi(const hbem_geometry_t* geoms, int ninst, const double
         std::vector<double> kap;
         for (int j = 0; j < nk; ++j) kap.push_back(ks[(size_t)i * nk + j] * cm);
         const size_t n_pad = (2 * (size_t)G[i]->N + gran - 1) / gran * gran;
-        need[i] = (size_t)nk * records_bytes_per_k(G[i], kap, 0, sweep_tdiff(ks + (size_t)i * nk, nk) ? 1 : 2, 2) +
+        need[i] = (size_t)nk * records_bytes_per_k(G[i], kap, 0, sweep_tdiff(ks + (size_t)i * nk, nk) ? 1 : 2, 2, true) +
                   (size_t)nk * (n_pad * n_pad * sizeof(cdbl) + n_pad * (8 + (4 * nc + 4) * sizeof(cdbl)));
     }
     size_t held = 0;

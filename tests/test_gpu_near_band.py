@@ -7,9 +7,9 @@ by Miller's recurrence and Neumann's series.
 Bar: 8 units of rounding (the last roundings of coefficients, basis and sums), plus the
 phase that rounded node positions put on H(kappa r): coordinates up to 1.3 are 18 panel
 diameters here, so a difference of two is off by up to 36 units of d, and the 64 nodes
-of a panel pair average it to an eighth; 8 kappa d units are allowed.  The node loops are
-at up to 1e-14 + 8 kappa d units (their tables of the Bessel functions are good to
-1e-14)."""
+of a panel pair average it to an eighth; 8 kappa d units are allowed.  Beyond kappa d =
+5 the real ones of these calls take the node loops, whose tables of the Bessel functions are good to
+1e-14: 1e-14 more there."""
 import numpy as np
 import pytest
 
@@ -94,7 +94,7 @@ def layers(O, mesh, kap):
     return CL(1j) / 4 * K, CL(1j) / 4 * V
 
 
-@pytest.mark.parametrize("kd", [0.3, 0.62, 2.4, 4.9, 9.9, 19.9, 0.4 + 0.03j, 9.0 + 0.045j, -9.0])
+@pytest.mark.parametrize("kd", [0.3, 0.62, 2.4, 4.9, 9.9, 19.9, 0.4 + 0.03j, 4.5 + 0.045j, 9.0 + 0.045j, -4.5, -9.0])
 def test_entries_next_to_the_diagonal(kd, H, O):
     if np.finfo(LD).eps > 1e-18:
         pytest.skip("long double is no wider than double here")
@@ -107,7 +107,7 @@ def test_entries_next_to_the_diagonal(kd, H, O):
     kap = CL(complex(0)) + LD(k.real) + CL(1j) * LD(k.imag) if k.imag or k.real < 0 else LD(k.real)
     m, n = np.indices((N, N))
     near = np.minimum((m - n) % N, (n - m) % N) <= APART
-    bar = (8 + 8 * abs(kd)) * U
+    bar = (8 + 8 * abs(kd)) * U + (1e-14 if np.isreal(kd) and kd > 5 else 0.0)
     for name, got, ref in zip("KV", (gb.getDoubleLayer(), gb.getSingleLayer()), layers(O, mesh, kap)):
         e = np.linalg.norm((got[near].astype(CL) - ref[near]).astype(complex)) / np.linalg.norm(ref[near].astype(complex))
         print("%s kd %s: %.1e of %.1e" % (name, kd, e, bar))
