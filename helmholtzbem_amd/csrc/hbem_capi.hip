@@ -632,9 +632,10 @@ hbem_geometry::Tier* radial_tier(hbem_geometry* g, int t) {
         if (b > 0 && it == cosoff.end()) {
             it = cosoff.emplace(p, (int)cosv.size()).first;
             for (int j = 0; j < p; ++j) points[p].push_back(cosl(acosl(-1.0L) * (2 * j + 1) / (2.0L * p)));
+            std::vector<double> c4(4 * p);        // cos of the multiples of pi / (2 p)
+            for (int k = 0; k < 4 * p; ++k) c4[k] = std::cos(M_PI * k / (2.0 * p));
             for (int j = 0; j < p; ++j)
-                for (int q = 0; q < p; ++q)
-                    cosv.push_back((q == 0 ? 1.0 : 2.0) / p * std::cos(M_PI * (double)((long long)q * (2 * j + 1) % (4 * p)) / (2.0 * p)));
+                for (int q = 0; q < p; ++q) cosv.push_back((q == 0 ? 1.0 : 2.0) / p * c4[q * (2 * j + 1) % (4 * p)]);
         }
         if (b > 0) B.cos = it->second;
         B.rad = (int)cosv.size();

@@ -200,8 +200,9 @@ __device__ __forceinline__ double gauss_node(const PairNode& x, int i, int j, co
     return vx * vx + vy * vy;
 }
 
-// Coefficients of the far bands.  Sixteen lanes per pair, two workgroups per tile:
-// lanes over the Gauss nodes of the four panel pairs; per node the five
+// Coefficients of the far bands.  L = 16 lanes per pair, two workgroups per tile (64,
+// eight, where there are few pairs: see launch_radial_far): lanes over the Gauss nodes
+// of the four panel pairs; per node the five
 // quadrature coefficients and the Chebyshev polynomials T_q of its position in
 // the band are formed, twelve q at a time (60 register sums a lane, totalled over
 // the sixteen lanes together), and the moments mu_q are carried to the points by
@@ -210,17 +211,18 @@ __device__ __forceinline__ double gauss_node(const PairNode& x, int i, int j, co
 // coefficients of the smooth function; a recurrence over the points would not be
 // damped.  The two double-layer coefficients are stored divided by r_j (they
 // multiply H1 / r).
+template <int L>
 __global__ __launch_bounds__(128) void k_radial_far(const int* __restrict__ recs, const BandTile* __restrict__ tiles,
                                                     int tile0, const Band* __restrict__ bands,
                                                     const double* __restrict__ gtab, const double* __restrict__ xg,
                                                     const double* __restrict__ wg, int N, int ns,
                                                     const unsigned char* __restrict__ flags,
                                                     const double* __restrict__ costab, double* __restrict__ tab, int pmax) {
-    constexpr int QC = 12;
-    extern __shared__ double mu_s[];          // [8 pairs][pmax][5]
-    const int row = (blockIdx.x & 1) * 8 + (threadIdx.x >> 4), l = threadIdx.x & 15;
-    const int tile = tile0 + (blockIdx.x >> 1);
-    double* mu = mu_s + (size_t)(threadIdx.x >> 4) * pmax * 5;
+    constexpr int QC = 12, PB = 128 / L, BT = 16 / PB;   // pairs of a workgroup, workgroups of a tile
+    extern __shared__ double mu_s[];          // [PB][pmax][5]
+    const int row = (blockIdx.x % BT) * PB + threadIdx.x / L, l = threadIdx.x % L;
+    const int tile = tile0 + blockIdx.x / BT;
+    double* mu = mu_s + (size_t)(threadIdx.x / L) * pmax * 5;
     const BandTile bt = tiles[tile];
     const Band bd = bands[bt.band];
     const int rec = recs[(size_t)tile * 16 + row];
@@ -234,7 +236,7 @@ __global__ __launch_bounds__(128) void k_radial_far(const int* __restrict__ recs
         for (int f = 0; f < 64; ++f) s[f] = 0.0;
         for (int ab = 0; ab < 4 && rec >= 0; ++ab) {
             const PairNode pn = pair_node(m, n, ab, N, flags);
-            for (int nd = l; nd < nn; nd += 16) {
+            for (int nd = l; nd < nn; nd += L) {
                 const int i = nd / ns, j = nd - i * ns;
                 double c[5];
                 const double r = sqrt(gauss_node(pn, i, j, gtab, ns, xg, wg, c));
@@ -255,10 +257,10 @@ __global__ __launch_bounds__(128) void k_radial_far(const int* __restrict__ recs
                 }
             }
         }
-        exchange_halves<8, 64>(s);
+        exchange_halves<L / 2, 64>(s);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int f = 4 * l + k;
+        for (int k = 0; k < 64 / L; ++k) {
+            const int f = 64 / L * l + k;
             if (f < QC * 5 && q0 * 5 + f < p * 5) mu[q0 * 5 + f] = s[k];
         }
     }
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(128) void k_radial_far(const int* __restrict__ recs
     const double* ct = costab + bd.cos;       // [j][q], weighted
     const double* rj = costab + bd.rad;
     double* out = tab + bt.off;
-    for (int it = l; it < p * 5; it += 16) {
+    for (int it = l; it < p * 5; it += L) {
         const int j = it / 5, g = it - 5 * j;
         double v = 0.0;
         for (int q = 0; q < p; ++q) v = fma(ct[j * p + q], mu[q * 5 + g], v);
@@ -1252,12 +1254,22 @@ void launch_radial_flags(const double* gtab, int ns, int npairs, unsigned char* 
     hipLaunchKernelGGL(k_radial_flags, dim3(grid_of(npairs)), dim3(256), 0, st, gtab, ns, npairs, flags);
 }
 
+constexpr int kFarFewTiles = 512;
 void launch_radial_far(const int* recs, const BandTile* tiles, int tile0, int ntile, const Band* bands, int pmax,
                        const double* gtab, const double* xg, const double* wg, int N, int ns, const unsigned char* flags,
                        const double* costab, double* tab, hipStream_t st) {
     if (ntile <= 0) return;
-    hipLaunchKernelGGL(k_radial_far, dim3(2 * (unsigned)ntile), dim3(128), 8 * pmax * 5 * sizeof(double), st, recs, tiles,
-                       tile0, bands, gtab, xg, wg, N, ns, flags, costab, tab, pmax);
+    const auto run = [&](auto kernel, int lanes) {
+        const int pairs = 128 / lanes;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)ntile * (16 / pairs)), dim3(128), pairs * pmax * 5 * sizeof(double), st, recs,
+                           tiles, tile0, bands, gtab, xg, wg, N, ns, flags, costab, tab, pmax);
+    };
+    // Below one wavefront a SIMD with 16 lanes a pair, 64 lanes shorten the chain of a
+    // pair's nodes (us, 16 -> 64 lanes, order 11): 48 panels, kappa d = 4.5 128 -> 53; 64
+    // panels, 0.5 82 -> 31; 100 panels 85 -> 63; 140 panels (over 600 tiles) 112 -> 117,
+    // where the sums over more lanes only cost.
+    if (ntile <= kFarFewTiles) run(k_radial_far<64>, 64);
+    else run(k_radial_far<16>, 16);
 }
 
 void launch_radial_moments(int cls, const int* ent, int cnt, const double* panels, const double* coefs, const double* xc,
