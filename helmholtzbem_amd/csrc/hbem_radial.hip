@@ -205,7 +205,7 @@ __device__ __forceinline__ double gauss_node(const PairNode& x, int i, int j, co
 // of the four panel pairs; per node the five
 // quadrature coefficients and the Chebyshev polynomials T_q of its position in
 // the band are formed, twelve q at a time (60 register sums a lane, totalled over
-// the sixteen lanes together), and the moments mu_q are carried to the points by
+// the pair's lanes together), and the moments mu_q are carried to the points by
 // C_j = sum_q (2 - delta_q0) / p T_q(s_j) mu_q (costab, built on the host).  The
 // T_q recurrence runs for the nodes only, where its errors meet the decaying
 // coefficients of the smooth function; a recurrence over the points would not be
@@ -1264,7 +1264,7 @@ void launch_radial_far(const int* recs, const BandTile* tiles, int tile0, int nt
         hipLaunchKernelGGL(kernel, dim3((unsigned)ntile * (16 / pairs)), dim3(128), pairs * pmax * 5 * sizeof(double), st, recs,
                            tiles, tile0, bands, gtab, xg, wg, N, ns, flags, costab, tab, pmax);
     };
-    // Below one wavefront a SIMD with 16 lanes a pair, 64 lanes shorten the chain of a
+    // Up to two wavefronts a SIMD with 16 lanes a pair, 64 lanes shorten the chain of a
     // pair's nodes (us, 16 -> 64 lanes, order 11): 48 panels, kappa d = 4.5 128 -> 53; 64
     // panels, 0.5 82 -> 31; 100 panels 85 -> 63; 140 panels (over 600 tiles) 112 -> 117,
     // where the sums over more lanes only cost.
